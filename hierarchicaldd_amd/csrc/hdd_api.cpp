@@ -573,10 +573,12 @@ hdd_status hdd_stats(const hdd_ctx* ctx, double* out, int n) {
     const SigmaDevice* G = S.sigma.get();
     int nsub = 0;
     for (auto& q : S.prob) nsub += q->sigma.nsub;
-    // fused heights of every triangular-solve plan, and how many use the wavefront-per-run form
+    // levels of the dense-node plans and fused heights of the per-height ones, and how many of
+    // those use the wavefront-per-run form
     double fused = 0, waved = 0;
     if (G) {
         auto count = [&](const TriPlan& T) {
+            fused += (double)T.nodes.levels.size();
             for (size_t h = 0; h < T.fused.size(); ++h)
                 if (T.fused[h]) { fused += 1; waved += (h < T.wave.size() && T.wave[h]) ? 1 : 0; }
         };

@@ -1,0 +1,487 @@
+// Dense-node form of the interface solver's exact solves (hdd_nodeplan.h): the
+// blocks' operators formed in double at set-up, and the two passes of a solve.
+//
+// An operator is kept in 16x16 tiles of 1 KiB in the lane order of the FP32
+// MFMA: lane l holds row l%16, columns 4(l/16) .. +3, so a wavefront loads a
+// tile with one contiguous 16-byte access per lane and uses it as the A
+// operand of four v_mfma_f32_16x16x4_f32 (instruction s takes the columns
+// 4q + s of the lanes' groups q; A and B agree on that order, so it only
+// permutes the summands). The B operand is the run's vectors, one node per
+// column, in LDS: a run of one node uses one column of the sixteen, which the
+// matrix unit can afford (it consumes tiles at about 20 TB/s over the chip, HBM
+// delivers 8). Forward tiles of a block: row tile rt < nk (Linv) has rt + 1 of
+// them, row tile nk + a (W) has nk. Backward: row tile rt has nk - rt (Linv^T)
+// and nrk (-W^T).
+#include <hip/hip_runtime.h>
+#include <algorithm>
+#include <stdexcept>
+#include "hdd_nodeplan_device.h"
+#include "hdd_parallel.h"
+
+namespace hdd {
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int T = NodePlanHost::kTile;
+
+__device__ __forceinline__ long long fwd_row(int rt, int nk) {
+    return rt < nk ? (long long)rt * (rt + 1) / 2 : (long long)nk * (nk + 1) / 2 + (long long)(rt - nk) * nk;
+}
+__device__ __forceinline__ long long bwd_row(int rt, int nk, int nrk) { return (long long)rt * (nk + nrk) - (long long)rt * (rt - 1) / 2; }
+
+__device__ __forceinline__ bool run_stopped(const int* __restrict__ active, const int* __restrict__ prob, int i0, int cnt) {
+    if (!active) return false;
+    for (int j = 0; j < cnt; ++j)
+        if (active[prob[i0 + j]]) return false;
+    return true;
+}
+
+// Children's sums of a level, one thread per row: t = b - sum at its columns (held in z until the
+// backward pass), the sum itself at its boundary rows (in c, where the forward product adds to it).
+// On its own because a node's row tiles go to several workgroups, which all need every t of the node:
+// with the sums inside the forward kernel, its gather was 3 times its product on the 256^3 level-0
+// interiors (171 us against 49 us for the backward pass of the same level).
+__global__ void __launch_bounds__(256) k_node_children(int y0, int y1, int c0, int c1, const NodePos* __restrict__ pos_y,
+                                                       const NodePos* __restrict__ pos_c, const int* __restrict__ more,
+                                                       const int* __restrict__ orig, const float* __restrict__ b,
+                                                       float* __restrict__ t, float* __restrict__ c) {
+    const int i = blockIdx.x * 256 + threadIdx.x, ny = y1 - y0;
+    if (i >= ny + c1 - c0) return;
+    const bool col = i < ny;
+    const NodePos p = col ? pos_y[y0 + i] : pos_c[c0 + i - ny];
+    float bv = 0.f;
+    if (col) {
+        const int o = orig[y0 + i];
+        if (o >= 0) bv = b[o];
+    }
+    float s = c[p.p0];
+    if (p.p1 >= 0) {
+        s += c[p.p1];
+    } else {
+        const int* m = more + ~p.p1;
+        const int cnt = m[0];
+#pragma unroll 4
+        for (int e = 1; e <= cnt; ++e) s += c[m[e]];
+    }
+    if (col) t[y0 + i] = bv - s;
+    else c[c0 + i - ny] = s;
+}
+
+// D (16 rows x 16 nodes) of one row tile: tiles [0, nt) at A against the operand vectors from tp on,
+// every KS-th tile from kw. The tiles are loaded kAhead at a time, a group ahead of the products
+// (`a` holds the first group on entry); four independent sums (one per tile column mod 4) keep the
+// chains short.
+constexpr int kAhead = 4;
+template <int KS>
+__device__ __forceinline__ void load_group(const f32x4* __restrict__ A, int k, int nt, f32x4 (&a)[kAhead]) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+        if (k + u * KS < nt) a[u] = A[(size_t)(k + u * KS) * 64];
+}
+template <int KS>
+__device__ __forceinline__ f32x4 row_tile(const f32x4* __restrict__ A, const f32x4* tp, int nt, int kw, f32x4 (&a)[kAhead]) {
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0, s2 = s0, s3 = s0;
+    for (int k = kw; k < nt; k += kAhead * KS) {
+        f32x4 nx[kAhead];
+        load_group<KS>(A, k + kAhead * KS, nt, nx);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            if (k + u * KS < nt) {
+                const f32x4 t = tp[(k + u * KS) * 4];
+                s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][0], t[0], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][1], t[1], s1, 0, 0, 0);
+                s2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][2], t[2], s2, 0, 0, 0);
+                s3 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][3], t[3], s3, 0, 0, 0);
+            }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) a[u] = nx[u];
+    }
+    return (s0 + s1) + (s2 + s3);
+}
+
+// adds the partial sums of the KS waves that share a row tile (the first of them returns the total);
+// every wave of the workgroup takes part
+template <int KS>
+__device__ __forceinline__ f32x4 join(f32x4 d, f32x4 (*red)[64], int w, int lane) {
+    if (KS == 1) return d;
+    __syncthreads();  // the previous row tile's sums have been read
+    red[w][lane] = d;
+    __syncthreads();
+    if (w % KS == 0)
+        for (int s = 1; s < KS; ++s) d += red[w + s][lane];
+    return d;
+}
+
+// The row tiles [rt0, rt1) of a workgroup of NW waves, KS of them per row tile: gather() fills the
+// operand vectors in LDS (while the first tiles load), where(rt, &A, &tp, &nt) gives a row tile's
+// tiles and operand, out(rt, d) takes its 16x16 result from the lanes that hold it.
+template <int NW, int KS, class Where, class Gather, class Out>
+__device__ __forceinline__ void row_tiles(int rt0, int rt1, f32x4 (*red)[64], Where where, Gather gather, Out out) {
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    constexpr int step = NW / KS;
+    int rt = rt0 + w / KS, nt = 0;
+    const f32x4* A = nullptr;
+    const f32x4* tp = nullptr;
+    f32x4 a[kAhead];
+    if (rt < rt1) {
+        where(rt, A, tp, nt);
+        load_group<KS>(A, w % KS, nt, a);
+    }
+    gather();
+    __syncthreads();
+    for (int r0 = rt0; r0 < rt1; r0 += step) {
+        const bool live = rt < rt1;
+        f32x4 d = {0.f, 0.f, 0.f, 0.f};
+        if (live) d = row_tile<KS>(A, tp, nt, w % KS, a);
+        const int rc = rt;
+        rt += step;
+        if (rt < rt1) {  // the next row tile's first tiles load beside this one's results
+            where(rt, A, tp, nt);
+            load_group<KS>(A, w % KS, nt, a);
+        }
+        d = join<KS>(d, red, w, lane);
+        if (live && w % KS == 0) out(rc, d);
+    }
+}
+template <int NW, class Where, class Gather, class Out>
+__device__ __forceinline__ void row_tiles(int split, int rt0, int rt1, f32x4 (*red)[64], Where where, Gather gather, Out out) {
+    if (NW == 16) return row_tiles<NW, 16>(rt0, rt1, red, where, gather, out);
+    if (split == 1) return row_tiles<NW, 1>(rt0, rt1, red, where, gather, out);
+    if (split == 2) return row_tiles<NW, 2>(rt0, rt1, red, where, gather, out);
+    row_tiles<NW, 4>(rt0, rt1, red, where, gather, out);
+}
+
+// Forward pass of a level: t into LDS, then the row tiles of [I + S; W] t. NW waves per workgroup;
+// INC: the nodes have children (t and the boundary rows' sums from k_node_children).
+template <int NW, bool INC>
+__global__ void __launch_bounds__(NW * 64) k_node_fwd(const NodeItem* __restrict__ items, const int* __restrict__ inst_y,
+                                                      const int* __restrict__ inst_c, const int* __restrict__ inst_prob,
+                                                      const int* __restrict__ active, const int* __restrict__ orig,
+                                                      const float* __restrict__ t, const float* __restrict__ tiles,
+                                                      const float* __restrict__ scale, const float* __restrict__ b,
+                                                      float* __restrict__ y, float* __restrict__ c) {
+    extern __shared__ f32x4 lds[];
+    __shared__ f32x4 red[NW][64];
+    const NodeItem it = items[blockIdx.x];
+    if (run_stopped(active, inst_prob, it.inst0, it.cnt)) return;
+    const int lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    const int np = it.nk * T, ld = np + 4, my_col = min(col, it.cnt - 1);
+    const int yb = inst_y[it.inst0 + my_col], cb = inst_c[it.inst0 + my_col];
+    const f32x4* base = reinterpret_cast<const f32x4*>(tiles) + (size_t)it.tile * 64 + lane;
+    const f32x4* tcol = lds + (my_col * ld) / 4 + q;
+    auto where = [&](int rt, const f32x4*& A, const f32x4*& tp, int& nt) {
+        A = base + (size_t)fwd_row(rt, it.nk) * 64;
+        tp = tcol;
+        nt = rt < it.nk ? rt + 1 : it.nk;
+    };
+    auto gather = [&]() {
+        for (int idx = threadIdx.x; idx < it.cnt * np / 4; idx += NW * 64) {
+            const int j = idx / (np / 4), k = idx - j * (np / 4);
+            const int i = inst_y[it.inst0 + j] + 4 * k;
+            f32x4 v;
+            if (INC) {
+                v = *reinterpret_cast<const f32x4*>(t + i);
+            } else {
+                const int4 o = *reinterpret_cast<const int4*>(orig + i);
+                v[0] = o.x >= 0 ? b[o.x] : 0.f; v[1] = o.y >= 0 ? b[o.y] : 0.f;
+                v[2] = o.z >= 0 ? b[o.z] : 0.f; v[3] = o.w >= 0 ? b[o.w] : 0.f;
+            }
+            lds[(j * ld) / 4 + k] = v;
+        }
+    };
+    auto out = [&](int rt, f32x4 d) {
+        if (col >= it.cnt) return;
+        if (rt < it.nk) {
+            d += tcol[rt * 4];  // the unit diagonal
+            d *= *reinterpret_cast<const f32x4*>(scale + it.scale + rt * T + 4 * q);
+            *reinterpret_cast<f32x4*>(y + yb + rt * T + 4 * q) = d;
+        } else {
+            f32x4* ca = reinterpret_cast<f32x4*>(c + cb + (rt - it.nk) * T + 4 * q);
+            if (INC) d += *ca;
+            *ca = d;
+        }
+    };
+    row_tiles<NW>(it.split, it.rt0, it.rt1, red, where, gather, out);
+}
+
+// Backward pass of a level: [D^-2 y; z of the boundary rows] into LDS, then the row tiles of
+// [I + S^T | -W^T]; the result goes to z and, in the original numbering, to x.
+template <int NW>
+__global__ void __launch_bounds__(NW * 64) k_node_bwd(const NodeItem* __restrict__ items, const int* __restrict__ inst_y,
+                                                      const int* __restrict__ inst_c, const int* __restrict__ inst_prob,
+                                                      const int* __restrict__ active, const int* __restrict__ orig,
+                                                      const int* __restrict__ zidx, const float* __restrict__ tiles,
+                                                      const float* __restrict__ y, float* __restrict__ z, float* __restrict__ x) {
+    extern __shared__ f32x4 lds[];
+    __shared__ f32x4 red[NW][64];
+    const NodeItem it = items[blockIdx.x];
+    if (run_stopped(active, inst_prob, it.inst0, it.cnt)) return;
+    const int lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    const int np = it.nk * T, nz = np + it.nrk * T, ld = nz + 4, my_col = min(col, it.cnt - 1);
+    const int yb = inst_y[it.inst0 + my_col];
+    const f32x4* base = reinterpret_cast<const f32x4*>(tiles) + (size_t)it.tile * 64 + lane;
+    const f32x4* tcol = lds + (my_col * ld) / 4 + q;
+    auto where = [&](int rt, const f32x4*& A, const f32x4*& tp, int& nt) {
+        A = base + (size_t)bwd_row(rt, it.nk, it.nrk) * 64;
+        tp = tcol + rt * 4;
+        nt = it.nk + it.nrk - rt;
+    };
+    auto gather = [&]() {
+        for (int idx = threadIdx.x; idx < it.cnt * nz / 4; idx += NW * 64) {
+            const int j = idx / (nz / 4), k = 4 * (idx - j * (nz / 4));
+            f32x4 v;
+            if (k < np) {
+                v = *reinterpret_cast<const f32x4*>(y + inst_y[it.inst0 + j] + k);
+            } else {
+                const int4 o = *reinterpret_cast<const int4*>(zidx + inst_c[it.inst0 + j] + k - np);
+                v[0] = z[o.x]; v[1] = z[o.y]; v[2] = z[o.z]; v[3] = z[o.w];
+            }
+            lds[(j * ld + k) / 4] = v;
+        }
+    };
+    auto out = [&](int rt, f32x4 d) {
+        if (col >= it.cnt) return;
+        d += tcol[rt * 4];
+        const int i = yb + rt * T + 4 * q;
+        *reinterpret_cast<f32x4*>(z + i) = d;
+        const int4 o = *reinterpret_cast<const int4*>(orig + i);
+        if (o.x >= 0) x[o.x] = d[0];
+        if (o.y >= 0) x[o.y] = d[1];
+        if (o.z >= 0) x[o.z] = d[2];
+        if (o.w >= 0) x[o.w] = d[3];
+    };
+    row_tiles<NW>(it.split, it.rt0, it.rt1, red, where, gather, out);
+}
+
+// ---- set-up: the operators from the factor columns, in double -----------------------------------
+
+struct SetupBlock {
+    long long l, x;   // first double of the block's columns ((nk + nrk) T x nk T, row-major) and of Linv
+    int nk, nrk, fwd, bwd, scale, pad;
+};
+
+// X = L11^{-1}, one workgroup per 16-column strip: X_i = L_ii^{-1} (E_i - sum_{k < i} L_ik X_k) down the
+// row tiles; thread (r, c) owns one element of the tile
+__global__ void __launch_bounds__(256) k_node_inverse(const SetupBlock* __restrict__ blocks, const int2* __restrict__ strips,
+                                                      const double* __restrict__ L, double* __restrict__ X) {
+    __shared__ double ls[T][T + 1], xs[T][T + 1];
+    const int2 st = strips[blockIdx.x];
+    const SetupBlock B = blocks[st.x];
+    const int r = threadIdx.x >> 4, c = threadIdx.x & 15, ct = st.y;
+    const long long np = (long long)B.nk * T;
+    const double* Lb = L + B.l;
+    double* Xb = X + B.x;
+    for (int it = 0; it < ct; ++it) Xb[(it * T + r) * np + ct * T + c] = 0.0;
+    for (int it = ct; it < B.nk; ++it) {
+        double s = it == ct && r == c ? 1.0 : 0.0;
+        double ln = 0.0, xn = 0.0;
+        if (ct < it) { ln = Lb[(it * T + r) * np + ct * T + c]; xn = Xb[(ct * T + r) * np + ct * T + c]; }
+        for (int kt = ct; kt < it; ++kt) {
+            ls[r][c] = ln; xs[r][c] = xn;
+            __syncthreads();
+            if (kt + 1 < it) {  // the next tiles load while this one is summed
+                ln = Lb[(it * T + r) * np + (kt + 1) * T + c];
+                xn = Xb[((kt + 1) * T + r) * np + ct * T + c];
+            }
+#pragma unroll
+            for (int k = 0; k < T; ++k) s -= ls[r][k] * xs[k][c];
+            __syncthreads();
+        }
+        ls[r][c] = Lb[(it * T + r) * np + it * T + c];
+        __syncthreads();
+        // forward substitution with the 16x16 diagonal tile, a row at a time
+        for (int k = 0; k < T; ++k) {
+            if (r == k) { s /= ls[k][k]; xs[k][c] = s; }
+            __syncthreads();
+            if (r > k) s -= ls[r][k] * xs[k][c];
+        }
+        Xb[(it * T + r) * np + ct * T + c] = s;
+        __syncthreads();
+    }
+}
+
+// forward operator, one workgroup per row tile: S = D Linv - I rounded to float (and D^-2), or W = L21 Linv (double sums)
+__global__ void __launch_bounds__(256) k_node_forward_tiles(const SetupBlock* __restrict__ blocks, const int2* __restrict__ rows,
+                                                            const double* __restrict__ L, const double* __restrict__ X,
+                                                            float* __restrict__ tiles, float* __restrict__ scale) {
+    __shared__ double ls[T][T + 1], xs[T][T + 1];
+    const int2 rw = rows[blockIdx.x];
+    const SetupBlock B = blocks[rw.x];
+    const int r = threadIdx.x >> 4, c = threadIdx.x & 15, rt = rw.y;
+    const long long np = (long long)B.nk * T;
+    const double* Xb = X + B.x;
+    float* out = tiles + ((size_t)B.fwd + fwd_row(rt, B.nk)) * 256 + ((c >> 2) * 16 + r) * 4 + (c & 3);
+    if (rt < B.nk) {
+        const double d = L[B.l + (rt * T + r) * np + rt * T + r];
+        for (int j = 0; j <= rt; ++j) {
+            const double v = Xb[(rt * T + r) * np + j * T + c];
+            out[(size_t)j * 256] = j == rt && r == c ? 0.f : (float)(d * v);
+        }
+        if (c == 0) scale[B.scale + rt * T + r] = (float)(1.0 / (d * d));
+        return;
+    }
+    const double* Lr = L + B.l + (long long)rt * T * np;
+    for (int j = 0; j < B.nk; ++j) {
+        double s = 0.0;
+        double ln = Lr[r * np + j * T + c], xn = Xb[(j * T + r) * np + j * T + c];
+        for (int kt = j; kt < B.nk; ++kt) {
+            ls[r][c] = ln; xs[r][c] = xn;
+            __syncthreads();
+            if (kt + 1 < B.nk) {
+                ln = Lr[r * np + (kt + 1) * T + c];
+                xn = Xb[((kt + 1) * T + r) * np + j * T + c];
+            }
+#pragma unroll
+            for (int k = 0; k < T; ++k) s += ls[r][k] * xs[k][c];
+            __syncthreads();
+        }
+        out[(size_t)j * 256] = (float)s;
+    }
+}
+
+// backward operator from the forward one: row tile rt holds the transposes of the forward tiles
+// (kt, rt), kt >= rt, and the negated transposes of the W tiles (a, rt)
+__global__ void __launch_bounds__(256) k_node_backward_tiles(const SetupBlock* __restrict__ blocks, const int2* __restrict__ rows,
+                                                             float* __restrict__ tiles) {
+    const int2 rw = rows[blockIdx.x];
+    const SetupBlock B = blocks[rw.x];
+    const int r = threadIdx.x >> 4, c = threadIdx.x & 15, rt = rw.y;
+    const int to = ((c >> 2) * 16 + r) * 4 + (c & 3), from = ((r >> 2) * 16 + c) * 4 + (r & 3);  // element (r, c) from (c, r)
+    float* out = tiles + ((size_t)B.bwd + bwd_row(rt, B.nk, B.nrk)) * 256 + to;
+    const float* in = tiles + (size_t)B.fwd * 256 + from;
+    for (int kt = rt; kt < B.nk + B.nrk; ++kt) {
+        const float v = in[(size_t)(fwd_row(kt, B.nk) + rt) * 256];
+        out[(size_t)(kt - rt) * 256] = kt < B.nk ? v : -v;
+    }
+}
+
+template <class K, class... A>
+void launch(K kernel, int grid, int waves, size_t lds, hipStream_t s, A... a) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3((unsigned)(waves * 64)), lds, s, a...);
+}
+
+// the kernels may use the whole LDS of a CU for their operand vectors (a default launch stops at 64 KiB)
+template <class K>
+void allow_lds(K kernel) {
+    hdd_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(NodePlanHost::kMaxLdsFloats * sizeof(float))),
+              "dense-node kernels' LDS");
+}
+
+struct Pinned {
+    double* p = nullptr;
+    explicit Pinned(size_t n) { hdd_check(hipHostMalloc((void**)&p, n * sizeof(double), hipHostMallocDefault), "hipHostMalloc"); }
+    ~Pinned() { (void)hipHostFree(p); }
+};
+
+}  // namespace
+
+bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, const std::vector<int>& prob_of) {
+    NodePlanHost P;
+    if (!build_nodeplan(F, offsets, prob_of, P)) return false;
+    bool wide = false;
+    for (const auto& L : P.levels) wide = wide || std::max(L.fwd_lds, L.bwd_lds) * sizeof(float) > 48 * 1024;
+    if (wide) {
+        allow_lds(k_node_fwd<4, false>); allow_lds(k_node_fwd<16, false>);
+        allow_lds(k_node_fwd<4, true>); allow_lds(k_node_fwd<16, true>);
+        allow_lds(k_node_bwd<4>); allow_lds(k_node_bwd<16>);
+    }
+    n = P.n;
+    levels = P.levels;
+    fwd.upload(P.fwd); bwd.upload(P.bwd);
+    inst_y.upload(P.inst_y); inst_c.upload(P.inst_c); inst_prob.upload(P.inst_prob);
+    orig.upload(P.orig);
+    P.zidx.resize(std::max<size_t>(1, P.zidx.size()), P.ysize); zidx.upload(P.zidx);
+    P.more.resize(std::max<size_t>(1, P.more.size()), 0); more.upload(P.more);
+    P.pos_c.resize(std::max<size_t>(1, P.pos_c.size()), NodePos{P.csize, P.csize});
+    pos_y.upload(P.pos_y); pos_c.upload(P.pos_c);
+    tiles.alloc((size_t)P.tiles * 256); scale.alloc(P.scales);
+    y.alloc(P.ysize); z.alloc((size_t)P.ysize + 1); c.alloc((size_t)P.csize + 1);
+    // the blocks in chunks: columns filled on the host, uploaded, inverted and packed
+    constexpr size_t kChunk = size_t(24) << 20;  // doubles per chunk, unless one block needs more
+    auto doubles = [](const NodePlanHost::Block& B) { return (size_t)(B.nk + B.nrk) * T * B.nk * T; };
+    size_t largest = 0, total = 0;
+    for (const auto& B : P.blocks) { largest = std::max(largest, doubles(B)); total += doubles(B); }
+    const size_t cap = std::min(total, std::max(largest, kChunk));
+    Pinned host(cap);
+    DBuf<double> dL, dX;
+    hdd_check(hipMalloc(&dL.p, cap * sizeof(double)), "hipMalloc"); dL.n = cap;
+    size_t xcap = 0;
+    std::vector<std::pair<size_t, size_t>> chunks;
+    for (size_t i = 0; i < P.blocks.size();) {
+        size_t used = 0, xs = 0, k = i;
+        while (k < P.blocks.size() && (k == i || used + doubles(P.blocks[k]) <= cap)) {
+            used += doubles(P.blocks[k]);
+            xs += (size_t)P.blocks[k].nk * T * P.blocks[k].nk * T;
+            ++k;
+        }
+        xcap = std::max(xcap, xs);
+        chunks.push_back({i, k});
+        i = k;
+    }
+    hdd_check(hipMalloc(&dX.p, xcap * sizeof(double)), "hipMalloc"); dX.n = xcap;
+    for (auto& ch : chunks) {
+        std::vector<SetupBlock> sb;
+        std::vector<int2> strips, rows, brows;
+        long long l = 0, xo = 0;
+        for (size_t k = ch.first; k < ch.second; ++k) {
+            const NodePlanHost::Block& B = P.blocks[k];
+            const int id = (int)sb.size();
+            sb.push_back({l, xo, B.nk, B.nrk, B.fwd, B.bwd, B.scale, 0});
+            l += (long long)doubles(B);
+            xo += (long long)B.nk * T * B.nk * T;
+            for (int r = 0; r < B.nk; ++r) { strips.push_back(make_int2(id, r)); brows.push_back(make_int2(id, r)); }
+            for (int r = 0; r < B.nk + B.nrk; ++r) rows.push_back(make_int2(id, r));
+        }
+        ParallelErrors errs;
+#pragma omp parallel for schedule(dynamic)
+        for (size_t k = ch.first; k < ch.second; ++k)
+            errs.run([&] { node_block_columns(P.blocks[k], host.p + sb[k - ch.first].l); });
+        errs.rethrow();
+        DBuf<SetupBlock> dsb; dsb.upload(sb);
+        DBuf<int2> dst, drw, dbr;
+        dst.upload(strips); drw.upload(rows); dbr.upload(brows);
+        hdd_check(hipMemcpy(dL.p, host.p, (size_t)l * sizeof(double), hipMemcpyHostToDevice), "node blocks upload");
+        launch(k_node_inverse, (int)strips.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)dst.p, (const double*)dL.p, dX.p);
+        launch(k_node_forward_tiles, (int)rows.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)drw.p, (const double*)dL.p,
+               (const double*)dX.p, tiles.p, scale.p);
+        launch(k_node_backward_tiles, (int)brows.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)dbr.p, tiles.p);
+        hdd_check(hipGetLastError(), "node blocks");
+        hdd_check(hipStreamSynchronize(nullptr), "node blocks");
+    }
+    return true;
+}
+
+size_t NodePlan::bytes() const {
+    return (fwd.n + bwd.n) * sizeof(NodeItem) + (inst_y.n + inst_c.n + inst_prob.n + orig.n + zidx.n + more.n) * 4 +
+           (pos_y.n + pos_c.n) * 8 + (tiles.n + scale.n + y.n + z.n + c.n) * 4;
+}
+
+void NodePlan::solve(const float* b, float* x, const int* active, hipStream_t s) {
+    auto fwd_level = [&](const NodePlanHost::Level& L) {
+        if (L.children)
+            hipLaunchKernelGGL(k_node_children, dim3((unsigned)((L.y1 - L.y0 + L.c1 - L.c0 + 255) / 256)), dim3(256), 0, s, L.y0, L.y1, L.c0, L.c1,
+                               (const NodePos*)pos_y.p, (const NodePos*)pos_c.p, (const int*)more.p, (const int*)orig.p, b, z.p, c.p);
+        auto go = [&](auto kernel) {
+            launch(kernel, L.fwd1 - L.fwd0, L.fwd_waves, L.fwd_lds * sizeof(float), s, (const NodeItem*)fwd.p + L.fwd0, (const int*)inst_y.p,
+                   (const int*)inst_c.p, (const int*)inst_prob.p, active, (const int*)orig.p, (const float*)z.p, (const float*)tiles.p,
+                   (const float*)scale.p, b, y.p, c.p);
+        };
+        if (L.fwd_waves == 4) { if (L.children) go(k_node_fwd<4, true>); else go(k_node_fwd<4, false>); }
+        else { if (L.children) go(k_node_fwd<16, true>); else go(k_node_fwd<16, false>); }
+    };
+    auto bwd_level = [&](const NodePlanHost::Level& L) {
+        auto go = [&](auto kernel) {
+            launch(kernel, L.bwd1 - L.bwd0, L.bwd_waves, L.bwd_lds * sizeof(float), s, (const NodeItem*)bwd.p + L.bwd0, (const int*)inst_y.p,
+                   (const int*)inst_c.p, (const int*)inst_prob.p, active, (const int*)orig.p, (const int*)zidx.p, (const float*)tiles.p,
+                   (const float*)y.p, z.p, x);
+        };
+        if (L.bwd_waves == 4) go(k_node_bwd<4>);
+        else go(k_node_bwd<16>);
+    };
+    for (const auto& L : levels) if (L.fwd1 > L.fwd0) fwd_level(L);
+    for (auto L = levels.rbegin(); L != levels.rend(); ++L) if (L->bwd1 > L->bwd0) bwd_level(*L);
+}
+
+}  // namespace hdd

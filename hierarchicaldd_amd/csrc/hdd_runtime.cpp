@@ -116,31 +116,22 @@ size_t ProblemHost::device_bytes() const {
     double bytes = 0;
     for (const PagedLevel& L : lv) bytes += (L.npages() + 1.0) * kPageCells * 20.0 + L.npages() * 36.0;
     bytes += (lv[0].npages() + 1.0) * kPageCells * 16.0;  // x, b, q, s
-    // interface solver: float plans of the factors (diagonal inverse twice, L21 once), operators, vectors
+    // interface solver: dense-node plans of the factors, operators, vectors
     for (int l = 0; l < sigma.levels; ++l) {
         for (const Csr& A : sigma.Air[l]) bytes += 16.0 * A.nnz();
         bytes += 8.0 * sigma.Arr[l].nnz() + 64.0 * sigma.n_if[l];
         if (l + 1 < sigma.levels) bytes += 16.0 * sigma.Prr[l].nnz();
         if (factors && l < (int)factors->lv.size()) {
             const SigmaFactors::Level& F = factors->lv[l];
-            for (const SupernodalFactor& f : F.Aii) bytes += 8.0 * f.nnz();
-            bytes += 8.0 * F.Arr.nnz();
-            // dense tops (m x m floats each); a batch gives them to fewer rows, so this bounds them
-            const int min_rows = dense_top_min_rows();
-            int members = 0, m = 0;
-            for (int s = 0; s < (int)F.rep.size(); ++s) members += min_rows > 0 && F.Aii[F.rep[s]].n >= min_rows;
-            for (const SupernodalFactor& f : F.Aii)
-                if (dense_top_cut(f, min_rows, members, &m) != INT_MAX) bytes += 4.0 * m * m;
-            if (dense_top_cut(F.Arr, min_rows, 1, &m) != INT_MAX) bytes += 4.0 * m * m;
+            for (const SupernodalFactor& f : F.Aii) bytes += nodeplan_bytes(f);
+            bytes += nodeplan_bytes(F.Arr);
         } else {
             for (const Csr& A : sigma.Aii[l]) bytes += 64.0 * A.nnz();
             bytes += 64.0 * sigma.Arr[l].nnz();
         }
     }
     if (factors) {
-        bytes += 8.0 * factors->bottom.nnz() + 8.0 * factors->spec.V.size();
-        int m = 0;
-        if (dense_top_cut(factors->bottom, dense_top_min_rows(), 1, &m) != INT_MAX) bytes += 4.0 * m * m;
+        bytes += nodeplan_bytes(factors->bottom) + 8.0 * factors->spec.V.size();
     }
     return (size_t)(bytes * 1.1) + (size_t(4) << 20);
 }
@@ -513,7 +504,7 @@ void Solver::set_sigma_refinement(int steps) {
     if (!sigma) throw std::runtime_error("no interface solver on this context");
     std::vector<const SigmaHost*> hosts;
     for (auto& q : prob) hosts.push_back(&q->sigma);
-    sigma->set_refinement(hosts, steps);
+    sigma->set_refinement(hosts, steps, stream);
     hdd_check(hipStreamSynchronize(stream), "sigma refinement setup");
     // captured applies hold the previous launch sequence
     for (auto& g : graphs) (void)hipGraphExecDestroy(g.exec);

@@ -6,6 +6,7 @@
 #include <vector>
 #include "hdd_device.h"
 #include "hdd_factor.h"
+#include "hdd_nodeplan_device.h"
 #include "hdd_runtime.h"
 #include "hdd_sigma.h"
 #include "hdd_spectral.h"
@@ -22,9 +23,17 @@ struct CsrDev {
 };
 
 // Exact solve x = (A + eps I)^{-1} b for a batch of independent matrices,
-// from their supernodal factors (plan layout in hdd_triplan.h).
+// from their supernodal factors: the dense-node form (hdd_nodeplan.h), or the
+// per-height form (layout in hdd_triplan.h) for refined solves, for batches
+// outside the dense-node form's limits, and where the environment asks for it.
 struct TriPlan {
-    int n = 0, H = -1;
+    int n = 0, H = -1;      // H: tree heights of the per-height form, -1 until it is built
+    bool use_nodes = false;
+    NodePlan nodes;
+    // the factors outlive the plan (the problems a solver holds own them)
+    std::vector<const SupernodalFactor*> F;
+    std::vector<int> offsets, prob_of;
+    void build_heights();
     size_t factor_nnz = 0;
     // per-height ranges and launch parameters (host copies)
     std::vector<int> sn_begin, sl_begin, sl_rows, row_begin, ci_begin, bi_begin, max_sz, big, fused, G, Gc, Gf, Gb, run_begin, run_max;
@@ -35,16 +44,10 @@ struct TriPlan {
     std::vector<int> pgrid;
     static constexpr int kFusedGroups = 1 << 30;
     DBuf<int> run_q, run_n, orig_of, s0, sz, nr, roff, srows, sn_of, sn_prob, sn_list, sl_sn, sl_r0, rowlist, inc_ptr, ci_sn, ci_a0, ci_a1, bi_sn, bi_c, bi_j0;
-    DBuf<long long> loff, doff, cofs, cpos, bofs, woff;
-    DBuf<float> diag, diagT, l21, c, bpart, t, y, w21;
-    // fused heights and heights with big supernodes use W = L21 Linv (one phase less per
-    // fused workgroup, one launch less per big height and pass; float rounding differs from
-    // the L21 form): on unless a fused form is forced (HDD_FUSED_WAVE) or the solves are
-    // refined (the exact mode keeps the L21 form)
-    bool wform = false;
-    bool use_w() const { return wform && refine == 0; }
+    DBuf<long long> loff, doff, cofs, cpos, bofs;
+    DBuf<float> diag, diagT, l21, c, bpart, t, y;
     // prob_of[m]: problem of factor m (empty: all problem 0)
-    void build(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, const std::vector<int>& prob_of = {});
+    void build(const std::vector<const SupernodalFactor*>& factors, const std::vector<int>& offs, const std::vector<int>& probs = {});
     // per-problem flags (device, 1 = iterating): supernodes of stopped problems are skipped; nullptr: none skipped
     const int* active = nullptr;
     // x = (A + eps I)^{-1} b; with refine > 0, each solve is followed by `refine`
@@ -157,7 +160,7 @@ struct SigmaDevice {
     void set_active(const int* active);
     // steps of iterative refinement after every exact solve (0: none, the default)
     int refine_steps = 0;
-    void set_refinement(const std::vector<const SigmaHost*>& hosts, int steps);
+    void set_refinement(const std::vector<const SigmaHost*>& hosts, int steps, hipStream_t stream);
 };
 
 // Device interface solver of a batch: the problems' operators stacked

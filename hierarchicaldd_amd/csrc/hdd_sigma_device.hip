@@ -5,7 +5,9 @@
 //   SIGMA_SMOOTHER::Compute_Residual  IFS/SIGMA_SMOOTHER.cpp:328-352
 //
 // Exact solves with (A + 1e-5 I) use supernodal Cholesky factors (host,
-// double) turned into float triangular-solve plans (hdd_triplan.h). A solve
+// double) turned into float plans: dense nodes in a few levels (hdd_nodeplan.h),
+// or, for refined solves and where the environment asks, the per-height plans
+// of this file (hdd_triplan.h). A per-height solve
 // walks the supernode tree by height (leaves first forward, root first
 // backward); each height is two launches: wavefronts over bounded gather
 // items of the sub-diagonal blocks, then workgroups over row slices of each
@@ -132,8 +134,7 @@ __global__ void __launch_bounds__(256) k_tri_fwd_sn(int q0, int slice_rows, cons
     fwd_sn_slice<G>(q0 + blockIdx.x, slice_rows, sl_sn, sl_r0, s0, sz, doff, diag, tg, inc_ptr, cpos, c, orig_of, b, y, sn_prob, active, ts);
 }
 
-// contributions c_g[a] = L_g[a, :] . v_g for the rows [a0, a1) of an item, G lanes per row:
-// L21 and v = y, or (W form) W = L21 Linv and v = t
+// contributions c_g[a] = L21_g[a, :] . y_g for the rows [a0, a1) of an item, G lanes per row
 template <int G>
 __device__ __forceinline__ void fwd_contrib_item(int it, const int* __restrict__ ci_sn, const int* __restrict__ ci_a0,
                                                  const int* __restrict__ ci_a1, const int* __restrict__ s0, const int* __restrict__ sz,
@@ -168,30 +169,9 @@ __global__ void __launch_bounds__(256) k_tri_fwd_contrib(int i0, int i1, const i
     fwd_contrib_item<G>(it, ci_sn, ci_a0, ci_a1, s0, sz, loff, cofs, l21, y, c, sn_prob, active);
 }
 
-// W form of a height with big supernodes, one launch after the reduce kernel's t:
-// workgroups [0, nq) are the diagonal step's slices (y = Linv t), the others the
-// contribution items (c = W t); neither waits for the other.
-template <int G1, int G2>
-__global__ void __launch_bounds__(256) k_tri_fwd_sn_contrib_w(int q0, int nq, int slice_rows, const int* __restrict__ sl_sn,
-                                                              const int* __restrict__ sl_r0, const int* __restrict__ s0,
-                                                              const int* __restrict__ sz, const long long* __restrict__ doff,
-                                                              const float* __restrict__ diag, const float* __restrict__ t,
-                                                              float* __restrict__ y, int i0, const int* __restrict__ ci_sn,
-                                                              const int* __restrict__ ci_a0, const int* __restrict__ ci_a1,
-                                                              const long long* __restrict__ woff, const long long* __restrict__ cofs,
-                                                              const float* __restrict__ w21, float* __restrict__ c,
-                                                              const int* __restrict__ sn_prob, const int* __restrict__ active) {
-    extern __shared__ float ts[];
-    if ((int)blockIdx.x < nq)
-        fwd_sn_slice<G1>(q0 + blockIdx.x, slice_rows, sl_sn, sl_r0, s0, sz, doff, diag, t, nullptr, nullptr, nullptr, nullptr, nullptr, y,
-                         sn_prob, active, ts);
-    else
-        fwd_contrib_item<G2>(i0 + (int)blockIdx.x - nq, ci_sn, ci_a0, ci_a1, s0, sz, woff, cofs, w21, t, c, sn_prob, active);
-}
-
 // backward tiles: one wavefront per (supernode g, row chunk cc, column block j0);
 // lane j accumulates L_g[a, j] z[rows_g[a]] over the chunk's rows (z: the
-// ancestors' backward results, final; L: L21, or W in the W form)
+// ancestors' backward results, final)
 __device__ __forceinline__ void bwd_tile_item(int it, const int* __restrict__ bi_sn, const int* __restrict__ bi_c,
                                               const int* __restrict__ bi_j0, const int* __restrict__ sz, const int* __restrict__ nr,
                                               const long long* __restrict__ loff, const int* __restrict__ roff,
@@ -228,9 +208,7 @@ __global__ void __launch_bounds__(256) k_tri_bwd_tiles(int i0, int i1, const int
 }
 
 // backward reduce (heights with big supernodes): t_j = y_j - sum over the row
-// chunks of the tile partials of column j of its supernode, G lanes per row.
-// W form (W set): v_j = t_j - (the partials), where t holds Linv^T y, is the
-// result: written to z and to x in the original numbering.
+// chunks of the tile partials of column j of its supernode, G lanes per row
 template <int G>
 __global__ void __launch_bounds__(256) k_tri_bwd_reduce(const int* __restrict__ rows, int nrows, const int* __restrict__ sn_of,
                                                         const int* __restrict__ s0, const int* __restrict__ sz, const int* __restrict__ nr,
@@ -250,36 +228,11 @@ __global__ void __launch_bounds__(256) k_tri_bwd_reduce(const int* __restrict__ 
     if (lane == 0) t[i] = y[i] - s;
 }
 
-template <int G>
-__global__ void __launch_bounds__(256) k_tri_bwd_reduce_w(const int* __restrict__ rows, int nrows, const int* __restrict__ sn_of,
-                                                          const int* __restrict__ s0, const int* __restrict__ sz, const int* __restrict__ nr,
-                                                          const long long* __restrict__ bofs, const float* __restrict__ bpart,
-                                                          const float* __restrict__ t, const int* __restrict__ orig_of,
-                                                          float* __restrict__ z, float* __restrict__ x,
-                                                          const int* __restrict__ sn_prob, const int* __restrict__ active) {
-    const int w = (blockIdx.x * 256 + threadIdx.x) / G, lane = threadIdx.x & (G - 1);
-    if (w >= nrows) return;
-    const int i = rows[w], g = sn_of[i], n = sz[g], k = i - s0[g];
-    if (sn_stopped(sn_prob, active, g)) return;
-    const int nch = (nr[g] + TriPlanHost::kTile - 1) / TriPlanHost::kTile;
-    const float* P = bpart + bofs[g] + k;
-    float s = 0.f;
-#pragma unroll 8
-    for (int cc = lane; cc < nch; cc += G) s += P[(long long)cc * n];
-    s = group_sum<G>(s);
-    if (lane == 0) {
-        const float v = t[i] - s;
-        z[i] = v;
-        x[orig_of[i]] = v;
-    }
-}
-
 // backward diagonal step: t of rows [r0, n) into LDS (reduce output on big
 // heights, else summed here), then z[r] = sum_{k>=r} Linv(k,r) t[k]; y holds
 // the forward result and z the backward one (separate arrays: the slices of
 // one supernode read rows that other slices write); also writes x in the
-// original numbering. With zout set (W form) the input is y itself and the
-// result, Linv^T y, goes to zout only.
+// original numbering
 template <int G>
 __device__ __forceinline__ void bwd_sn_slice(int q, int slice_rows, const int* __restrict__ sl_sn, const int* __restrict__ sl_r0,
                                              const int* __restrict__ s0, const int* __restrict__ sz, const int* __restrict__ nr,
@@ -287,8 +240,7 @@ __device__ __forceinline__ void bwd_sn_slice(int q, int slice_rows, const int* _
                                              const float* __restrict__ tg, const long long* __restrict__ bofs,
                                              const float* __restrict__ bpart, const int* __restrict__ orig_of,
                                              const float* __restrict__ y, float* __restrict__ z, float* __restrict__ x,
-                                             float* __restrict__ zout, const int* __restrict__ sn_prob, const int* __restrict__ active,
-                                             float* ts) {
+                                             const int* __restrict__ sn_prob, const int* __restrict__ active, float* ts) {
     const int g = sl_sn[q], r0 = sl_r0[q], n = sz[g], base = s0[g];
     if (sn_stopped(sn_prob, active, g)) return;
     const int rend = min(n, r0 + slice_rows);
@@ -314,12 +266,8 @@ __device__ __forceinline__ void bwd_sn_slice(int q, int slice_rows, const int* _
         for (int k = r + lane; k < n; k += G) acc += Dr[k] * ts[k];
         acc = group_sum<G>(acc);
         if (lane == 0) {
-            if (zout) {
-                zout[base + r] = acc;
-            } else {
-                z[base + r] = acc;
-                x[orig_of[base + r]] = acc;
-            }
+            z[base + r] = acc;
+            x[orig_of[base + r]] = acc;
         }
     }
 }
@@ -333,34 +281,8 @@ __global__ void __launch_bounds__(256) k_tri_bwd_sn(int q0, int slice_rows, cons
                                                     const float* __restrict__ y, float* __restrict__ z, float* __restrict__ x,
                                                     const int* __restrict__ sn_prob, const int* __restrict__ active) {
     extern __shared__ float ts[];
-    bwd_sn_slice<G>(q0 + blockIdx.x, slice_rows, sl_sn, sl_r0, s0, sz, nr, doff, diagT, tg, bofs, bpart, orig_of, y, z, x, nullptr,
-                    sn_prob, active, ts);
-}
-
-// W form of a height with big supernodes, backward, one launch before the W reduce:
-// workgroups [0, nq) are the diagonal step's slices on y (Linv^T y into zout), the
-// others the tiles of W^T z (four per workgroup); neither waits for the other.
-template <int G>
-__global__ void __launch_bounds__(256) k_tri_bwd_sn_tiles_w(int q0, int nq, int slice_rows, const int* __restrict__ sl_sn,
-                                                            const int* __restrict__ sl_r0, const int* __restrict__ s0,
-                                                            const int* __restrict__ sz, const int* __restrict__ nr,
-                                                            const long long* __restrict__ doff, const float* __restrict__ diagT,
-                                                            const float* __restrict__ y, float* __restrict__ zout, int i0, int i1,
-                                                            const int* __restrict__ bi_sn, const int* __restrict__ bi_c,
-                                                            const int* __restrict__ bi_j0, const long long* __restrict__ woff,
-                                                            const int* __restrict__ roff, const int* __restrict__ srows,
-                                                            const long long* __restrict__ bofs, const float* __restrict__ w21,
-                                                            const float* __restrict__ z, float* __restrict__ bpart,
-                                                            const int* __restrict__ sn_prob, const int* __restrict__ active) {
-    extern __shared__ float ts[];
-    if ((int)blockIdx.x < nq) {
-        bwd_sn_slice<G>(q0 + blockIdx.x, slice_rows, sl_sn, sl_r0, s0, sz, nr, doff, diagT, y, bofs, nullptr, nullptr, nullptr, nullptr,
-                        nullptr, zout, sn_prob, active, ts);
-        return;
-    }
-    const int it = i0 + ((int)blockIdx.x - nq) * 4 + (int)(threadIdx.x >> 6);
-    if (it >= i1) return;
-    bwd_tile_item(it, bi_sn, bi_c, bi_j0, sz, nr, woff, roff, srows, bofs, w21, z, bpart, sn_prob, active);
+    bwd_sn_slice<G>(q0 + blockIdx.x, slice_rows, sl_sn, sl_r0, s0, sz, nr, doff, diagT, tg, bofs, bpart, orig_of, y, z, x, sn_prob,
+                    active, ts);
 }
 
 // Row products of the fused kernels: rows r = threadIdx.x / G + i 256/G below
@@ -426,9 +348,7 @@ __device__ __forceinline__ void row_products(const float* __restrict__ A, int n,
 // launch. Every block entry is loaded once and applied to each member in turn,
 // and each member's sums run in exactly the order of a one-member run.
 // forward: t = b - (incidence sums) -> y = Linv t (LDS) -> c_g = L21_g y.
-// With WF the block passed as l21 is W_g = L21_g Linv_g (formed in double at
-// set-up), so c_g = W_g t needs only t: both products run in one phase.
-template <int G, int M, bool WF, int S>
+template <int G, int M, int S>
 __device__ __forceinline__ void fwd_small_run(int run, int r0, const int* __restrict__ run_q, const int* __restrict__ run_n,
                                                        const int* __restrict__ sn_list, const int* __restrict__ s0,
                                                        const int* __restrict__ sz, const int* __restrict__ nr,
@@ -467,19 +387,19 @@ __device__ __forceinline__ void fwd_small_run(int run, int r0, const int* __rest
         diag + doff[g0], n, n, cnt, ts, [](int) { return 0; }, [](int r) { return r + 1; },
         [&](int r, int j, float v, bool leader) {
             if (leader) {
-                if (!WF) ys[r][j] = v;
+                ys[r][j] = v;
                 y[base_s[j] + r] = v;
             }
         });
-    if (!WF) __syncthreads();  // WF: the contributions read t, complete since the gather
+    __syncthreads();
     row_products<G, M, S>(
-        l21 + loff[g0], n, m, cnt, WF ? ts : ys, [](int) { return 0; }, [n](int) { return n; },
+        l21 + loff[g0], n, m, cnt, ys, [](int) { return 0; }, [n](int) { return n; },
         [&](int a, int j, float v, bool leader) {
             if (leader) c[cofs[sn_list[q0 + j]] + a] = v;
         });
 }
 
-template <int G, int M, bool WF, int S>
+template <int G, int M, int S>
 __global__ void __launch_bounds__(256) k_tri_fwd_small(int r0, int nruns, const int* __restrict__ run_q, const int* __restrict__ run_n,
                                                        const int* __restrict__ sn_list, const int* __restrict__ s0,
                                                        const int* __restrict__ sz, const int* __restrict__ nr,
@@ -490,17 +410,15 @@ __global__ void __launch_bounds__(256) k_tri_fwd_small(int r0, int nruns, const 
                                                        const float* __restrict__ l21, float* __restrict__ c, float* __restrict__ y,
                                                        const int* __restrict__ sn_prob, const int* __restrict__ active) {
     for (int run = blockIdx.x; run < nruns; run += gridDim.x) {
-        fwd_small_run<G, M, WF, S>(run, r0, run_q, run_n, sn_list, s0, sz, nr, doff, diag, inc_ptr, cpos, orig_of, b, loff, cofs, l21, c, y, sn_prob, active);
+        fwd_small_run<G, M, S>(run, r0, run_q, run_n, sn_list, s0, sz, nr, doff, diag, inc_ptr, cpos, orig_of, b, loff, cofs, l21, c, y, sn_prob, active);
         __syncthreads();  // the next run reuses the LDS vectors
     }
 }
 
 // backward: t_j = y_j - sum_a L21_g[a, j] z[rows_g[a]] (four wavefronts split
 // the rows: wavefront w takes rows a = w mod 4 in ascending order; lanes own
-// columns j and j + 64; LDS reduction) -> z = Linv^T t. With WF the block is
-// W_g = L21_g Linv_g and z = Linv^T y - W^T z[rows]: the diagonal product needs
-// no ancestor value and runs beside the tile sums.
-template <int G, int M, bool WF, int S>
+// columns j and j + 64; LDS reduction) -> z = Linv^T t.
+template <int G, int M, int S>
 __device__ __forceinline__ void bwd_small_run(int run, int r0, const int* __restrict__ run_q, const int* __restrict__ run_n,
                                                        const int* __restrict__ sn_list, const int* __restrict__ s0,
                                                        const int* __restrict__ sz, const int* __restrict__ nr,
@@ -514,7 +432,6 @@ __device__ __forceinline__ void bwd_small_run(int run, int r0, const int* __rest
     __shared__ __align__(16) float zr[kChunk][M];  // member-minor, as ts
     __shared__ float part[4][M][S];
     __shared__ __align__(16) float ts[S][M];
-    __shared__ __align__(16) float z1[WF ? S : 1][M];  // WF: Linv^T y
     __shared__ int base_s[M], roff_s[M];
     const int q0 = run_q[r0 + run], cnt = run_n[r0 + run];
     const int g0 = sn_list[q0], n = sz[g0], m = nr[g0];
@@ -530,25 +447,6 @@ __device__ __forceinline__ void bwd_small_run(int run, int r0, const int* __rest
     for (int j = 0; j < M; ++j) { acc0[j] = 0.f; acc1[j] = 0.f; }
     __syncthreads();
     const float* DT = diagT + doff[g0];
-    // WF: Linv^T y into z1, rows and sums as in the diagonal step below
-    auto diag_of_y = [&]() {
-        row_products<G, M, S>(
-            DT, n, n, cnt, ts, [](int r) { return r; }, [n](int) { return n; },
-            [&](int r, int j, float v, bool leader) {
-                if (leader) z1[r][j] = v;
-            });
-    };
-    if (WF) {
-        // t = y, visible after the first chunk's barrier (or the one below without sub-diagonal rows)
-        for (int idx = threadIdx.x; idx < M * n; idx += 256) {
-            const int j = idx / n, k = idx - j * n;
-            ts[k][j] = j < cnt ? y[base_s[j] + k] : 0.f;
-        }
-        if (m == 0) {
-            __syncthreads();
-            diag_of_y();
-        }
-    }
     for (int a0 = 0; a0 < m; a0 += kChunk) {
         const int cm = min(kChunk, m - a0);
         for (int idx = threadIdx.x; idx < M * cm; idx += 256) {
@@ -556,7 +454,6 @@ __device__ __forceinline__ void bwd_small_run(int run, int r0, const int* __rest
             zr[q][j] = j < cnt ? z[srows[roff_s[j] + a0 + q]] : 0.f;
         }
         __syncthreads();
-        if (WF && a0 == 0) diag_of_y();
 #pragma unroll 4
         for (int q = w; q < cm; q += 4) {
             const float* La = L + (long long)(a0 + q) * n;
@@ -580,17 +477,6 @@ __device__ __forceinline__ void bwd_small_run(int run, int r0, const int* __rest
             if (lane + 64 < n) part[w][j][lane + 64] = acc1[j];
         }
     __syncthreads();
-    if (WF) {
-        for (int idx = threadIdx.x; idx < M * n; idx += 256) {
-            const int j = idx / n, k = idx - j * n;
-            if (j < cnt) {
-                const float v = z1[k][j] - ((part[0][j][k] + part[1][j][k]) + (part[2][j][k] + part[3][j][k]));
-                z[base_s[j] + k] = v;
-                x[orig_of[base_s[j] + k]] = v;
-            }
-        }
-        return;
-    }
     for (int idx = threadIdx.x; idx < M * n; idx += 256) {
         const int j = idx / n, k = idx - j * n;
         ts[k][j] = j < cnt ? y[base_s[j] + k] - ((part[0][j][k] + part[1][j][k]) + (part[2][j][k] + part[3][j][k])) : 0.f;
@@ -606,7 +492,7 @@ __device__ __forceinline__ void bwd_small_run(int run, int r0, const int* __rest
         });
 }
 
-template <int G, int M, bool WF, int S>
+template <int G, int M, int S>
 __global__ void __launch_bounds__(256) k_tri_bwd_small(int r0, int nruns, const int* __restrict__ run_q, const int* __restrict__ run_n,
                                                        const int* __restrict__ sn_list, const int* __restrict__ s0,
                                                        const int* __restrict__ sz, const int* __restrict__ nr,
@@ -617,7 +503,7 @@ __global__ void __launch_bounds__(256) k_tri_bwd_small(int r0, int nruns, const 
                                                        float* __restrict__ z, float* __restrict__ x,
                                                        const int* __restrict__ sn_prob, const int* __restrict__ active) {
     for (int run = blockIdx.x; run < nruns; run += gridDim.x) {
-        bwd_small_run<G, M, WF, S>(run, r0, run_q, run_n, sn_list, s0, sz, nr, roff, srows, loff, l21, doff, diagT, orig_of, y, z, x, sn_prob, active);
+        bwd_small_run<G, M, S>(run, r0, run_q, run_n, sn_list, s0, sz, nr, roff, srows, loff, l21, doff, diagT, orig_of, y, z, x, sn_prob, active);
         __syncthreads();  // the next run reuses the LDS vectors
     }
 }
@@ -1113,13 +999,30 @@ static void dense_top_inverse(const TriPlanHost::TopBlock& B, float* P) {
     hdd_check(hipStreamSynchronize(nullptr), "dense top");
 }
 
-void TriPlan::build(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, const std::vector<int>& prob_of) {
+// HDD_DENSE_TOP or HDD_FUSED_WAVE in the environment asks for the per-height form
+static bool heights_forced() {
+    const char* top = std::getenv("HDD_DENSE_TOP");
+    const char* wave = std::getenv("HDD_FUSED_WAVE");
+    return (top && *top) || (wave && (std::string(wave) == "0" || std::string(wave) == "1"));
+}
+
+void TriPlan::build(const std::vector<const SupernodalFactor*>& factors, const std::vector<int>& offs, const std::vector<int>& probs) {
+    F = factors; offsets = offs; prob_of = probs;
+    for (size_t m = 0; m < F.size(); ++m) { n = std::max(n, offsets[m] + F[m]->n); factor_nnz += F[m]->nnz(); }
+    if (n == 0) return;
+    auto tp = std::chrono::steady_clock::now();
+    use_nodes = !heights_forced() && nodes.build(F, offsets, prob_of);
+    setup_phase("  dense-node plan", (int)F.size(), tp, "factors");
+    if (!use_nodes) build_heights();
+}
+
+void TriPlan::build_heights() {
+    if (n == 0 || H >= 0) return;
     TriPlanHost P;
     auto tp = std::chrono::steady_clock::now();
     build_triplan(F, offsets, P, dense_top_min_rows());
     setup_phase("  plan lists and float blocks", (int)F.size(), tp, "factors");
-    n = P.n; H = P.H; factor_nnz = P.factor_nnz;
-    if (n == 0) return;
+    H = P.H;
     {
         // problem of each supernode (supernodes are numbered factor by factor, in order)
         std::vector<int> sp(P.s0.size(), 0);
@@ -1138,7 +1041,6 @@ void TriPlan::build(const std::vector<const SupernodalFactor*>& F, const std::ve
         const char* e = std::getenv("HDD_FUSED_WAVE");
         wave_forced = e && (std::string(e) == "0" || std::string(e) == "1");
         wave.assign(P.H + 1, wave_forced && std::string(e) == "1" ? 1 : 0);
-        wform = !wave_forced && !P.w21.empty();
     }
     pgrid.assign(P.H + 1, kFusedGroups);
     run_q.upload(P.run_q); run_n.upload(P.run_n);
@@ -1148,7 +1050,6 @@ void TriPlan::build(const std::vector<const SupernodalFactor*>& F, const std::ve
     ci_sn.upload(P.ci_sn); ci_a0.upload(P.ci_a0); ci_a1.upload(P.ci_a1); bi_sn.upload(P.bi_sn); bi_c.upload(P.bi_c); bi_j0.upload(P.bi_j0);
     loff.upload(P.loff); doff.upload(P.doff); cofs.upload(P.cofs); cpos.upload(P.cpos); bofs.upload(P.bofs);
     diag.upload(P.diag); diagT.upload(P.diagT); l21.upload(P.l21);
-    if (wform) { woff.upload(P.woff); w21.upload(P.w21); }
     c.alloc(std::max<long long>(1, P.c_size)); bpart.alloc(std::max<long long>(1, P.bpart_size));
     t.alloc(n); y.alloc(2 * (size_t)n);  // forward result, then backward result
     setup_phase("  plan uploaded", (int)F.size(), tp, "factors");
@@ -1175,9 +1076,9 @@ void TriPlan::build(const std::vector<const SupernodalFactor*>& F, const std::ve
 }
 
 size_t TriPlan::bytes() const {
-    return (run_q.n + run_n.n + orig_of.n + s0.n + sz.n + nr.n + roff.n + srows.n + sn_of.n + sn_prob.n + sn_list.n + sl_sn.n + sl_r0.n + rowlist.n + inc_ptr.n + ci_sn.n + ci_a0.n +
+    return nodes.bytes() + (run_q.n + run_n.n + orig_of.n + s0.n + sz.n + nr.n + roff.n + srows.n + sn_of.n + sn_prob.n + sn_list.n + sl_sn.n + sl_r0.n + rowlist.n + inc_ptr.n + ci_sn.n + ci_a0.n +
             ci_a1.n + bi_sn.n + bi_c.n + bi_j0.n) * 4 +
-           (loff.n + doff.n + cofs.n + cpos.n + bofs.n + woff.n) * 8 + (diag.n + diagT.n + l21.n + c.n + bpart.n + t.n + y.n + w21.n) * 4 +
+           (loff.n + doff.n + cofs.n + cpos.n + bofs.n) * 8 + (diag.n + diagT.n + l21.n + c.n + bpart.n + t.n + y.n) * 4 +
            (top_rows.n + top_of.n + top_inc_ptr.n + top_base.n + top_ld.n + top_W.n + top_t.n) * 4 + (top_cpos.n + top_woff.n) * 8;
 }
 
@@ -1202,34 +1103,28 @@ static constexpr int kRunM = TriPlanHost::kRunMembers;
         }                                                                                                       \
     } while (0)
 
-#define HDD_RUN_WF_DISPATCH(G, M, WF, S64, KERNEL, BLOCKS, STREAM, ...)                                             \
+#define HDD_RUN_S_DISPATCH(G, M, S64, KERNEL, BLOCKS, STREAM, ...)                                             \
     do {                                                                                                            \
         switch (G) {                                                                                                \
             case 4:                                                                                                 \
-                if (S64) hipLaunchKernelGGL((KERNEL<4, M, WF, 64>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); \
-                else hipLaunchKernelGGL((KERNEL<4, M, WF, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__);    \
+                if (S64) hipLaunchKernelGGL((KERNEL<4, M, 64>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); \
+                else hipLaunchKernelGGL((KERNEL<4, M, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__);    \
                 break;                                                                                              \
             case 8:                                                                                                 \
-                if (S64) hipLaunchKernelGGL((KERNEL<8, M, WF, 64>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); \
-                else hipLaunchKernelGGL((KERNEL<8, M, WF, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__);    \
+                if (S64) hipLaunchKernelGGL((KERNEL<8, M, 64>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); \
+                else hipLaunchKernelGGL((KERNEL<8, M, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__);    \
                 break;                                                                                              \
-            case 16: hipLaunchKernelGGL((KERNEL<16, M, WF, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); break; \
-            case 32: hipLaunchKernelGGL((KERNEL<32, M, WF, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); break; \
-            default: hipLaunchKernelGGL((KERNEL<64, M, WF, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); break; \
+            case 16: hipLaunchKernelGGL((KERNEL<16, M, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); break; \
+            case 32: hipLaunchKernelGGL((KERNEL<32, M, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); break; \
+            default: hipLaunchKernelGGL((KERNEL<64, M, 128>), dim3(BLOCKS), dim3(256), 0, STREAM, __VA_ARGS__); break; \
         }                                                                                                           \
     } while (0)
-// the fused workgroup kernels: run length (runs of one or of up to kRunM) x block form (L21 or W);
-// at 4 and 8 lanes per row, heights whose supernodes have at most 64 rows take the 64-row
-// form (half the fixed trip count and registers, the same sums: level-0 Aii 711 -> 691 us)
-#define HDD_FUSED_DISPATCH(H, WF, KERNEL, BLOCKS, STREAM, ...)                                                       \
-    do {                                                                                                            \
-        if (run_max[H] > 1) {                                                                                       \
-            if (WF) HDD_RUN_WF_DISPATCH(G[H], kRunM, true, max_sz[H] <= 64, KERNEL, BLOCKS, STREAM, __VA_ARGS__);    \
-            else HDD_RUN_WF_DISPATCH(G[H], kRunM, false, max_sz[H] <= 64, KERNEL, BLOCKS, STREAM, __VA_ARGS__);      \
-        } else {                                                                                                    \
-            if (WF) HDD_RUN_WF_DISPATCH(G[H], 1, true, max_sz[H] <= 64, KERNEL, BLOCKS, STREAM, __VA_ARGS__);        \
-            else HDD_RUN_WF_DISPATCH(G[H], 1, false, max_sz[H] <= 64, KERNEL, BLOCKS, STREAM, __VA_ARGS__);          \
-        }                                                                                                           \
+// the fused workgroup kernels: runs of one or of up to kRunM; at 4 and 8 lanes per row, heights whose
+// supernodes have at most 64 rows take the 64-row form (half the fixed trip count and registers, the same sums)
+#define HDD_FUSED_DISPATCH(H, KERNEL, BLOCKS, STREAM, ...)                                                      \
+    do {                                                                                                        \
+        if (run_max[H] > 1) HDD_RUN_S_DISPATCH(G[H], kRunM, max_sz[H] <= 64, KERNEL, BLOCKS, STREAM, __VA_ARGS__); \
+        else HDD_RUN_S_DISPATCH(G[H], 1, max_sz[H] <= 64, KERNEL, BLOCKS, STREAM, __VA_ARGS__);                  \
     } while (0)
 
 #define HDD_ROWS_DISPATCH(G, KERNEL, ROWS, ...)                                                                \
@@ -1240,28 +1135,6 @@ static constexpr int kRunM = TriPlanHost::kRunMembers;
         case 32: hipLaunchKernelGGL(KERNEL<32>, dim3(blocks_for((ROWS) * 32, 256)), dim3(256), 0, __VA_ARGS__); break; \
         default: hipLaunchKernelGGL(KERNEL<64>, dim3(blocks_for((ROWS) * 64, 256)), dim3(256), 0, __VA_ARGS__); break; \
     }
-
-// k_tri_fwd_sn_contrib_w with the diagonal step's and the contributions' lanes per row
-template <int G1, class... A>
-static void launch_fwd_w_g2(int g2, unsigned grid, size_t shmem, hipStream_t s, A... a) {
-    switch (g2) {
-        case 4: hipLaunchKernelGGL((k_tri_fwd_sn_contrib_w<G1, 4>), dim3(grid), dim3(256), shmem, s, a...); break;
-        case 8: hipLaunchKernelGGL((k_tri_fwd_sn_contrib_w<G1, 8>), dim3(grid), dim3(256), shmem, s, a...); break;
-        case 16: hipLaunchKernelGGL((k_tri_fwd_sn_contrib_w<G1, 16>), dim3(grid), dim3(256), shmem, s, a...); break;
-        case 32: hipLaunchKernelGGL((k_tri_fwd_sn_contrib_w<G1, 32>), dim3(grid), dim3(256), shmem, s, a...); break;
-        default: hipLaunchKernelGGL((k_tri_fwd_sn_contrib_w<G1, 64>), dim3(grid), dim3(256), shmem, s, a...); break;
-    }
-}
-template <class... A>
-static void launch_fwd_w(int g1, int g2, unsigned grid, size_t shmem, hipStream_t s, A... a) {
-    switch (g1) {
-        case 4: launch_fwd_w_g2<4>(g2, grid, shmem, s, a...); break;
-        case 8: launch_fwd_w_g2<8>(g2, grid, shmem, s, a...); break;
-        case 16: launch_fwd_w_g2<16>(g2, grid, shmem, s, a...); break;
-        case 32: launch_fwd_w_g2<32>(g2, grid, shmem, s, a...); break;
-        default: launch_fwd_w_g2<64>(g2, grid, shmem, s, a...); break;
-    }
-}
 
 void TriPlan::fwd_height(int h, const float* b, hipStream_t s) {
     float* yf = y.p;
@@ -1283,13 +1156,10 @@ void TriPlan::fwd_height(int h, const float* b, hipStream_t s) {
                                      (const long long*)loff.p, (const long long*)cofs.p, (const float*)l21.p, c.p, yf, SP, active);
             } else if (nr_) {
                 const int grid = std::min(nr_, pgrid[h]);
-                const bool wf = use_w();
-                const long long* blo = wf ? woff.p : loff.p;
-                const float* blk = wf ? w21.p : l21.p;
-                HDD_FUSED_DISPATCH(h, wf, k_tri_fwd_small, grid, s, r0, nr_, (const int*)run_q.p, (const int*)run_n.p, (const int*)sn_list.p,
+                HDD_FUSED_DISPATCH(h, k_tri_fwd_small, grid, s, r0, nr_, (const int*)run_q.p, (const int*)run_n.p, (const int*)sn_list.p,
                                    (const int*)s0.p, (const int*)sz.p, (const int*)nr.p, (const long long*)doff.p, (const float*)diag.p,
-                                   (const int*)inc_ptr.p, (const long long*)cpos.p, (const int*)orig_of.p, b, blo, (const long long*)cofs.p,
-                                   blk, c.p, yf, SP, active);
+                                   (const int*)inc_ptr.p, (const long long*)cpos.p, (const int*)orig_of.p, b, (const long long*)loff.p,
+                                   (const long long*)cofs.p, (const float*)l21.p, c.p, yf, SP, active);
             }
             return;
         }
@@ -1299,16 +1169,6 @@ void TriPlan::fwd_height(int h, const float* b, hipStream_t s) {
             HDD_ROWS_DISPATCH(Gf[h], k_tri_fwd_reduce, nrows, s, rows, nrows, (const int*)inc_ptr.p, (const long long*)cpos.p,
                               (const float*)c.p, (const int*)orig_of.p, b, t.p, (const int*)sn_of.p, SP, active);
         const int q0 = sl_begin[h], nq = sl_begin[h + 1] - sl_begin[h];
-        if (big[h] && use_w()) {
-            // W form: the slices (y = Linv t) and the contribution items (c = W t) in one launch
-            const int i0 = ci_begin[h], ni = ci_begin[h + 1] - ci_begin[h];
-            if (nq + ni)
-                launch_fwd_w(G[h], Gc[h], (unsigned)(nq + ni), (size_t)max_sz[h] * sizeof(float), s, q0, nq, sl_rows[h], (const int*)sl_sn.p,
-                             (const int*)sl_r0.p, (const int*)s0.p, (const int*)sz.p, (const long long*)doff.p, (const float*)diag.p,
-                             (const float*)t.p, yf, i0, (const int*)ci_sn.p, (const int*)ci_a0.p, (const int*)ci_a1.p,
-                             (const long long*)woff.p, (const long long*)cofs.p, (const float*)w21.p, c.p, SP, active);
-            return;
-        }
         if (nq)
             HDD_SN_DISPATCH(G[h], k_tri_fwd_sn, nq, (size_t)max_sz[h] * sizeof(float), s, q0, sl_rows[h], (const int*)sl_sn.p, (const int*)sl_r0.p,
                             (const int*)s0.p, (const int*)sz.p, (const long long*)doff.p, (const float*)diag.p,
@@ -1343,35 +1203,13 @@ void TriPlan::bwd_height(int h, float* x, hipStream_t s) {
                                      (const float*)diagT.p, (const int*)orig_of.p, (const float*)yf, zb, x, SP, active);
             } else if (nr_) {
                 const int grid = std::min(nr_, pgrid[h]);
-                const bool wf = use_w();
-                const long long* blo = wf ? woff.p : loff.p;
-                const float* blk = wf ? w21.p : l21.p;
-                HDD_FUSED_DISPATCH(h, wf, k_tri_bwd_small, grid, s, r0, nr_, (const int*)run_q.p, (const int*)run_n.p, (const int*)sn_list.p,
-                                   (const int*)s0.p, (const int*)sz.p, (const int*)nr.p, (const int*)roff.p, (const int*)srows.p, blo, blk,
-                                   (const long long*)doff.p, (const float*)diagT.p, (const int*)orig_of.p, (const float*)yf, zb, x, SP, active);
+                HDD_FUSED_DISPATCH(h, k_tri_bwd_small, grid, s, r0, nr_, (const int*)run_q.p, (const int*)run_n.p, (const int*)sn_list.p,
+                                   (const int*)s0.p, (const int*)sz.p, (const int*)nr.p, (const int*)roff.p, (const int*)srows.p, (const long long*)loff.p,
+                                   (const float*)l21.p, (const long long*)doff.p, (const float*)diagT.p, (const int*)orig_of.p, (const float*)yf, zb, x, SP, active);
             }
             return;
         }
         const int i0 = bi_begin[h], ni = bi_begin[h + 1] - bi_begin[h];
-        if (big[h] && use_w()) {
-            // W form: the slices (Linv^T y into t) and the tiles of W^T z in one launch, then
-            // z = t - (the tile partials) row by row
-            const int q0 = sl_begin[h], nq = sl_begin[h + 1] - sl_begin[h];
-            const int grid = nq + (int)blocks_for(ni, 4);
-            if (grid)
-                HDD_SN_DISPATCH(G[h], k_tri_bwd_sn_tiles_w, grid, (size_t)max_sz[h] * sizeof(float), s, q0, nq, sl_rows[h], (const int*)sl_sn.p,
-                                (const int*)sl_r0.p, (const int*)s0.p, (const int*)sz.p, (const int*)nr.p, (const long long*)doff.p,
-                                (const float*)diagT.p, (const float*)yf, t.p, i0, i0 + ni, (const int*)bi_sn.p, (const int*)bi_c.p,
-                                (const int*)bi_j0.p, (const long long*)woff.p, (const int*)roff.p, (const int*)srows.p, (const long long*)bofs.p,
-                                (const float*)w21.p, (const float*)zb, bpart.p, SP, active);
-            const int nrows = row_begin[h + 1] - row_begin[h];
-            const int* rows = rowlist.p + row_begin[h];
-            if (nrows)
-                HDD_ROWS_DISPATCH(Gb[h], k_tri_bwd_reduce_w, nrows, s, rows, nrows, (const int*)sn_of.p, (const int*)s0.p, (const int*)sz.p,
-                                  (const int*)nr.p, (const long long*)bofs.p, (const float*)bpart.p, (const float*)t.p, (const int*)orig_of.p,
-                                  zb, x, SP, active);
-            return;
-        }
         if (ni)
             hipLaunchKernelGGL(k_tri_bwd_tiles, dim3(blocks_for(ni, 4)), dim3(256), 0, s, i0, i0 + ni, (const int*)bi_sn.p, (const int*)bi_c.p,
                                (const int*)bi_j0.p, (const int*)sz.p, (const int*)nr.p, (const long long*)loff.p, (const int*)roff.p,
@@ -1405,6 +1243,8 @@ void TriPlan::top_solve(const float* b, float* x, hipStream_t s) {
 
 void TriPlan::solve_once(const float* b, float* x, hipStream_t s) {
     if (n == 0) return;
+    // refined solves keep the per-height form, whose rounding the reference-exact histories were checked with
+    if (use_nodes && refine == 0) { nodes.solve(b, x, active, s); return; }
     for (int h = 0; h <= H; ++h) fwd_height(h, b, s);
     if (top_nq) top_solve(b, x, s);
     for (int h = H; h >= 0; --h) bwd_height(h, x, s);
@@ -1457,7 +1297,7 @@ void TriPlan::rebuild_lists(hipStream_t s) {
 // choice changes the order of any sum, so the solve's results do not depend on
 // what the timings pick.
 int TriPlan::tune(hipStream_t s) {
-    if (n < kTuneMinRows) return 0;  // small plans: every launch is latency-bound, little to choose
+    if (n < kTuneMinRows || H < 0) return 0;  // small plans: every launch is latency-bound, little to choose
     // capacity for the largest lists any candidate produces (8-row slices, 1024-entry items)
     {
         const std::vector<int> keep_sl = sl_rows, keep_ci = ci_entries;
@@ -1487,7 +1327,7 @@ int TriPlan::tune(hipStream_t s) {
     int changed = 0;
     for (int h = 0; h <= H; ++h) {
         if (fused[h]) {
-            // a workgroup or a wavefront per run (L21 form): the same bits, whichever is faster
+            // a workgroup or a wavefront per run: the same bits, whichever is faster
             if (run_begin[h + 1] == run_begin[h]) continue;
             // workgroups of the persistent launch (each loops over runs): a cap, or one per run
             float best = time_height(h);
@@ -1500,8 +1340,7 @@ int TriPlan::tune(hipStream_t s) {
                 else pgrid[h] = keep;
             }
             changed += pgrid[h] != p0;
-            // the wavefront form has the L21 blocks only: not a candidate beside the W form
-            if (wave_forced || wform) continue;
+            if (wave_forced) continue;
             wave[h] = 1;
             const float t_wave = time_height(h);
             if (!(t_wave < 0.97f * best)) wave[h] = 0;
@@ -1940,7 +1779,7 @@ void SigmaDevice::vcycle(hipStream_t s, bool first) {
 // single-precision PARDISO solves have no counterpart): the plans' matrices are
 // rebuilt from the host operators in the plans' numbering, problems and
 // subdomains in the order make_sigma_device lays them out.
-void SigmaDevice::set_refinement(const std::vector<const SigmaHost*>& hosts, int steps) {
+void SigmaDevice::set_refinement(const std::vector<const SigmaHost*>& hosts, int steps, hipStream_t stream) {
     if (steps < 0 || steps > 3) throw std::runtime_error("sigma refinement: steps must be 0..3");
     const int NP = (int)hosts.size();
     if (NP != nprob) throw std::runtime_error("sigma refinement: one host operator set per problem");
@@ -1977,6 +1816,20 @@ void SigmaDevice::set_refinement(const std::vector<const SigmaHost*>& hosts, int
             cb.cols = cb.rows;
             if (cb.rows != Lbottom.n) throw std::runtime_error("sigma refinement: bottom system size differs from its plan");
             Lbottom.refA.upload(cb); Lbottom.ref_r.alloc(cb.rows); Lbottom.ref_d.alloc(cb.rows);
+        }
+    }
+    if (steps > 0) {
+        // the per-height plans the refined solves use, built on their first use
+        std::vector<TriPlan*> plans;
+        for (auto& L : lv) { plans.push_back(&L.Lii); plans.push_back(&L.Lrr); }
+        plans.push_back(&Lbottom);
+        for (TriPlan* p : plans) {
+            if (p->n == 0 || p->H >= 0) continue;
+            plan_bytes -= p->bytes();
+            p->build_heights();
+            if (autotune()) tuned_choices += p->tune(stream);
+            plan_bytes += p->bytes();
+            dense_top_rows += p->top_dense_rows;
         }
     }
     refine_steps = steps;

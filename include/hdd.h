@@ -359,26 +359,25 @@ hdd_status hdd_profile_copy(hdd_ctx* ctx, int reps, double* avg_ms, double* byte
  * eigenmodes in that correction, out[10] seconds of its eigen-solve, out[11]
  * block Krylov steps of it (0: dense), out[12] relative max difference of that
  * evaluation against the 200 smooths on a random right-hand side (-1: not run),
- * out[13] launch shapes of the triangular-solve plans that the setup's
- * autotuner changed from their defaults (HDD_AUTOTUNE=0 in the environment
- * turns it off; results do not depend on it), out[14] rows of the dense top
- * blocks of the triangular-solve plans (each tall tree's top heights solved as
- * two dense triangular matvecs; HDD_DENSE_TOP=0 in the environment turns them
- * off, HDD_DENSE_TOP=k gives a dense top to factors of at least k rows, 4096
- * by default), out[15] 1 if the interior V-cycle's 200 coarsest-level sweeps
+ * out[13] launch shapes of the per-height triangular-solve plans that the
+ * setup's autotuner changed from their defaults (HDD_AUTOTUNE=0 in the
+ * environment turns it off; results do not depend on it), out[14] rows of the
+ * dense top blocks of the per-height plans (each tall tree's top heights solved
+ * as two dense triangular matvecs; HDD_DENSE_TOP=0 in the environment turns
+ * them off, HDD_DENSE_TOP=k gives a dense top to factors of at least k rows,
+ * 4096 by default), out[15] 1 if the interior V-cycle's 200 coarsest-level sweeps
  * run page by page in one launch (bit-identical to 200 launches; set-up picks
  * it when that level's Active cells couple only within their pages,
- * HDD_BOTTOM_LOCAL=0 turns it off), else 0, out[16] tree heights of the
- * triangular-solve plans done by one fused launch per height (a workgroup or
- * a wavefront per run of supernodes), out[17] how many of those use the
- * wavefront form. By default the fused heights and the heights with big
- * supernodes use the W form (their sub-diagonal blocks stored as
- * W = L21 Linv: one dependent phase less per fused workgroup, two launches
- * instead of three per big height and pass) with a workgroup per run;
- * HDD_FUSED_WAVE=1 / 0 in the environment forces the L21 form with a
- * wavefront / a workgroup per run (the same bits as each other; the W form
- * rounds differently), and refined solves (hdd_set_sigma_refinement) use the
- * L21 form.
+ * HDD_BOTTOM_LOCAL=0 turns it off), else 0, out[16] levels of the dense-node
+ * plans (one launch per level and pass), plus tree heights of the per-height
+ * plans done by one fused launch per height (a workgroup or a wavefront per run
+ * of supernodes), out[17] how many of those heights use the wavefront form.
+ * The exact solves use the dense-node plans: the elimination trees cut into a
+ * few levels of dense nodes. The per-height plans (a launch or more per tree
+ * height) are built where HDD_DENSE_TOP=k or HDD_FUSED_WAVE=1 / 0 (a wavefront /
+ * a workgroup per run, the same bits) is set in the environment at set-up, for
+ * separators beyond the dense nodes' limits, and for refined solves at the first
+ * hdd_set_sigma_refinement with steps > 0; they round differently.
  * n = number of slots provided (up to 18). No reference counterpart. */
 hdd_status hdd_stats(const hdd_ctx* ctx, double* out, int n);
 
