@@ -35,13 +35,22 @@ void upload_constants();
 // V-cycle kernels, float storage and half (FP16) storage with float arithmetic
 void launch_smooth(const DevLevel& L, const float* u_in, float* u_out, const float* b, bool interior, bool boundary, hipStream_t s);
 void launch_smooth(const DevLevel& L, const __half* u_in, __half* u_out, const __half* b, bool interior, bool boundary, hipStream_t s);
-// `count` sweeps (interior and boundary) of a level whose Active cells couple only within clusters of at most
-// four pages, in one launch: nwg workgroups of four page slots (wg_page, -1: empty), nb_slot[p*6+f] the slot
-// of page p's face-f neighbour when it is in p's cluster, else -1
-void launch_smooth_local(const DevLevel& L, const int* wg_page, int nwg, const int* nb_slot, const float* u_in, float* u_out,
-                         const float* b, int count, hipStream_t s);
-void launch_smooth_local(const DevLevel& L, const int* wg_page, int nwg, const int* nb_slot, const __half* u_in, __half* u_out,
-                         const __half* b, int count, hipStream_t s);
+// Sweeps of a level whose Active cells couple only within small clusters of pages, several in one
+// launch (k_cluster_sweeps): workgroups of `slots` page slots hold whole clusters in LDS.
+struct DevClusters {
+    int nwg = 0, slots = 0, entries = 0;       // workgroups, page slots each, LDS values (the slots' cells, then the halo)
+    const int* wg_page = nullptr;              // [nwg*slots] page of each slot, -1: empty
+    const uint16_t* nbr = nullptr;             // [nwg][6][slots*256] LDS value of each cell's face neighbour (its own where the face bit is not set)
+    const int *halo_ptr = nullptr, *halo_cell = nullptr;  // values past the slots' cells: cells of the level ([nwg+1], then the lists)
+};
+// in turn: count[i] sweeps of the interior (kSweepInterior) and / or boundary (kSweepBoundary) cells
+enum { kSweepInterior = 1, kSweepBoundary = 2 };
+struct SweepPhases { int n = 0, count[3] = {0, 0, 0}, cells[3] = {0, 0, 0}; };
+// u in place; u_zero: u is zero at the start (and not read); r (may be nullptr): the residual after the sweeps
+void launch_cluster_sweeps(const DevLevel& L, const DevClusters& C, float* u, const float* b, float* r, const SweepPhases& ph, bool u_zero,
+                           hipStream_t s);
+void launch_cluster_sweeps(const DevLevel& L, const DevClusters& C, __half* u, const __half* b, __half* r, const SweepPhases& ph,
+                           bool u_zero, hipStream_t s);
 void launch_residual(const DevLevel& L, const float* u, const float* b, float* r, hipStream_t s);
 void launch_residual(const DevLevel& L, const __half* u, const __half* b, __half* r, hipStream_t s);
 void launch_fill(float* a, float v, size_t n, hipStream_t s);

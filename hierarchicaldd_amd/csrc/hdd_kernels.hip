@@ -58,6 +58,9 @@ __device__ __forceinline__ float ld(const float* __restrict__ p, size_t i) { ret
 __device__ __forceinline__ float ld(const __half* __restrict__ p, size_t i) { return __half2float(p[i]); }
 __device__ __forceinline__ void st(float* __restrict__ p, size_t i, float v) { p[i] = v; }
 __device__ __forceinline__ void st(__half* __restrict__ p, size_t i, float v) { p[i] = __float2half_rn(v); }
+// v as a store and load through the storage type would give it
+__device__ __forceinline__ float stored(const float*, float v) { return v; }
+__device__ __forceinline__ float stored(const __half*, float v) { return __half2float(__float2half_rn(v)); }
 
 // Stencil sweeps: one 64-lane wavefront per page, lane l owns the four cells
 // 4l .. 4l+3 (z = 4(l&1) .. +3 of row x = l>>4, y = (l>>1)&7) and moves them
@@ -153,71 +156,105 @@ __global__ void __launch_bounds__(64 * kSweepPages) k_smooth(DevLevel L, const S
     st4(u_out, (size_t)p * 64 + l, out);
 }
 
-// All `count` sweeps (interior and boundary cells) of a level whose Active
-// cells couple only within small clusters of pages (the bottom of the V-cycle:
-// each subdomain's coarsest block lies in one or two pages). A workgroup holds
-// up to four pages, whole clusters (wg_page, -1 for an empty slot), 256
-// threads per page, thread t owning cell t, and sweeps them in LDS with the
-// operations of Stencil4 and k_smooth, storing every iterate in the level's
-// storage type, so the result is bit-identical to `count` launches of
-// k_smooth. A face neighbour page of the same cluster is read from its LDS
-// slot (nb_slot[p*6+f], -1: none); other neighbour pages hold no cell a
-// coupled Active cell reads that a sweep writes, so they are read once. Every
-// thread takes part in the barriers; only those of a live page compute. The
-// result goes to u_out, a buffer other than u_in (other workgroups read u_in's
-// pages).
-template <class S>
-__global__ void __launch_bounds__(1024) k_smooth_local(DevLevel L, const int* __restrict__ wg_page, const int* __restrict__ nb_slot,
-                                                       const S* __restrict__ u_in, S* __restrict__ u_out, const S* __restrict__ b,
-                                                       int count) {
-    __shared__ S us[2][4][kPageCells];
-    const int c = threadIdx.x & 255, w = threadIdx.x >> 8;
-    const int p = wg_page[blockIdx.x * 4 + w];
-    const bool live = p >= 0 && !page_stopped(L, p);
-    const int x = c >> 6, y = (c >> 3) & 7, z = c & 7;
-    // per face: the in-page neighbour cell, or (at the page face) the
-    // neighbour page's cell, read from its LDS slot or once from u_in
-    const int nc[6] = {x > 0 ? c - 64 : c + 192, x < 3 ? c + 64 : c - 192, y > 0 ? c - 8 : c + 56,
-                       y < 7 ? c + 8 : c - 56, z > 0 ? c - 1 : c + 7, z < 7 ? c + 1 : c - 7};
-    const bool inside[6] = {x > 0, x < 3, y > 0, y < 7, z > 0, z < 7};
-    int slot[6];
-    float cst[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    uint32_t f = 0u;
-    float bv = 0.f, wgt = 0.f;
-    if (live) {
-        f = L.flags[(size_t)p * 256 + c];
-        const uint32_t sel = f & (kActive | kBoundary);
-        if (sel == kActive || sel == (kActive | kBoundary)) wgt = c_omega_fc[__popc(f & (0x3fu * kFaceMX))];
+// Several sweeps of a level in one launch, and the residual after them, where
+// its Active cells couple only within small clusters of pages (the coarse
+// levels: a cluster is the part of a subdomain, or of a few that meet inside an
+// obstacle). A workgroup holds whole clusters in LDS, C cells per thread
+// (cell i of thread t: i * blockDim + t of the workgroup's slots * 256), and
+// sweeps them with the operations of Stencil4 and k_smooth, keeping every
+// iterate in the level's storage type, so the result is bit-identical to one
+// launch per sweep. nbr gives each cell's face neighbours as LDS values; a
+// neighbour outside the workgroup is a cell no sweep writes, held in the halo
+// behind the slots' cells. Where a face bit is not set it names the cell itself,
+// whose difference is an exact zero. The cells ping-pong between two copies (the
+// halo is in both), one barrier per sweep. u is updated in place: no other
+// workgroup reads the Active cells of this one's pages.
+//
+// Bound by instruction issue and the barrier: a sweep is 6 LDS reads, about 25
+// operations and one write per cell, against a launch of 3.3-5 us per sweep of a
+// small level. The 200 sweeps of a V-cycle's bottom take 36 us where clusters are
+// single pages (71 with four pages to every workgroup, whose 16 waves share the
+// barrier), 51 us at up to four pages (200 launches: 650), 76 us at up to eight;
+// the seven sweeps and the residual of a small level 5-12 us instead of 35.
+// More than 32 pages would spill (68 us for the seven sweeps of 46-page clusters
+// at 100^3, 45 us as launches), so those levels keep one launch per sweep.
+template <class S, int C>
+__global__ void __launch_bounds__(1024) k_cluster_sweeps(DevLevel L, DevClusters W, S* u, const S* __restrict__ b, S* __restrict__ r,
+                                                         SweepPhases ph, int u_zero) {
+    extern __shared__ __align__(16) unsigned char cluster_lds[];
+    S* us = reinterpret_cast<S*>(cluster_lds);
+    const int wg = blockIdx.x, nt = blockDim.x, cells = W.slots * kPageCells;
+    float cur[C], bv[C], wgt[C];
+    unsigned nb[C][3];    // LDS values of the six face neighbours, two per register
+    unsigned kind = 0;    // two bits per cell: kSweepInterior, kSweepBoundary, 0 (never swept)
+    // cell i's place in the level, -1 in an empty slot or a stopped problem's page
+    auto place = [&](int i) {
+        const int ci = i * nt + (int)threadIdx.x, p = W.wg_page[wg * W.slots + (ci >> 8)];
+        return p >= 0 && !page_stopped(L, p) ? p * kPageCells + (ci & 255) : -1;
+    };
 #pragma unroll
-        for (int q = 0; q < 6; ++q) {
-            slot[q] = inside[q] ? w : nb_slot[p * 6 + q];
-            if (slot[q] < 0) cst[q] = ld(u_in, (size_t)L.nbr[p * 6 + q] * 256 + nc[q]);
+    for (int i = 0; i < C; ++i) {
+        const int ci = i * nt + (int)threadIdx.x, e = place(i);
+        const uint16_t* q = W.nbr + (size_t)wg * 6 * cells + ci;
+#pragma unroll
+        for (int f = 0; f < 3; ++f) nb[i][f] = (unsigned)q[(size_t)(2 * f) * cells] | (unsigned)q[(size_t)(2 * f + 1) * cells] << 16;
+        cur[i] = bv[i] = wgt[i] = 0.f;
+        if (e >= 0) {
+            const uint32_t fl = L.flags[e], sel = fl & (kActive | kBoundary);
+            if (sel == kActive) kind |= (unsigned)kSweepInterior << (2 * i);
+            if (sel == (kActive | kBoundary)) kind |= (unsigned)kSweepBoundary << (2 * i);
+            wgt[i] = c_omega_fc[__popc(fl & (0x3fu * kFaceMX))];
+            bv[i] = ld(b, e);
+            if (!u_zero) cur[i] = ld(u, e);
         }
-        bv = ld(b, (size_t)p * 256 + c);
-        us[0][w][c] = u_in[(size_t)p * 256 + c];
+        st(us, ci, cur[i]);
+        st(us, W.entries + ci, cur[i]);
+    }
+    const int h0 = W.halo_ptr[wg], nh = W.halo_ptr[wg + 1] - h0;
+    for (int h = threadIdx.x; h < nh; h += nt) {
+        const float v = u_zero ? 0.f : ld(u, W.halo_cell[h0 + h]);
+        st(us, cells + h, v);
+        st(us, W.entries + cells + h, v);
     }
     __syncthreads();
-    int cur = 0;
-    for (int it = 0; it < count; ++it) {
-        if (live) {
-            const float cv = ld(us[cur][w], c);
-            float nv[6];
+    int from = 0;  // the copy that holds the current iterate: 0, or W.entries
+    auto residual = [&](int i, int at) {
+        float result = 0.f;
+        const S* v = us + at;
 #pragma unroll
-            for (int q = 0; q < 6; ++q) nv[q] = slot[q] >= 0 ? ld(us[cur][slot[q]], nc[q]) : cst[q];
-            float result = 0.f;
-#pragma unroll
-            for (int q = 0; q < 6; ++q)
-                if (f & (kFaceMX << q)) result -= (nv[q] - cv);
-            const float r = bv - result;
-            const uint32_t sel = f & (kActive | kBoundary);
-            float u = cv;
-            if (sel == kActive || sel == (kActive | kBoundary)) u += wgt * r;
-            st(us[1 - cur][w], c, u);
+        for (int f = 0; f < 3; ++f) {
+            result -= (ld(v, nb[i][f] & 0xffffu) - cur[i]);
+            result -= (ld(v, nb[i][f] >> 16) - cur[i]);
         }
-        __syncthreads();
-        cur = 1 - cur;
+        return bv[i] - result;
+    };
+    const bool any = __ballot(kind != 0) != 0;  // a wavefront without Active cells only keeps the barriers
+    for (int k = 0; k < ph.n; ++k) {
+        const unsigned sel = kind & ((unsigned)ph.cells[k] * 0x55555555u);
+        for (int it = 0; it < ph.count[k]; ++it) {
+            const int to = W.entries - from;
+            if (any) {
+#pragma unroll
+                for (int i = 0; i < C; ++i) {
+                    // many cells per thread: the neighbours stay packed (unpacked ahead of the loop they would spill)
+                    if (C > 4) asm volatile("" : "+v"(nb[i][0]), "+v"(nb[i][1]), "+v"(nb[i][2]));
+                    const float v = stored(us, cur[i] + wgt[i] * residual(i, from));
+                    cur[i] = (sel >> (2 * i)) & 3u ? v : cur[i];
+                    st(us, to + i * nt + (int)threadIdx.x, cur[i]);
+                }
+            }
+            __syncthreads();
+            from = to;
+        }
     }
-    if (live) u_out[(size_t)p * 256 + c] = us[cur][w][c];
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+        const int e = place(i);
+        if (e < 0) continue;
+        const bool act = ((kind >> (2 * i)) & 3u) != 0;
+        if (act) st(u, e, cur[i]);
+        if (r) st(r, e, act ? residual(i, from) : 0.f);
+    }
 }
 
 // residual at Active cells; other cells of r are written 0 (the value they
@@ -656,10 +693,25 @@ static void smooth_t(const DevLevel& L, const S* u_in, S* u_out, const S* b, boo
     if (L.np) hipLaunchKernelGGL(k_smooth<S>, dim3(kXcds * xcd_chunk(sweep_groups(L.np))), dim3(64 * kSweepPages), 0, s, L, u_in, u_out, b, (int)interior,
                                  (int)boundary);
 }
+template <class S, int C>
+static void cluster_sweeps_c(const DevLevel& L, const DevClusters& W, S* u, const S* b, S* r, const SweepPhases& ph, bool u_zero, hipStream_t s) {
+    const size_t lds = 2 * (size_t)W.entries * sizeof(S);
+    if (lds > 48 * 1024)
+        hdd_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cluster_sweeps<S, C>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+                  "cluster sweeps' LDS");
+    hipLaunchKernelGGL((k_cluster_sweeps<S, C>), dim3(W.nwg), dim3(W.slots * kPageCells / C), lds, s, L, W, u, b, r, ph, (int)u_zero);
+}
 template <class S>
-static void smooth_local_t(const DevLevel& L, const int* wg_page, int nwg, const int* nb_slot, const S* u_in, S* u_out, const S* b,
-                           int count, hipStream_t s) {
-    if (nwg) hipLaunchKernelGGL(k_smooth_local<S>, dim3(nwg), dim3(1024), 0, s, L, wg_page, nb_slot, u_in, u_out, b, count);
+static void cluster_sweeps_t(const DevLevel& L, const DevClusters& W, S* u, const S* b, S* r, const SweepPhases& ph, bool u_zero, hipStream_t s) {
+    if (!W.nwg) return;
+    // up to 1024 threads: one cell each up to four page slots, then C = slots / 4 cells each
+    switch (W.slots) {
+        case 1: case 2: case 4: cluster_sweeps_c<S, 1>(L, W, u, b, r, ph, u_zero, s); break;
+        case 8: cluster_sweeps_c<S, 2>(L, W, u, b, r, ph, u_zero, s); break;
+        case 16: cluster_sweeps_c<S, 4>(L, W, u, b, r, ph, u_zero, s); break;
+        case 32: cluster_sweeps_c<S, 8>(L, W, u, b, r, ph, u_zero, s); break;
+        default: throw std::runtime_error("cluster sweeps: slots must be a power of two up to 32");
+    }
 }
 template <class S>
 static void residual_t(const DevLevel& L, const S* u, const S* b, S* r, hipStream_t s) {
@@ -683,13 +735,13 @@ void launch_smooth(const DevLevel& L, const float* u_in, float* u_out, const flo
 void launch_smooth(const DevLevel& L, const __half* u_in, __half* u_out, const __half* b, bool interior, bool boundary, hipStream_t s) {
     smooth_t(L, u_in, u_out, b, interior, boundary, s);
 }
-void launch_smooth_local(const DevLevel& L, const int* wg_page, int nwg, const int* nb_slot, const float* u_in, float* u_out,
-                         const float* b, int count, hipStream_t s) {
-    smooth_local_t(L, wg_page, nwg, nb_slot, u_in, u_out, b, count, s);
+void launch_cluster_sweeps(const DevLevel& L, const DevClusters& C, float* u, const float* b, float* r, const SweepPhases& ph, bool u_zero,
+                           hipStream_t s) {
+    cluster_sweeps_t(L, C, u, b, r, ph, u_zero, s);
 }
-void launch_smooth_local(const DevLevel& L, const int* wg_page, int nwg, const int* nb_slot, const __half* u_in, __half* u_out,
-                         const __half* b, int count, hipStream_t s) {
-    smooth_local_t(L, wg_page, nwg, nb_slot, u_in, u_out, b, count, s);
+void launch_cluster_sweeps(const DevLevel& L, const DevClusters& C, __half* u, const __half* b, __half* r, const SweepPhases& ph,
+                           bool u_zero, hipStream_t s) {
+    cluster_sweeps_t(L, C, u, b, r, ph, u_zero, s);
 }
 void launch_residual(const DevLevel& L, const float* u, const float* b, float* r, hipStream_t s) { residual_t(L, u, b, r, s); }
 void launch_residual(const DevLevel& L, const __half* u, const __half* b, __half* r, hipStream_t s) { residual_t(L, u, b, r, s); }

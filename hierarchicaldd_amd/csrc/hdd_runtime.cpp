@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <map>
 #include <thread>
 #include <omp.h>
 
@@ -199,64 +200,139 @@ void Solver::merge_levels() {
     }
 }
 
-// Page-by-page sweeps of a level (the V-cycle bottom): pages are linked when
-// an Active cell has a set face bit to an Active cell of the other page;
-// linked pages form clusters. When no cluster has more than four pages, whole
-// clusters are packed into workgroups of four page slots (wg_page, -1 for an
-// empty slot) and nb_slot[p*6+f] gives the slot of page p's face-f neighbour
-// page when it is in p's cluster (else -1). Every other face neighbour then
-// holds no cell that a coupled Active cell reads and a sweep writes. Returns
-// false (sweeps stay global) when a cluster is larger.
-static bool plan_local_sweeps(const PagedLevel& H, std::vector<int>& wg_page, std::vector<int>& nb_slot) {
+DevClusters LevelBuffers::clusters() const {
+    DevClusters c;
+    c.slots = cl_slots; c.entries = cl_entries;
+    c.nwg = cl_slots ? (int)(cl_page.n / cl_slots) : 0;
+    c.wg_page = cl_page.p; c.nbr = cl_nbr.p; c.halo_ptr = cl_halo_ptr.p; c.halo_cell = cl_halo_cell.p;
+    return c;
+}
+
+// Clusters of a level's pages: pages are linked when an Active cell of one has a
+// set face bit to an Active cell of the other; a sweep of one cluster reads no
+// cell that a sweep of another writes. Whole clusters are packed into workgroups
+// of `slots` page slots (the largest cluster, rounded up to a power of two;
+// one cluster each while there are no more than kSpread, so that they run side
+// by side), each with the LDS value of every cell's face neighbours and the
+// list of cells outside the workgroup that its faces read. zero_outside: cells
+// that are not Active hold zero on this level (every level but 0), so that
+// list is one of them. False when a cluster is larger than kMaxSlots pages or
+// a workgroup's two copies exceed the LDS.
+static bool plan_clusters(LevelBuffers& LB, bool zero_outside) {
+    constexpr int kMaxSlots = 32, kSpread = 512, kLdsBytes = 150 * 1024;
     static const int d[6][3] = {{-1, 0, 0}, {1, 0, 0}, {0, -1, 0}, {0, 1, 0}, {0, 0, -1}, {0, 0, 1}};
+    const PagedLevel& H = LB.host;
     const int np = H.npages();
-    std::vector<int> parent(np);
-    for (int p = 0; p < np; ++p) parent[p] = p;
+    if (np == 0) return false;
+    std::vector<int> parent(np), size(np, 1), nbp((size_t)np * 6);
     auto find = [&](int a) {
         while (parent[a] != a) a = parent[a] = parent[parent[a]];
         return a;
     };
-    for (int p = 0; p < np; ++p) {
-        const Int3 o = H.page_base[p];
-        for (int c = 0; c < kPageCells; ++c) {
-            const uint32_t f = H.flags[(size_t)p * kPageCells + c];
-            if (!(f & kActive)) continue;
-            const int x = o.x + (c >> 6), y = o.y + ((c >> 3) & 7), z = o.z + (c & 7);
+    // cell c's neighbour across face q: its cell in the page, or in the face's neighbour page (outside = true)
+    auto step = [](int c, int q, bool& outside) {
+        const int x = c >> 6, y = (c >> 3) & 7, z = c & 7;
+        const int X = x + d[q][0], Y = y + d[q][1], Z = z + d[q][2];
+        outside = X < 0 || X >= kPX || Y < 0 || Y >= kPY || Z < 0 || Z >= kPZ;
+        return page_cell(X + kPX, Y + kPY, Z + kPZ);
+    };
+    for (int p = 0; p < np; ++p) parent[p] = p;
+    constexpr int kBlock = 4096;  // pages whose links are found in parallel before they are joined
+    std::vector<char> link((size_t)kBlock * 6);
+    for (int p0 = 0; p0 < np; p0 += kBlock) {
+        const int p1 = std::min(np, p0 + kBlock);
+#pragma omp parallel for schedule(static)
+        for (int p = p0; p < p1; ++p) {
+            const Int3 o = H.page_base[p];
+            const uint32_t* fl = &H.flags[(size_t)p * kPageCells];
             for (int q = 0; q < 6; ++q) {
-                if (!(f & (kFaceMX << q))) continue;
-                const int nx = x + d[q][0], ny = y + d[q][1], nz = z + d[q][2];
-                const int pn = H.page_at(nx, ny, nz);
-                if (pn == p || pn < 0 || !(H.flag(nx, ny, nz) & kActive)) continue;
-                parent[find(pn)] = find(p);
+                const int pn = H.page_at(o.x + d[q][0] * kPX, o.y + d[q][1] * kPY, o.z + d[q][2] * kPZ);
+                nbp[(size_t)p * 6 + q] = pn;
+                bool linked = false;
+                for (int c = 0; pn >= 0 && c < kPageCells && !linked; ++c) {
+                    bool out;
+                    if ((fl[c] & kActive) && (fl[c] & (kFaceMX << q))) {
+                        const int nc = step(c, q, out);
+                        linked = out && (H.flags[(size_t)pn * kPageCells + nc] & kActive);
+                    }
+                }
+                link[(size_t)(p - p0) * 6 + q] = linked;
             }
         }
+        for (int p = p0; p < p1; ++p)
+            for (int q = 0; q < 6; ++q) {
+                if (!link[(size_t)(p - p0) * 6 + q]) continue;
+                const int a = find(p), b = find(nbp[(size_t)p * 6 + q]);
+                if (a == b) continue;
+                parent[b] = a;
+                if ((size[a] += size[b]) > kMaxSlots) return false;
+            }
     }
     std::vector<std::vector<int>> members(np);
     for (int p = 0; p < np; ++p) members[find(p)].push_back(p);  // ascending pages per cluster
-    for (int r = 0; r < np; ++r)
-        if (members[r].size() > 4) return false;
-    wg_page.clear();
-    std::vector<int> slot(np, -1), wg_of(np, -1);
-    int used = 4;
+    size_t largest = 0, count = 0;
+    for (auto& m : members) { largest = std::max(largest, m.size()); count += !m.empty(); }
+    int slots = 1;
+    while (slots < (int)largest) slots *= 2;
+    std::vector<int> wg_page, slot(np, -1), wg_of(np, -1);
+    int used = slots;
     for (int p = 0; p < np; ++p) {
         const std::vector<int>& m = members[find(p)];
         if (m.front() != p) continue;  // clusters in the order of their first page (Morton order keeps them local)
-        if (used + (int)m.size() > 4) { wg_page.insert(wg_page.end(), 4, -1); used = 0; }
+        if (used + (int)m.size() > slots || count <= (size_t)kSpread) { wg_page.insert(wg_page.end(), slots, -1); used = 0; }
         for (int q : m) {
             slot[q] = used;
-            wg_of[q] = (int)wg_page.size() / 4 - 1;
-            wg_page[wg_page.size() - 4 + used] = q;
+            wg_of[q] = (int)wg_page.size() / slots - 1;
+            wg_page[wg_page.size() - slots + used] = q;
             ++used;
         }
     }
-    nb_slot.assign((size_t)np * 6, -1);
-    for (int p = 0; p < np; ++p) {
-        const Int3 o = H.page_base[p];
-        for (int q = 0; q < 6; ++q) {
-            const int pn = H.page_at(o.x + d[q][0] * kPX, o.y + d[q][1] * kPY, o.z + d[q][2] * kPZ);
-            if (pn >= 0 && find(pn) == find(p) && wg_of[pn] == wg_of[p]) nb_slot[(size_t)p * 6 + q] = slot[pn];
+    const int nwg = (int)wg_page.size() / slots, cells = slots * kPageCells;
+    std::vector<uint16_t> nbr((size_t)nwg * 6 * cells);
+    std::vector<std::vector<int>> halo(nwg);
+    std::vector<char> wide(nwg, 0);
+#pragma omp parallel for schedule(static)
+    for (int w = 0; w < nwg; ++w) {
+        std::map<int, int> seen;  // cell outside the workgroup -> its halo value
+        for (int s = 0; s < slots; ++s) {
+            const int p = wg_page[(size_t)w * slots + s];
+            for (int c = 0; c < kPageCells; ++c) {
+                const int ci = s * kPageCells + c;
+                const uint32_t f = p < 0 ? 0u : H.flags[(size_t)p * kPageCells + c];
+                for (int q = 0; q < 6; ++q) {
+                    int v = ci;
+                    if ((f & kActive) && (f & (kFaceMX << q))) {
+                        bool out;
+                        const int nc = step(c, q, out), pn = out ? nbp[(size_t)p * 6 + q] : p;
+                        if (pn >= 0 && wg_of[pn] == w) {
+                            v = slot[pn] * kPageCells + nc;
+                        } else {
+                            const int cell = zero_outside || pn < 0 ? np * kPageCells : pn * kPageCells + nc;
+                            const auto at = seen.emplace(cell, (int)seen.size());
+                            if (at.second) halo[w].push_back(cell);
+                            v = cells + at.first->second;
+                        }
+                    }
+                    wide[w] = wide[w] || v > 0xffff;
+                    nbr[((size_t)w * 6 + q) * cells + ci] = (uint16_t)v;
+                }
+            }
         }
     }
+    std::vector<int> halo_ptr(1, 0), halo_cell;
+    int most = 0;
+    for (int w = 0; w < nwg; ++w) {
+        if (wide[w]) return false;
+        most = std::max(most, (int)halo[w].size());
+        halo_cell.insert(halo_cell.end(), halo[w].begin(), halo[w].end());
+        halo_ptr.push_back((int)halo_cell.size());
+    }
+    if (2 * sizeof(float) * (size_t)(cells + most) > (size_t)kLdsBytes) return false;
+    LB.cl_slots = slots;
+    LB.cl_entries = (cells + most + 3) / 4 * 4;
+    halo_cell.push_back(np * kPageCells);  // never empty
+    LB.cl_page.upload(wg_page); LB.cl_nbr.upload(nbr);
+    LB.cl_halo_ptr.upload(halo_ptr); LB.cl_halo_cell.upload(halo_cell);
     return true;
 }
 
@@ -273,9 +349,12 @@ void Solver::build_device() {
     upload_levels();
     {
         const char* e = std::getenv("HDD_BOTTOM_LOCAL");
-        std::vector<int> wp, ns;
-        bottom_local = !(e && std::string(e) == "0") && plan_local_sweeps(lv.back().host, wp, ns);
-        if (bottom_local) { bottom_wg_page.upload(wp); bottom_nb_slot.upload(ns); }
+        if (!(e && std::string(e) == "0")) {
+            for (int l = 0; l < (int)lv.size(); ++l) {
+                const bool ok = plan_clusters(lv[l], l > 0);
+                if (l + 1 == (int)lv.size()) bottom_local = ok;
+            }
+        }
     }
     for (int l = 0; l < (int)lv.size(); ++l) {
         std::vector<int> pp((size_t)lv[l].host.npages() + 1, -1);
@@ -462,28 +541,42 @@ template <class S>
 void Solver::vcycle_t() {
     using V = VStore<S>;
     const int L = (int)lv.size();
-    for (int l = 0; l < L - 1; ++l) {
+    // a level's smoothing (boundary, interior, boundary sweeps) and, going down, its residual
+    auto smooth_level = [&](int l, bool u_zero, bool residual) {
+        LevelBuffers& B = lv[l];
+        if (B.cl_slots) {
+            SweepPhases ph;
+            ph.n = 3;
+            ph.count[0] = ph.count[2] = P.bnd_s; ph.count[1] = P.int_s;
+            ph.cells[0] = ph.cells[2] = kSweepBoundary; ph.cells[1] = kSweepInterior;
+            launch_cluster_sweeps(B.view(), B.clusters(), V::u(B, B.cur), V::b(B), residual ? V::r(B) : nullptr, ph, u_zero, stream);
+            return;
+        }
+        if (u_zero) launch_fill(V::u(B, B.cur), 0.f, B.cells(), stream);
         sweeps_t<S>(l, P.bnd_s, false, true);
         sweeps_t<S>(l, P.int_s, true, false);
         sweeps_t<S>(l, P.bnd_s, false, true);
-        launch_residual(lv[l].view(), V::u(lv[l], lv[l].cur), V::b(lv[l]), V::r(lv[l]), stream);
-        launch_fill(V::u(lv[l + 1], lv[l + 1].cur), 0.f, lv[l + 1].cells(), stream);
+        if (residual) launch_residual(B.view(), V::u(B, B.cur), V::b(B), V::r(B), stream);
+    };
+    for (int l = 0; l < L - 1; ++l) {
+        smooth_level(l, l > 0, true);
         launch_restrict(lv[l].view(), lv[l + 1].view(), V::r(lv[l]), V::b(lv[l + 1]), stream);
     }
-    if (bottom_local) {
-        // one launch; the result goes to the other buffer (other workgroups read this one's neighbour pages)
+    {
         LevelBuffers& B = lv[L - 1];
-        launch_smooth_local(B.view(), bottom_wg_page.p, (int)(bottom_wg_page.n / 4), bottom_nb_slot.p, V::u(B, B.cur), V::u(B, 1 - B.cur),
-                            V::b(B), 200, stream);
-        B.cur = 1 - B.cur;
-    } else {
-        sweeps_t<S>(L - 1, 200, true, true);
+        if (bottom_local) {
+            SweepPhases ph;
+            ph.n = 1;
+            ph.count[0] = 200; ph.cells[0] = kSweepInterior | kSweepBoundary;
+            launch_cluster_sweeps(B.view(), B.clusters(), V::u(B, B.cur), V::b(B), (decltype(V::r(B)))nullptr, ph, L > 1, stream);
+        } else {
+            if (L > 1) launch_fill(V::u(B, B.cur), 0.f, B.cells(), stream);
+            sweeps_t<S>(L - 1, 200, true, true);
+        }
     }
     for (int l = L - 2; l >= 0; --l) {
         launch_prolong(lv[l].view(), lv[l + 1].view(), V::u(lv[l], lv[l].cur), V::u(lv[l + 1], lv[l + 1].cur), stream);
-        sweeps_t<S>(l, P.bnd_s, false, true);
-        sweeps_t<S>(l, P.int_s, true, false);
-        sweeps_t<S>(l, P.bnd_s, false, true);
+        smooth_level(l, false, false);
     }
 }
 

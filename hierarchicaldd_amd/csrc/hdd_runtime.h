@@ -100,6 +100,11 @@ struct LevelBuffers {
     DBuf<float> u[2], b, r;
     DBuf<__half> hu[2], hb, hr;     // FP16-storage variant of u, b, r (allocated when it is selected)
     int cur = 0;  // which u buffer holds the current iterate
+    // clusters of pages that its sweeps couple (empty: one launch per sweep)
+    int cl_slots = 0, cl_entries = 0;
+    DBuf<int> cl_page, cl_halo_ptr, cl_halo_cell;
+    DBuf<uint16_t> cl_nbr;
+    DevClusters clusters() const;
     DevLevel view() const;
     size_t cells() const { return (size_t)(host.npages() + 1) * kPageCells; }
 };
@@ -174,11 +179,9 @@ public:
     bool use_graph = false;            // replay the preconditioner apply from captured HIP graphs (opt-in)
     bool half_storage = false;         // V-cycles store u, b, r in FP16 (FP32 arithmetic); z then lives in zf
     DBuf<float> zf;                    // preconditioner output of the FP16-storage variant
-    // the coarsest level's 200 sweeps run in one launch, a workgroup per four
-    // page slots of whole page clusters (its Active cells couple only within
-    // clusters of at most four pages; HDD_BOTTOM_LOCAL=0 turns it off)
+    // the coarsest level's 200 sweeps run in one launch (its clusters fit workgroups;
+    // HDD_BOTTOM_LOCAL=0 keeps one launch per sweep on every level)
     bool bottom_local = false;
-    DBuf<int> bottom_wg_page, bottom_nb_slot;
 
     // one problem; host_only: run the host setup and skip every device allocation (introspection)
     Solver(const SolverParams& p, int n_pages, const uint64_t* page_offsets, const uint32_t* flags, const float* b,
