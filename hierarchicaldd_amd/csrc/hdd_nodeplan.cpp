@@ -465,12 +465,18 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
     return true;
 }
 
+void node_block_rows(const NodePlanHost::Block& B, std::vector<int>& rows) {
+    local_rows(*B.f, B.sns, B.n, rows);
+    for (int& r : rows)
+        if (r >= B.n) r += T * B.nk - B.n;
+}
+
 void node_block_columns(const NodePlanHost::Block& B, double* L) {
     const SupernodalFactor& f = *B.f;
     const int np = T * B.nk, rows = np + T * B.nrk;
     std::fill(L, L + (size_t)rows * np, 0.0);
     std::vector<int> at;
-    local_rows(f, B.sns, B.n, at);
+    node_block_rows(B, at);
     for (int i = B.n; i < np; ++i) L[(size_t)i * np + i] = 1.0;
     int col = 0;
     size_t first = 0;
@@ -478,10 +484,7 @@ void node_block_columns(const NodePlanHost::Block& B, double* L) {
         const int n = f.sn[s].n, nr = (int)f.sn[s].rows.size();
         for (int j = 0; j < n; ++j) {
             for (int r = j; r < n; ++r) L[(size_t)(col + r) * np + col + j] = f.L11[s][(size_t)j * n + r];
-            for (int a = 0; a < nr; ++a) {
-                const int t = at[first + a];
-                L[(size_t)(t < B.n ? t : np + t - B.n) * np + col + j] = f.L21[s][(size_t)j * nr + a];
-            }
+            for (int a = 0; a < nr; ++a) L[(size_t)at[first + a] * np + col + j] = f.L21[s][(size_t)j * nr + a];
         }
         col += n;
         first += nr;

@@ -80,6 +80,10 @@ struct NodePlanHost {
 bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, const std::vector<int>& prob_of,
                     NodePlanHost& P);
 
+// Row of a block's padded columns (16 nk + 16 nrk of them: L11, then L21) that each sub-diagonal row of
+// its supernodes falls on, supernode after supernode.
+void node_block_rows(const NodePlanHost::Block& B, std::vector<int>& rows);
+
 // Factor columns of a block, row-major, (16 nk + 16 nrk) x 16 nk doubles: L11 (padding: identity), then L21.
 void node_block_columns(const NodePlanHost::Block& B, double* L);
 

@@ -16,7 +16,6 @@
 #include <algorithm>
 #include <stdexcept>
 #include "hdd_nodeplan_device.h"
-#include "hdd_parallel.h"
 
 namespace hdd {
 
@@ -261,43 +260,90 @@ struct SetupBlock {
     int nk, nrk, fwd, bwd, scale, pad;
 };
 
+// A supernode's factor columns on their way into its block: L11 (n x n) and L21 (nr x n), column-major
+struct SetupSupernode {
+    long long src, l;      // first double of L11 (L21 follows), first of the block's columns
+    int np, col, n, nr;    // row length of the block, first column of the supernode
+    int rows;              // first of its block rows in the row lists
+    int pad0, pad1;        // padding columns [pad0, pad1) of the block, set by its first supernode
+    int unused;
+};
+
+// One workgroup per supernode: its columns into the zeroed block, one on the padding's diagonal
+__global__ void __launch_bounds__(256) k_node_columns(const SetupSupernode* __restrict__ sn, const int* __restrict__ rows,
+                                                      const double* __restrict__ src, double* __restrict__ L) {
+    const SetupSupernode S = sn[blockIdx.x];
+    double* Lb = L + S.l;
+    const double* a = src + S.src;
+    const long long n11 = (long long)S.n * S.n, n21 = (long long)S.nr * S.n;
+    for (long long e = threadIdx.x; e < n11; e += 256) {
+        const int j = (int)(e / S.n), r = (int)(e - (long long)j * S.n);
+        if (r >= j) Lb[(long long)(S.col + r) * S.np + S.col + j] = a[e];
+    }
+    for (long long e = threadIdx.x; e < n21; e += 256) {
+        const int j = (int)(e / S.nr), r = (int)(e - (long long)j * S.nr);
+        Lb[(long long)rows[S.rows + r] * S.np + S.col + j] = a[n11 + e];
+    }
+    for (int i = S.pad0 + (int)threadIdx.x; i < S.pad1; i += 256) Lb[(long long)i * S.np + i] = 1.0;
+}
+
+// s += sign * sum over the tiles k in [k0, k1) of A(., k) B(k, .), element (r, c) of a 16x16 tile, with
+// A's tiles along a row at a + 16 k and B's down a column at b + 16 k * ld. Four tile pairs go through
+// LDS at a time and the next four load meanwhile: one at a time, the wait for each pair made the
+// inverse of a 2080-row block take 30 ms.
+constexpr int kPairs = 4;
+__device__ __forceinline__ double tile_products(double s, double sign, const double* __restrict__ a, const double* b, long long ld, int k0,
+                                                int k1, double (*as)[T][T + 1], double (*bs)[T][T + 1]) {
+    const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+    double an[kPairs], bn[kPairs];
+    auto fetch = [&](int k) {
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u) {
+            const bool in = k + u < k1;
+            an[u] = in ? a[r * ld + (long long)(k + u) * T + c] : 0.0;
+            bn[u] = in ? b[((long long)(k + u) * T + r) * ld + c] : 0.0;
+        }
+    };
+    if (k0 < k1) fetch(k0);
+    for (int k = k0; k < k1; k += kPairs) {
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u) { as[u][r][c] = sign * an[u]; bs[u][r][c] = bn[u]; }
+        __syncthreads();
+        if (k + kPairs < k1) fetch(k + kPairs);
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u)
+#pragma unroll
+            for (int q = 0; q < T; ++q) s = __builtin_fma(as[u][r][q], bs[u][q][c], s);
+        __syncthreads();
+    }
+    return s;
+}
+
 // X = L11^{-1}, one workgroup per 16-column strip: X_i = L_ii^{-1} (E_i - sum_{k < i} L_ik X_k) down the
 // row tiles; thread (r, c) owns one element of the tile
 __global__ void __launch_bounds__(256) k_node_inverse(const SetupBlock* __restrict__ blocks, const int2* __restrict__ strips,
-                                                      const double* __restrict__ L, double* __restrict__ X) {
-    __shared__ double ls[T][T + 1], xs[T][T + 1];
+                                                      const double* __restrict__ L, double* X) {
+    __shared__ double ls[kPairs][T][T + 1], xs[kPairs][T][T + 1];
     const int2 st = strips[blockIdx.x];
     const SetupBlock B = blocks[st.x];
     const int r = threadIdx.x >> 4, c = threadIdx.x & 15, ct = st.y;
     const long long np = (long long)B.nk * T;
     const double* Lb = L + B.l;
-    double* Xb = X + B.x;
-    for (int it = 0; it < ct; ++it) Xb[(it * T + r) * np + ct * T + c] = 0.0;
+    double* Xb = X + B.x + ct * T;  // the strip's columns
+    for (int it = 0; it < ct; ++it) Xb[(it * T + r) * np + c] = 0.0;
     for (int it = ct; it < B.nk; ++it) {
-        double s = it == ct && r == c ? 1.0 : 0.0;
-        double ln = 0.0, xn = 0.0;
-        if (ct < it) { ln = Lb[(it * T + r) * np + ct * T + c]; xn = Xb[(ct * T + r) * np + ct * T + c]; }
-        for (int kt = ct; kt < it; ++kt) {
-            ls[r][c] = ln; xs[r][c] = xn;
-            __syncthreads();
-            if (kt + 1 < it) {  // the next tiles load while this one is summed
-                ln = Lb[(it * T + r) * np + (kt + 1) * T + c];
-                xn = Xb[((kt + 1) * T + r) * np + ct * T + c];
-            }
-#pragma unroll
-            for (int k = 0; k < T; ++k) s -= ls[r][k] * xs[k][c];
-            __syncthreads();
-        }
-        ls[r][c] = Lb[(it * T + r) * np + it * T + c];
+        const double diag = Lb[(it * T + r) * np + it * T + c];
+        double s = tile_products(it == ct && r == c ? 1.0 : 0.0, -1.0, Lb + it * T * np, Xb, np, ct, it, ls, xs);
+        ls[0][r][c] = diag;
         __syncthreads();
         // forward substitution with the 16x16 diagonal tile, a row at a time
         for (int k = 0; k < T; ++k) {
-            if (r == k) { s /= ls[k][k]; xs[k][c] = s; }
+            if (r == k) { s /= ls[0][k][k]; xs[0][k][c] = s; }
             __syncthreads();
-            if (r > k) s -= ls[r][k] * xs[k][c];
+            if (r > k) s = __builtin_fma(-ls[0][r][k], xs[0][k][c], s);
         }
-        Xb[(it * T + r) * np + ct * T + c] = s;
-        __syncthreads();
+        Xb[(it * T + r) * np + c] = s;
+        __syncthreads();  // the next row tile reads it (and the LDS is reused)
     }
 }
 
@@ -305,7 +351,7 @@ __global__ void __launch_bounds__(256) k_node_inverse(const SetupBlock* __restri
 __global__ void __launch_bounds__(256) k_node_forward_tiles(const SetupBlock* __restrict__ blocks, const int2* __restrict__ rows,
                                                             const double* __restrict__ L, const double* __restrict__ X,
                                                             float* __restrict__ tiles, float* __restrict__ scale) {
-    __shared__ double ls[T][T + 1], xs[T][T + 1];
+    __shared__ double ls[kPairs][T][T + 1], xs[kPairs][T][T + 1];
     const int2 rw = rows[blockIdx.x];
     const SetupBlock B = blocks[rw.x];
     const int r = threadIdx.x >> 4, c = threadIdx.x & 15, rt = rw.y;
@@ -322,22 +368,8 @@ __global__ void __launch_bounds__(256) k_node_forward_tiles(const SetupBlock* __
         return;
     }
     const double* Lr = L + B.l + (long long)rt * T * np;
-    for (int j = 0; j < B.nk; ++j) {
-        double s = 0.0;
-        double ln = Lr[r * np + j * T + c], xn = Xb[(j * T + r) * np + j * T + c];
-        for (int kt = j; kt < B.nk; ++kt) {
-            ls[r][c] = ln; xs[r][c] = xn;
-            __syncthreads();
-            if (kt + 1 < B.nk) {
-                ln = Lr[r * np + (kt + 1) * T + c];
-                xn = Xb[((kt + 1) * T + r) * np + j * T + c];
-            }
-#pragma unroll
-            for (int k = 0; k < T; ++k) s += ls[r][k] * xs[k][c];
-            __syncthreads();
-        }
-        out[(size_t)j * 256] = (float)s;
-    }
+    for (int j = 0; j < B.nk; ++j)
+        out[(size_t)j * 256] = (float)tile_products(0.0, 1.0, Lr, Xb + j * T, np, j, B.nk, ls, xs);
 }
 
 // backward operator from the forward one: row tile rt holds the transposes of the forward tiles
@@ -369,12 +401,6 @@ void allow_lds(K kernel) {
               "dense-node kernels' LDS");
 }
 
-struct Pinned {
-    double* p = nullptr;
-    explicit Pinned(size_t n) { hdd_check(hipHostMalloc((void**)&p, n * sizeof(double), hipHostMallocDefault), "hipHostMalloc"); }
-    ~Pinned() { (void)hipHostFree(p); }
-};
-
 }  // namespace
 
 bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, const std::vector<int>& prob_of) {
@@ -398,13 +424,12 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
     pos_y.upload(P.pos_y); pos_c.upload(P.pos_c);
     tiles.alloc((size_t)P.tiles * 256); scale.alloc(P.scales);
     y.alloc(P.ysize); z.alloc((size_t)P.ysize + 1); c.alloc((size_t)P.csize + 1);
-    // the blocks in chunks: columns filled on the host, uploaded, inverted and packed
+    // the blocks in chunks: their supernodes' columns uploaded and put in place, inverted and packed
     constexpr size_t kChunk = size_t(24) << 20;  // doubles per chunk, unless one block needs more
     auto doubles = [](const NodePlanHost::Block& B) { return (size_t)(B.nk + B.nrk) * T * B.nk * T; };
     size_t largest = 0, total = 0;
     for (const auto& B : P.blocks) { largest = std::max(largest, doubles(B)); total += doubles(B); }
     const size_t cap = std::min(total, std::max(largest, kChunk));
-    Pinned host(cap);
     DBuf<double> dL, dX;
     hdd_check(hipMalloc(&dL.p, cap * sizeof(double)), "hipMalloc"); dL.n = cap;
     size_t xcap = 0;
@@ -434,15 +459,39 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
             for (int r = 0; r < B.nk; ++r) { strips.push_back(make_int2(id, r)); brows.push_back(make_int2(id, r)); }
             for (int r = 0; r < B.nk + B.nrk; ++r) rows.push_back(make_int2(id, r));
         }
-        ParallelErrors errs;
-#pragma omp parallel for schedule(dynamic)
-        for (size_t k = ch.first; k < ch.second; ++k)
-            errs.run([&] { node_block_columns(P.blocks[k], host.p + sb[k - ch.first].l); });
-        errs.rethrow();
+        std::vector<SetupSupernode> ss;
+        std::vector<std::pair<const SupernodalFactor*, int>> from;
+        std::vector<int> list, at;
+        long long packed = 0;
+        for (size_t k = ch.first; k < ch.second; ++k) {
+            const NodePlanHost::Block& B = P.blocks[k];
+            node_block_rows(B, at);
+            int col = 0, first = (int)list.size();
+            list.insert(list.end(), at.begin(), at.end());
+            for (int g : B.sns) {
+                const int n = B.f->sn[g].n, nr = (int)B.f->sn[g].rows.size(), np = B.nk * T;
+                ss.push_back({packed, sb[k - ch.first].l, np, col, n, nr, first, col ? np : B.n, np, 0});
+                from.push_back({B.f, g});
+                packed += (long long)n * n + (long long)nr * n;
+                col += n;
+                first += nr;
+            }
+        }
+        std::vector<double> host(packed);
+#pragma omp parallel for schedule(dynamic, 16)
+        for (size_t k = 0; k < ss.size(); ++k) {
+            const std::vector<double>&a = from[k].first->L11[from[k].second], &b = from[k].first->L21[from[k].second];
+            std::copy(a.begin(), a.end(), host.begin() + ss[k].src);
+            std::copy(b.begin(), b.end(), host.begin() + ss[k].src + (long long)a.size());
+        }
         DBuf<SetupBlock> dsb; dsb.upload(sb);
         DBuf<int2> dst, drw, dbr;
         dst.upload(strips); drw.upload(rows); dbr.upload(brows);
-        hdd_check(hipMemcpy(dL.p, host.p, (size_t)l * sizeof(double), hipMemcpyHostToDevice), "node blocks upload");
+        DBuf<SetupSupernode> dss; dss.upload(ss);
+        DBuf<int> dlist; dlist.upload(list.empty() ? std::vector<int>(1, 0) : list);
+        DBuf<double> dsrc; dsrc.upload(host);
+        hdd_check(hipMemset(dL.p, 0, (size_t)l * sizeof(double)), "node blocks");
+        launch(k_node_columns, (int)ss.size(), 4, 0, nullptr, (const SetupSupernode*)dss.p, (const int*)dlist.p, (const double*)dsrc.p, dL.p);
         launch(k_node_inverse, (int)strips.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)dst.p, (const double*)dL.p, dX.p);
         launch(k_node_forward_tiles, (int)rows.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)drw.p, (const double*)dL.p,
                (const double*)dX.p, tiles.p, scale.p);
