@@ -295,8 +295,7 @@ hdd_status hdd_set_channel(hdd_ctx* ctx, int ch, const float* host) {
     HDD_TRY(ctx, {
         Solver& S = *ctx->solver;
         const size_t n = (size_t)S.lv[0].host.npages() * kPageCells;
-        hdd_check(hipMemcpyAsync(S.channel(ch), host, n * sizeof(float), hipMemcpyHostToDevice, S.stream), "set_channel");
-        hdd_check(hipStreamSynchronize(S.stream), "set_channel");
+        S.stage.to_device(S.channel(ch), host, n * sizeof(float), S.stream);
     })
 }
 
@@ -307,8 +306,7 @@ hdd_status hdd_get_channel(hdd_ctx* ctx, int ch, float* host) {
         Solver& S = *ctx->solver;
         hdd_check(hipStreamSynchronize(S.stream), "sync");
         const size_t n = (size_t)S.lv[0].host.npages() * kPageCells;
-        hdd_check(hipMemcpyAsync(host, S.channel(ch), n * sizeof(float), hipMemcpyDeviceToHost, S.stream), "get_channel");
-        hdd_check(hipStreamSynchronize(S.stream), "get_channel");
+        S.stage.to_host(host, S.channel(ch), n * sizeof(float), S.stream);
     })
 }
 

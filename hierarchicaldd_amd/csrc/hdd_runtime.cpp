@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <thread>
 #include <omp.h>
@@ -18,6 +19,64 @@ static void host_phase(const char* what, std::chrono::steady_clock::time_point& 
     const auto now = std::chrono::steady_clock::now();
     if (verbose) std::fprintf(stderr, "[setup] %s: %.3fs\n", what, std::chrono::duration<double>(now - t).count());
     t = now;
+}
+
+HostStage::~HostStage() {
+    for (hipEvent_t e : done) if (e) (void)hipEventDestroy(e);
+}
+
+void HostStage::init(size_t largest_bytes) {
+    if (largest_bytes < kMin || ring.p) return;
+    ring.alloc(kChunk * kRing);
+    for (hipEvent_t& e : done) hdd_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+}
+
+// memcpy of one chunk over the host's threads, in pieces of whole pages
+static void copy_parallel(char* to, const char* from, size_t bytes) {
+    constexpr size_t kPiece = size_t(256) << 10;
+    const int pieces = (int)((bytes + kPiece - 1) / kPiece);
+#pragma omp parallel for schedule(static)
+    for (int k = 0; k < pieces; ++k) std::memcpy(to + k * kPiece, from + k * kPiece, std::min(kPiece, bytes - k * kPiece));
+}
+
+void HostStage::to_host(void* host, const void* dev, size_t bytes, hipStream_t s) {
+    if (bytes < kMin || !ring.p) {
+        hdd_check(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s), "copy to the host");
+        hdd_check(hipStreamSynchronize(s), "copy to the host");
+        return;
+    }
+    const size_t chunks = (bytes + kChunk - 1) / kChunk;
+    auto queue = [&](size_t k) {
+        const size_t at = k * kChunk;
+        hdd_check(hipMemcpyAsync(ring.p + (k % kRing) * kChunk, static_cast<const char*>(dev) + at, std::min(kChunk, bytes - at),
+                                 hipMemcpyDeviceToHost, s), "copy to the host");
+        hdd_check(hipEventRecord(done[k % kRing], s), "copy to the host");
+    };
+    for (size_t k = 0; k < chunks && k < (size_t)kRing; ++k) queue(k);
+    for (size_t k = 0; k < chunks; ++k) {
+        const size_t at = k * kChunk;
+        hdd_check(hipEventSynchronize(done[k % kRing]), "copy to the host");
+        copy_parallel(static_cast<char*>(host) + at, ring.p + (k % kRing) * kChunk, std::min(kChunk, bytes - at));
+        if (k + kRing < chunks) queue(k + kRing);
+    }
+}
+
+void HostStage::to_device(void* dev, const void* host, size_t bytes, hipStream_t s) {
+    if (bytes < kMin || !ring.p) {
+        hdd_check(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s), "copy to the device");
+        hdd_check(hipStreamSynchronize(s), "copy to the device");
+        return;
+    }
+    const size_t chunks = (bytes + kChunk - 1) / kChunk;
+    for (size_t k = 0; k < chunks; ++k) {
+        const size_t at = k * kChunk, len = std::min(kChunk, bytes - at);
+        char* slot = ring.p + (k % kRing) * kChunk;
+        if (k >= (size_t)kRing) hdd_check(hipEventSynchronize(done[k % kRing]), "copy to the device");
+        copy_parallel(slot, static_cast<const char*>(host) + at, len);
+        hdd_check(hipMemcpyAsync(static_cast<char*>(dev) + at, slot, len, hipMemcpyHostToDevice, s), "copy to the device");
+        hdd_check(hipEventRecord(done[k % kRing], s), "copy to the device");
+    }
+    hdd_check(hipStreamSynchronize(s), "copy to the device");
 }
 
 DevLevel LevelBuffers::view() const {
@@ -371,6 +430,7 @@ void Solver::build_device() {
     }
     const size_t n0 = lv[0].cells();
     x.alloc(n0); q.alloc(n0); s.alloc(n0);
+    stage.init(n0 * sizeof(float));
     // per-problem reductions: each problem's partials as for a one-problem grid of its own size
     {
         std::vector<int> parts(NP), pp((size_t)np0 + 1, -1);
@@ -964,8 +1024,7 @@ void Solver::download_x(int p, float* host) {
     if (p < 0 || p >= nprob()) throw std::runtime_error("no such problem in the batch");
     hdd_check(hipStreamSynchronize(stream), "sync");
     const size_t first = (size_t)pg0[0][p] * kPageCells, n = (size_t)(pg0[0][p + 1] - pg0[0][p]) * kPageCells;
-    hdd_check(hipMemcpyAsync(host, x.p + first, n * sizeof(float), hipMemcpyDeviceToHost, stream), "download x");
-    hdd_check(hipStreamSynchronize(stream), "download x");
+    stage.to_host(host, x.p + first, n * sizeof(float), stream);
 }
 
 }  // namespace hdd
