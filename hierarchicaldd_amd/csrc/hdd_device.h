@@ -84,6 +84,7 @@ struct DevSegments {
     const int* active = nullptr;      // [nprob] 1 while the problem iterates
     double* dpart = nullptr;          // [nprob*max_parts]
     float* fpart = nullptr;           // [nprob*max_parts]
+    unsigned* ticket = nullptr;       // [nprob] zero between reductions
     float* scal = nullptr;            // [nprob*8]
     double* dscal = nullptr;          // [nprob*8]
     bool serial_dots = false;         // inner products in the reference's serial order (k_seg_dot_serial)

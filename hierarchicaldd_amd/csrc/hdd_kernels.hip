@@ -18,6 +18,8 @@
 //   PCG Laplace (double accumulation)       DDS/SPGrid_Gemini_Arithmetic_Helpers.h:240-262
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
+#include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include "hdd_device.h"
@@ -495,30 +497,134 @@ __global__ void k_cast_to_float(const double* __restrict__ x, float* __restrict_
     for (; i < n; i += (size_t)gridDim.x * blockDim.x) y[i] = (float)x[i];
 }
 
-// block-partial double dot products of float products (a*b rounded to float, then summed in double);
-// block (c, p) = partial c of problem p
-__global__ void __launch_bounds__(256) k_seg_dot_partial(const float* __restrict__ a, const float* __restrict__ b, double* __restrict__ part,
-                                                         const int* __restrict__ pg0, const int* __restrict__ parts, int max_parts) {
-    const int p = blockIdx.y, c = blockIdx.x, g = parts[p];
-    if (c >= g) return;
-    const size_t base = (size_t)pg0[p] * 256, n = (size_t)(pg0[p + 1] - pg0[p]) * 256;
-    __shared__ double sh[4];
-    double s = 0.0;
-    for (size_t i = (size_t)c * 256 + threadIdx.x; i < n; i += (size_t)g * 256) s += (double)(a[base + i] * b[base + i]);
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) part[(size_t)p * max_parts + c] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+constexpr int kDotThreads = 1024;
+// Sum of a thread's share of float products (a*b rounded to float, then summed in double): every
+// g*kDotThreads-th group of four cells from group c*kDotThreads + thread on, four groups in flight, one sum per place
+// in a group: 127 MB at 256^3 at 6.1 TB/s (21 us, with the second launch it saves 24.6), one cell at a time
+// and in two launches 32 us and 4.
+template <bool kWide>
+__device__ __forceinline__ double dot_share(const float* __restrict__ a, const float* __restrict__ b, size_t groups, int c, int g) {
+    auto four = [](const float* __restrict__ p, size_t i) {
+        if (kWide) return reinterpret_cast<const float4*>(p)[i];
+        return make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
+    };
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    auto add = [&](const float4& u, const float4& v) {
+        s0 += (double)(u.x * v.x); s1 += (double)(u.y * v.y); s2 += (double)(u.z * v.z); s3 += (double)(u.w * v.w);
+    };
+    const size_t step = (size_t)g * kDotThreads;
+    size_t i = (size_t)c * kDotThreads + threadIdx.x;
+    for (; i + 3 * step < groups; i += 4 * step) {
+        const float4 u0 = four(a, i), u1 = four(a, i + step), u2 = four(a, i + 2 * step), u3 = four(a, i + 3 * step);
+        const float4 v0 = four(b, i), v1 = four(b, i + step), v2 = four(b, i + 2 * step), v3 = four(b, i + 3 * step);
+        add(u0, v0); add(u1, v1); add(u2, v2); add(u3, v3);
+    }
+    for (; i < groups; i += step) add(four(a, i), four(b, i));
+    return (s0 + s1) + (s2 + s3);
 }
+
+// total of one value per thread of a workgroup (the same in every thread)
+template <class V, class Add>
+__device__ __forceinline__ V block_total(V v, Add add) {
+    constexpr int NW = kDotThreads / 64;
+    __shared__ V sh[NW];
+    for (int o = 32; o > 0; o >>= 1) v = add(v, __shfl_down(v, o, 64));
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    V t = sh[0];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) t = add(t, sh[k]);
+    return t;
+}
+__device__ __forceinline__ double block_sum(double s) {
+    return block_total(s, [](double x, double y) { return x + y; });
+}
+__device__ __forceinline__ float block_max(float m) {
+    return block_total(m, [](float x, float y) { return fmaxf(x, y); });
+}
+
+// Reductions end in their own launch: every block leaves its partial, and the block that draws the last
+// ticket adds them, in the order a second launch would (which cost 3-4 us more for each of the three
+// reductions of an iteration). The ticket is zero between launches. Partials are exchanged and loaded past
+// the caches, and a block draws its ticket when its exchange has returned, so no cache is written back or
+// invalidated: with a release and acquire of the device's scope instead, 1024 blocks took 45 us longer.
+template <class V>
+__device__ __forceinline__ void leave_partial(V* p, V v) {
+    const V old = __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::"v"(old) : "memory");  // the exchange is complete
+}
+__device__ __forceinline__ bool last_block(unsigned* ticket, int g) {
+    __shared__ bool last;
+    if (threadIdx.x == 0) {
+        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)g - 1u;
+        if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    return last;
+}
+template <class V>
+__device__ __forceinline__ V partial(const V* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Scalar logic of CONJUGATE_GRADIENT_DUMPING::Solve (:193-205) in float, on a problem's inner product:
+//   mode 0: rho = (float)dot -> scal[0]; beta = rho/rho_old -> scal[2]
+//   mode 1: s_dot_q = (float)dot; alpha = rho/s_dot_q -> scal[1]; rho_old = rho -> scal[3]
+//   mode 3: the plain sum -> dscal[2], no PCG scalar touched
+//   modes 5 / 6: as 0 / 1 with the scalars in double (dscal: 0 rho, 1 s_dot_q,
+//   3 alpha, 4 beta, 5 rho_old)
+// Mode 3 is for every problem, the others for those that iterate.
+__device__ __forceinline__ bool dot_skipped(int mode, const int* __restrict__ active, int p) { return mode != 3 && !active[p]; }
+__device__ __forceinline__ void dot_scalars(int mode, double s, float* __restrict__ scal, double* __restrict__ dscal) {
+    if (mode == 0) {
+        const float rho = (float)s;
+        scal[0] = rho;
+        scal[2] = rho / scal[3];
+        dscal[0] = s;
+    } else if (mode == 3) {
+        dscal[2] = s;
+    } else if (mode == 5) {
+        dscal[0] = s;
+        dscal[4] = s / dscal[5];
+    } else if (mode == 6) {
+        dscal[1] = s;
+        dscal[3] = s != 0.0 ? dscal[0] / s : 3.40282347e+38;
+        dscal[5] = dscal[0];
+    } else {
+        const float sdq = (float)s;
+        const float rho = scal[0];
+        scal[1] = sdq != 0.f ? rho / sdq : 3.40282347e+38f;
+        scal[3] = rho;
+        dscal[1] = s;
+    }
+}
+
+// block (c, p) = partial dot product c of problem p
+__global__ void __launch_bounds__(kDotThreads) k_seg_dot(const float* __restrict__ a, const float* __restrict__ b, double* part,
+                                                 unsigned* ticket, const int* __restrict__ pg0, const int* __restrict__ parts,
+                                                 int max_parts, int mode, const int* __restrict__ active, float* __restrict__ scal,
+                                                 double* __restrict__ dscal) {
+    const int p = blockIdx.y, c = blockIdx.x, g = parts[p];
+    if (c >= g || dot_skipped(mode, active, p)) return;
+    const size_t base = (size_t)pg0[p] * 256, groups = (size_t)(pg0[p + 1] - pg0[p]) * 64;
+    double s = block_sum(dot_share<true>(a + base, b + base, groups, c, g));
+    double* pp = part + (size_t)p * max_parts;
+    if (threadIdx.x == 0) leave_partial(pp + c, s);
+    if (!last_block(ticket + p, g)) return;
+    s = 0.0;
+    for (int i = threadIdx.x; i < g; i += kDotThreads) s += partial(pp + i);
+    s = block_sum(s);
+    if (threadIdx.x == 0) dot_scalars(mode, s, scal + p * 8, dscal + p * 8);
+}
+
 // The reference's order of CG_SYSTEM::Inner_Product (DDS/CG_SYSTEM.cpp:62-72): one
 // running double sum over the problem's pages in page order and their cells in
 // cell order, each term the float product. One workgroup per problem stages 1024
-// products at a time in LDS and one lane adds them in sequence; the sum goes to
-// the problem's first partial and its other partials are zero, so k_seg_finish
-// gives it unchanged. For checking against the reference's rounding, not speed.
-__global__ void __launch_bounds__(256) k_seg_dot_serial(const float* __restrict__ a, const float* __restrict__ b, double* __restrict__ part,
-                                                        const int* __restrict__ pg0, const int* __restrict__ parts, int max_parts) {
+// products at a time in LDS and one lane adds them in sequence. For checking
+// against the reference's rounding, not speed.
+__global__ void __launch_bounds__(256) k_seg_dot_serial(const float* __restrict__ a, const float* __restrict__ b, const int* __restrict__ pg0,
+                                                        int mode, const int* __restrict__ active, float* __restrict__ scal,
+                                                        double* __restrict__ dscal) {
     const int p = blockIdx.x;
+    if (dot_skipped(mode, active, p)) return;
     const size_t base = (size_t)pg0[p] * 256, n = (size_t)(pg0[p + 1] - pg0[p]) * 256;
     __shared__ double buf[1024];
     double s = 0.0;
@@ -530,80 +636,33 @@ __global__ void __launch_bounds__(256) k_seg_dot_serial(const float* __restrict_
             for (size_t t = 0; t < cnt; ++t) s += buf[t];
         __syncthreads();
     }
-    for (int c = threadIdx.x; c < parts[p]; c += 256) part[(size_t)p * max_parts + c] = c == 0 ? s : 0.0;
+    if (threadIdx.x == 0) dot_scalars(mode, s, scal + p * 8, dscal + p * 8);
 }
 
-__global__ void __launch_bounds__(256) k_seg_maxabs_partial(const float* __restrict__ a, float* __restrict__ part,
-                                                            const int* __restrict__ pg0, const int* __restrict__ parts, int max_parts) {
+// max |a| of every problem -> scal[4]
+__global__ void __launch_bounds__(kDotThreads) k_seg_maxabs(const float* __restrict__ a, float* part, unsigned* ticket,
+                                                    const int* __restrict__ pg0, const int* __restrict__ parts, int max_parts,
+                                                    float* __restrict__ scal) {
     const int p = blockIdx.y, c = blockIdx.x, g = parts[p];
     if (c >= g) return;
-    const size_t base = (size_t)pg0[p] * 256, n = (size_t)(pg0[p + 1] - pg0[p]) * 256;
-    __shared__ float sh[4];
+    const size_t groups = (size_t)(pg0[p + 1] - pg0[p]) * 64;
+    const float4* a4 = reinterpret_cast<const float4*>(a + (size_t)pg0[p] * 256);
     float m = 0.f;
-    for (size_t i = (size_t)c * 256 + threadIdx.x; i < n; i += (size_t)g * 256) m = fmaxf(m, fabsf(a[base + i]));
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_down(m, o, 64));
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) part[(size_t)p * max_parts + c] = fmaxf(fmaxf(sh[0], sh[1]), fmaxf(sh[2], sh[3]));
+#pragma unroll 4
+    for (size_t i = (size_t)c * kDotThreads + threadIdx.x; i < groups; i += (size_t)g * kDotThreads) {
+        const float4 v = a4[i];
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    }
+    m = block_max(m);
+    float* pp = part + (size_t)p * max_parts;
+    if (threadIdx.x == 0) leave_partial(pp + c, m);
+    if (!last_block(ticket + p, g)) return;
+    m = 0.f;
+    for (int i = threadIdx.x; i < g; i += kDotThreads) m = fmaxf(m, partial(pp + i));
+    m = block_max(m);
+    if (threadIdx.x == 0) scal[p * 8 + 4] = m;
 }
 
-// Final reduction of one problem's partials (workgroup p) and the PCG scalar
-// logic of CONJUGATE_GRADIENT_DUMPING::Solve (:193-205) in float:
-//   mode 0: rho = (float)dot -> scal[0]; beta = rho/rho_old -> scal[2]
-//   mode 1: s_dot_q = (float)dot; alpha = rho/s_dot_q -> scal[1]; rho_old = rho -> scal[3]
-//   mode 2: max-abs norm -> scal[4] (every problem; modes 0 and 1 active problems only)
-//   mode 3: the plain sum -> dscal[2] (every problem)
-//   modes 5 / 6: as 0 / 1 with the scalars in double (dscal: 0 rho, 1 s_dot_q,
-//   3 alpha, 4 beta, 5 rho_old), active problems only
-__global__ void __launch_bounds__(256) k_seg_finish(const double* __restrict__ dpart, const float* __restrict__ fpart,
-                                                    const int* __restrict__ parts, int max_parts, int mode, const int* __restrict__ active,
-                                                    float* __restrict__ scal_all, double* __restrict__ dscal_all) {
-    const int p = blockIdx.x;
-    if ((mode == 0 || mode == 1 || mode == 5 || mode == 6) && !active[p]) return;
-    const int nparts = parts[p];
-    float* scal = scal_all + p * 8;
-    double* dscal = dscal_all + p * 8;
-    __shared__ double sd[256];
-    __shared__ float sf[256];
-    double s = 0.0;
-    float m = 0.f;
-    for (int i = threadIdx.x; i < nparts; i += 256) {
-        if (mode != 2) s += dpart[(size_t)p * max_parts + i]; else m = fmaxf(m, fpart[(size_t)p * max_parts + i]);
-    }
-    sd[threadIdx.x] = s; sf[threadIdx.x] = m;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) { sd[threadIdx.x] += sd[threadIdx.x + o]; sf[threadIdx.x] = fmaxf(sf[threadIdx.x], sf[threadIdx.x + o]); }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        if (mode == 0) {
-            const float rho = (float)sd[0];
-            scal[0] = rho;
-            scal[2] = rho / scal[3];
-            dscal[0] = sd[0];
-        } else if (mode == 3) {
-            dscal[2] = sd[0];  // a plain inner product (Inner_Product), no PCG scalar touched
-        } else if (mode == 5) {
-            // FP64 outer scalars: rho and beta = rho / rho_old in double
-            dscal[0] = sd[0];
-            dscal[4] = sd[0] / dscal[5];
-        } else if (mode == 6) {
-            // FP64 outer scalars: alpha = rho / s_dot_q, rho_old = rho
-            dscal[1] = sd[0];
-            dscal[3] = sd[0] != 0.0 ? dscal[0] / sd[0] : 3.40282347e+38;
-            dscal[5] = dscal[0];
-        } else if (mode == 1) {
-            const float sdq = (float)sd[0];
-            const float rho = scal[0];
-            scal[1] = sdq != 0.f ? rho / sdq : 3.40282347e+38f;
-            scal[3] = rho;
-            dscal[1] = sd[0];
-        } else {
-            scal[4] = sf[0];
-        }
-    }
-}
 // FP16 storage: the preconditioner is linear, so it runs on r / a and its
 // result is scaled back by a, with a = max|r| of the cell's problem (slot 4 of
 // its scalars; 1 where r = 0). Values then stay O(1), inside half's normal range.
@@ -628,38 +687,33 @@ __global__ void __launch_bounds__(256) k_unscale_project(DevLevel L, const __hal
 
 // ---------------------------------------------------------------------------
 // Inner product that allocates nothing (hdd_inner_product_noalloc): the block
-// partials of k_seg_dot_partial for one problem of n_pages pages go to the
-// file-scope array `scratch` (one copy per device, held until the process
-// ends), and the final sum of k_seg_finish (mode 3) to the caller's device
-// double. The blocks stride over the cells, and both reductions add, exactly
-// as those kernels do for a one-problem context, so the value has the bits of
-// hdd_inner_product on a context holding the same pages.
-constexpr int kNoAllocParts = 1024;  // reduce_parts never exceeds it
-static __device__ __align__(256) double scratch[kNoAllocParts];
+// partials of k_seg_dot for one problem of n_pages pages go to the file-scope
+// array `scratch` (one copy per device, held until the process ends), and their
+// sum to the caller's device double. The blocks stride over the cells, and both
+// reductions add, exactly as k_seg_dot does for a one-problem context, so the
+// value has the bits of hdd_inner_product on a context holding the same pages.
+// Calls take the tickets in turn and clear the one half a round away: calls that
+// overlapped (they may not) spoil no later call's ticket for more than a round.
+constexpr int kNoAllocParts = 1024, kNoAllocTickets = 64;  // reduce_parts never exceeds the first
+struct NoAllocScratch {
+    double part[kNoAllocParts];
+    unsigned ticket[kNoAllocTickets];
+};
+static __device__ __align__(256) NoAllocScratch scratch;
 
-__global__ void __launch_bounds__(256) k_dot_partial_flat(const float* __restrict__ a, const float* __restrict__ b, size_t n, int g,
-                                                          double* __restrict__ part) {
-    const int c = blockIdx.x;
-    __shared__ double sh[4];
-    double s = 0.0;
-    for (size_t i = (size_t)c * 256 + threadIdx.x; i < n; i += (size_t)g * 256) s += (double)(a[i] * b[i]);
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) part[c] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-}
-
-__global__ void __launch_bounds__(256) k_dot_finish_flat(const double* __restrict__ part, int nparts, double* __restrict__ out) {
-    __shared__ double sd[256];
-    double s = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += 256) s += part[i];
-    sd[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) sd[threadIdx.x] += sd[threadIdx.x + o];
-        __syncthreads();
+template <bool kWide>
+__global__ void __launch_bounds__(kDotThreads) k_dot_flat(const float* __restrict__ a, const float* __restrict__ b, size_t groups, int g,
+                                                  NoAllocScratch* w, int ticket, double* __restrict__ out) {
+    double s = block_sum(dot_share<kWide>(a, b, groups, blockIdx.x, g));
+    if (threadIdx.x == 0) {
+        leave_partial(w->part + blockIdx.x, s);
+        if (blockIdx.x == 0) __hip_atomic_store(w->ticket + (ticket + kNoAllocTickets / 2) % kNoAllocTickets, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (threadIdx.x == 0) *out = sd[0];
+    if (!last_block(w->ticket + ticket, g)) return;
+    s = 0.0;
+    for (int i = threadIdx.x; i < g; i += kDotThreads) s += partial(w->part + i);
+    s = block_sum(s);
+    if (threadIdx.x == 0) *out = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -775,16 +829,18 @@ void launch_project(const DevLevel& L, float* v, hipStream_t s) {
 void launch_sub_project(const DevLevel& L, const float* b, const float* q, float* r, hipStream_t s) {
     if (L.np) hipLaunchKernelGGL(k_sub_project, dim3(L.np), dim3(256), 0, s, L, b, q, r);
 }
-int reduce_parts(size_t n) { return grid_for(n) > 1024 ? 1024 : grid_for(n); }
+// Blocks of a reduction over n cells: four cells per thread, and one block per CU at most (the blocks draw
+// their tickets one after the other, about 12 ns each)
+int reduce_parts(size_t n) { return (int)std::max<size_t>(1, std::min<size_t>(256, (n + 4 * kDotThreads - 1) / (4 * kDotThreads))); }
 
 // Device address of `scratch` on the current device: hipGetSymbolAddress once
 // per device, with that device current, kept for later calls (each device
 // holds its own copy of the array at its own address; the array's name in
 // host code is not a device address).
-static double* noalloc_scratch() {
+static NoAllocScratch* noalloc_scratch() {
     constexpr int kMaxDevices = 64;
     static std::mutex mu;
-    static double* ptr[kMaxDevices] = {};
+    static NoAllocScratch* ptr[kMaxDevices] = {};
     int dev = 0;
     hdd_check(hipGetDevice(&dev), "hipGetDevice");
     if (dev < 0 || dev >= kMaxDevices) throw std::runtime_error("inner product (no allocation): device index out of range");
@@ -792,7 +848,7 @@ static double* noalloc_scratch() {
     if (!ptr[dev]) {
         void* p = nullptr;
         hdd_check(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)");
-        ptr[dev] = static_cast<double*>(p);
+        ptr[dev] = static_cast<NoAllocScratch*>(p);
     }
     return ptr[dev];
 }
@@ -801,9 +857,11 @@ void launch_inner_product_noalloc(const float* a, const float* b, int64_t n_page
     const size_t n = (size_t)n_pages * kPageCells;
     const int g = reduce_parts((size_t)(n_pages + 1) * kPageCells);  // the partition of a context of n_pages pages
     if (g > kNoAllocParts) throw std::runtime_error("inner product (no allocation): more partial sums than the scratch holds");
-    double* part = noalloc_scratch();
-    hipLaunchKernelGGL(k_dot_partial_flat, dim3(g), dim3(256), 0, s, a, b, n, g, part);
-    hipLaunchKernelGGL(k_dot_finish_flat, dim3(1), dim3(256), 0, s, (const double*)part, g, out);
+    static std::atomic<unsigned> calls{0};
+    const int ticket = (int)(calls.fetch_add(1, std::memory_order_relaxed) % kNoAllocTickets);
+    // the caller's arrays may start anywhere
+    const bool wide = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
+    hipLaunchKernelGGL((wide ? k_dot_flat<true> : k_dot_flat<false>), dim3(g), dim3(kDotThreads), 0, s, a, b, n / 4, g, noalloc_scratch(), ticket, out);
     hdd_check(hipGetLastError(), "inner product (no allocation)");
 }
 void launch_seg_copy2(const DevSegments& S, float* out, const float* in1, const float* in2, int slot, hipStream_t s) {
@@ -816,11 +874,10 @@ void launch_seg_xr_update(const DevSegments& S, float* x, float* r, const float*
 }
 void launch_seg_dot(const DevSegments& S, const float* a, const float* b, int mode, hipStream_t s) {
     if (S.serial_dots)
-        hipLaunchKernelGGL(k_seg_dot_serial, dim3(S.nprob), dim3(256), 0, s, a, b, S.dpart, S.pg0, S.parts, S.max_parts);
+        hipLaunchKernelGGL(k_seg_dot_serial, dim3(S.nprob), dim3(256), 0, s, a, b, S.pg0, mode, S.active, S.scal, S.dscal);
     else
-        hipLaunchKernelGGL(k_seg_dot_partial, dim3(S.max_parts, S.nprob), dim3(256), 0, s, a, b, S.dpart, S.pg0, S.parts, S.max_parts);
-    hipLaunchKernelGGL(k_seg_finish, dim3(S.nprob), dim3(256), 0, s, (const double*)S.dpart, (const float*)nullptr, S.parts, S.max_parts,
-                       mode, S.active, S.scal, S.dscal);
+        hipLaunchKernelGGL(k_seg_dot, dim3(S.max_parts, S.nprob), dim3(kDotThreads), 0, s, a, b, S.dpart, S.ticket, S.pg0, S.parts, S.max_parts, mode,
+                           S.active, S.scal, S.dscal);
 }
 void launch_seg_copy2_d(const DevSegments& S, float* out, const float* in1, const float* in2, int slot, hipStream_t s) {
     hipLaunchKernelGGL(k_seg_copy2_d, dim3(grid_for(S.ncells)), dim3(256), 0, s, out, in1, in2, (const double*)S.dscal, slot, S.page_prob,
@@ -837,9 +894,7 @@ void launch_cast_to_float(const double* x, float* y, size_t n, hipStream_t s) {
     if (n) hipLaunchKernelGGL(k_cast_to_float, dim3(grid_for(n)), dim3(256), 0, s, x, y, n);
 }
 void launch_seg_maxabs(const DevSegments& S, const float* a, hipStream_t s) {
-    hipLaunchKernelGGL(k_seg_maxabs_partial, dim3(S.max_parts, S.nprob), dim3(256), 0, s, a, S.fpart, S.pg0, S.parts, S.max_parts);
-    hipLaunchKernelGGL(k_seg_finish, dim3(S.nprob), dim3(256), 0, s, (const double*)nullptr, (const float*)S.fpart, S.parts, S.max_parts,
-                       2, S.active, S.scal, S.dscal);
+    hipLaunchKernelGGL(k_seg_maxabs, dim3(S.max_parts, S.nprob), dim3(kDotThreads), 0, s, a, S.fpart, S.ticket, S.pg0, S.parts, S.max_parts, S.scal);
 }
 
 }  // namespace hdd

@@ -444,6 +444,7 @@ void Solver::build_device() {
         active.upload(std::vector<int>(NP, 1));
         dpart.alloc((size_t)NP * max_parts); fpart.alloc((size_t)NP * max_parts);
         scal.alloc((size_t)NP * 8); dscal.alloc((size_t)NP * 8);
+        ticket.alloc(NP);
     }
     // interface dof -> level-0 cell index (problems' dofs concatenated in problem order)
     {
@@ -755,7 +756,7 @@ DevSegments Solver::segments() {
     DevSegments sg;
     sg.nprob = nprob(); sg.max_parts = max_parts; sg.ncells = (size_t)lv[0].host.npages() * kPageCells;
     sg.pg0 = seg_pg0.p; sg.parts = seg_parts.p; sg.page_prob = page_prob.p; sg.active = active.p;
-    sg.dpart = dpart.p; sg.fpart = fpart.p; sg.scal = scal.p; sg.dscal = dscal.p;
+    sg.dpart = dpart.p; sg.fpart = fpart.p; sg.ticket = ticket.p; sg.scal = scal.p; sg.dscal = dscal.p;
     sg.serial_dots = serial_dots;
     return sg;
 }

@@ -189,6 +189,7 @@ public:
     std::vector<LevelBuffers> lv;      // V-cycle levels of the shared grid; lv[0] is the main grid
     DBuf<float> x, bvec, q, s;         // second-allocator channels (x, b, q, s)
     DBuf<double> dpart, dscal;
+    DBuf<unsigned> ticket;             // per problem, zero between reductions
     DBuf<float> fpart, scal;           // scal: 8 per problem (rho, alpha, beta, rho_old, max|r|)
     DBuf<int> seg_pg0, seg_parts, page_prob, active;
     int max_parts = 1;
