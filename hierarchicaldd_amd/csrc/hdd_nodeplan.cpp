@@ -16,10 +16,11 @@ using P_ = NodePlanHost;
 constexpr int T = NodePlanHost::kTile;
 int tiles_of(int rows) { return (rows + T - 1) / T; }
 
-// Cost of a level (both passes) in microseconds, from which the cuts are chosen: two launches
-// of dependent gathers and stores, the distinct blocks read from memory, the blocks that further
-// runs read again from cache, and the workgroups' own latency where there are many.
-constexpr double kLevelUs = 12.0, kMemoryMBPerUs = 4.5, kCacheMBPerUs = 12.0, kRunUs = 8.0 / 1280.0;
+// Cost of a level in microseconds, from which the cuts are chosen: its launches of dependent gathers
+// and stores (forward; children's sums above the first level; backward below the last), the distinct
+// blocks read from memory, the blocks that further runs read again from cache, and the workgroups'
+// own latency where there are many.
+constexpr double kLaunchUs = 5.0, kMemoryMBPerUs = 4.5, kCacheMBPerUs = 12.0, kRunUs = 8.0 / 1280.0;
 constexpr int kMaxMergedColumns = 6144;  // a node of several heights (a taller merge costs more set-up than it saves)
 constexpr int kMaxBand = 9;              // heights per band at most
 
@@ -53,7 +54,9 @@ Hash supernode_hash(const SupernodalFactor& f, int s) {
     return h;
 }
 
-long long block_tiles(long long nk, long long nrk) { return nk * (nk + 1) / 2 + nk * nrk; }
+// tiles a solve reads of a block: the inverse of a closed one (no boundary rows), or one of the two operators twice
+long long pass_tiles(long long nk, long long nrk) { return nrk ? nk * (nk + 1) / 2 + nk * nrk : nk * nk; }
+long long block_tiles(long long nk, long long nrk) { return (nrk ? 2 : 1) * pass_tiles(nk, nrk); }
 
 int run_limit(int k) {  // nodes per run whose operand vectors of k rows fit
     return std::max(1, std::min(P_::kRun, P_::kRunLdsFloats / (k + 4)));
@@ -73,7 +76,7 @@ struct Nodes {
 };
 
 double estimate_level(const std::vector<const SupernodalFactor*>& distinct, const std::vector<int>& members,
-                      const std::vector<std::vector<Hash>>& sh, int a, int b, bool* ok) {
+                      const std::vector<std::vector<Hash>>& sh, int H, int a, int b, bool* ok) {
     std::unordered_map<Hash, std::pair<long long, double>, HashKey> seen;  // node content -> members, bytes
     std::unordered_map<Hash, int, HashKey> limit;
     *ok = true;
@@ -97,7 +100,7 @@ double estimate_level(const std::vector<const SupernodalFactor*>& distinct, cons
             if (T * (nk + nrk) + 4 > P_::kMaxLdsFloats || (b > a + 1 && n[s] > kMaxMergedColumns)) { *ok = false; return 0; }
             auto& e = seen[h[s]];
             e.first += members[d];
-            e.second = 2.0 * 1024.0 * (double)block_tiles(nk, nrk) * 1e-6;
+            e.second = 1024.0 * (double)block_tiles(nk, nrk) * 1e-6;
             limit[h[s]] = run_limit(T * (nk + nrk));
         }
     }
@@ -110,7 +113,7 @@ double estimate_level(const std::vector<const SupernodalFactor*>& distinct, cons
         again_mb += (r - 1) * e.second.second;
         runs += r;
     }
-    return kLevelUs + distinct_mb / kMemoryMBPerUs + again_mb / kCacheMBPerUs + runs * kRunUs;
+    return kLaunchUs * (1 + (a > 0) + (b <= H)) + distinct_mb / kMemoryMBPerUs + again_mb / kCacheMBPerUs + runs * kRunUs;
 }
 
 // band boundaries 0 = c_0 < c_1 < .. = H + 1 of least estimated time (empty: none is possible)
@@ -124,7 +127,7 @@ std::vector<int> choose_cuts(const std::vector<const SupernodalFactor*>& distinc
     ParallelErrors errs;
 #pragma omp parallel for schedule(dynamic)
     for (size_t i = 0; i < bands.size(); ++i)
-        errs.run([&] { bands[i].us = estimate_level(distinct, members, sh, bands[i].a, bands[i].b, &bands[i].ok); });
+        errs.run([&] { bands[i].us = estimate_level(distinct, members, sh, H, bands[i].a, bands[i].b, &bands[i].ok); });
     errs.rethrow();
     std::vector<double> best(H + 2, inf);
     std::vector<int> from(H + 2, -1);
@@ -272,7 +275,7 @@ double nodeplan_bytes(const SupernodalFactor& f) {
         const Supernode& S = f.sn[s];
         n[s] += S.n;
         if (!cuts.empty() && S.parent >= 0 && level_of[f.sn[S.parent].height] == level_of[S.height]) { n[S.parent] += n[s]; continue; }
-        bytes += 2048.0 * block_tiles(tiles_of((int)n[s]), tiles_of((int)S.rows.size())) + 40.0 * (n[s] + S.rows.size());
+        bytes += 1024.0 * block_tiles(tiles_of((int)n[s]), tiles_of((int)S.rows.size())) + 44.0 * (n[s] + S.rows.size());
     }
     return bytes;
 }
@@ -359,10 +362,11 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
     }
     for (P_::Block& B : P.blocks) {
         const long long t = block_tiles(B.nk, B.nrk);
-        if (P.tiles + 2 * t > INT_MAX || (long long)P.scales + T * B.nk > INT_MAX) return false;
+        if (P.tiles + t > INT_MAX || (long long)P.scales + T * B.nk > INT_MAX) return false;
         B.scale = P.scales; P.scales += T * B.nk;
-        B.fwd = (int)P.tiles; P.tiles += t;
-        B.bwd = (int)P.tiles; P.tiles += t;
+        B.fwd = B.bwd = (int)P.tiles;
+        if (B.nrk) B.bwd += (int)(t / 2);
+        P.tiles += t;
     }
     // instances: every node of every member, its padded columns and boundary rows
     struct Inst { int y, c, prob, block; };
@@ -436,7 +440,7 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
         });
         struct Run { int i0, cnt, block; };
         std::vector<Run> runs;
-        long long frows = 0, brows = 0, ftiles = 0;
+        long long frows = 0, brows = 0, ftiles = 0, btiles = 0;
         for (size_t i = 0; i < v.size();) {
             const P_::Block& B = P.blocks[v[i].block];
             const int lim = run_limit(T * (B.nk + B.nrk));
@@ -444,19 +448,24 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
             while (k < lim && i + k < v.size() && v[i + k].block == v[i].block) ++k;
             runs.push_back({(int)(P.inst_y.size()), k, v[i].block});
             for (int j = 0; j < k; ++j) { P.inst_y.push_back(v[i + j].y); P.inst_c.push_back(v[i + j].c); P.inst_prob.push_back(v[i + j].prob); }
-            frows += B.nk + B.nrk; brows += B.nk;
-            ftiles += block_tiles(B.nk, B.nrk);
+            frows += B.nk + B.nrk;
+            ftiles += pass_tiles(B.nk, B.nrk);
             L.fwd_lds = std::max(L.fwd_lds, k * (T * B.nk + 4));
-            L.bwd_lds = std::max(L.bwd_lds, k * (T * (B.nk + B.nrk) + 4));
+            if (B.nrk) {
+                brows += B.nk;
+                btiles += pass_tiles(B.nk, B.nrk);
+                L.bwd_lds = std::max(L.bwd_lds, k * (T * (B.nk + B.nrk) + 4));
+            }
             i += k;
         }
         L.fwd_waves = level_waves(frows, frows ? (double)ftiles / frows : 0);
-        L.bwd_waves = level_waves(brows, brows ? (double)ftiles / brows : 0);
+        L.bwd_waves = level_waves(brows, brows ? (double)btiles / brows : 0);
         L.fwd0 = (int)P.fwd.size(); L.bwd0 = (int)P.bwd.size();
         for (const Run& r : runs) {
             const P_::Block& B = P.blocks[r.block];
             NodeItem it = {B.fwd, r.i0, (short)r.cnt, 1, B.nk, B.nrk, 0, 0, B.scale};
             push_items(P.fwd, it, B.nk + B.nrk, B.nk, L.fwd_waves, frows);
+            if (!B.nrk) continue;
             it.tile = B.bwd;
             push_items(P.bwd, it, B.nk, B.nk + B.nrk, L.bwd_waves, brows);
         }

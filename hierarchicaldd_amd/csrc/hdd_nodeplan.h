@@ -11,7 +11,10 @@
 //             t = b - sum of the children's u at the node's columns,
 //             u += the children's u at the node's boundary rows
 //   backward  z = [I + S^T | -W^T] [D^-2 y; z of the boundary rows]
-// so a pass is one launch per band (level), and one more forward for the
+// A closed node (no boundary rows: the root of a tree) holds its inverse, z = Linv^T Linv t, in
+// place of the triangle and its transpose (the same number of elements in one launch instead of
+// two; a launch of a few us is most of a small solve) and has no backward pass. So a pass is one
+// launch per band (level), less the last band's backward, and one more forward for the
 // children's sums where there are any. Blocks are formed in double on the
 // device at set-up and held in float, as the per-height plan holds its own. With
 // D taken out, the triangle's diagonal is exactly one: it is not stored, and
@@ -30,12 +33,12 @@ namespace hdd {
 
 // One workgroup's work: row tiles [rt0, rt1) of a run of `cnt` nodes that share a block.
 struct NodeItem {
-    int tile;            // first tile of the block's operator for this pass
+    int tile;            // first tile of the block's operator for this pass (forward of a closed block: its inverse)
     int inst0;           // the run: instances [inst0, inst0 + cnt)
     short cnt, split;    // split: waves that share a row tile
     int nk, nrk;         // column and boundary tiles of the block
     int rt0, rt1;
-    int scale;           // first of the block's D^-2
+    int scale;           // first of the block's D^-2 (closed: of its inverse's diagonal)
 };
 
 struct NodePos {  // child contributions of one row: positions in c (the zero slot when there is none);
@@ -51,8 +54,8 @@ struct NodePlanHost {
         const SupernodalFactor* f = nullptr;
         std::vector<int> sns;                // its supernodes, ascending; the last is the node's root
         int n = 0, nr = 0, nk = 0, nrk = 0;
-        int fwd = 0, bwd = 0;                // first tile of the forward and backward operator
-        int scale = 0;                       // first of its 16 nk entries of D^-2
+        int fwd = 0, bwd = 0;                // first tile of the forward and backward operator (closed: of its inverse)
+        int scale = 0;                       // first of its 16 nk entries of D^-2 (closed: of its inverse's diagonal)
     };
     struct Level {
         int fwd0 = 0, fwd1 = 0, bwd0 = 0, bwd1 = 0;  // items

@@ -13,7 +13,7 @@ struct NodePlan {
     DBuf<int> inst_y, inst_c, inst_prob, orig, zidx, more;
     DBuf<NodePos> pos_y, pos_c;
     DBuf<float> tiles, scale;  // the blocks' operators, 256 floats per tile, and their D^-2
-    DBuf<float> y, z, c;       // padded columns (forward: D^-2 y; backward, and t before it), boundary rows; a zero slot follows z and c
+    DBuf<float> t, y, z, c;    // padded columns (b less the children's sums, D^-2 y, the result), boundary rows; a zero slot follows z and c
     // false when the batch is outside the form's limits
     bool build(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, const std::vector<int>& prob_of);
     // x = (A + eps I)^{-1} b; supernodes of problems with active[p] == 0 are skipped (nullptr: none)

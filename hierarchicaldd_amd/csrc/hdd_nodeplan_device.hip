@@ -11,7 +11,7 @@
 // matrix unit can afford (it consumes tiles at about 20 TB/s over the chip, HBM
 // delivers 8). Forward tiles of a block: row tile rt < nk (Linv) has rt + 1 of
 // them, row tile nk + a (W) has nk. Backward: row tile rt has nk - rt (Linv^T)
-// and nrk (-W^T).
+// and nrk (-W^T). A closed block (nrk = 0): every row tile of its inverse has nk.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <stdexcept>
@@ -36,8 +36,8 @@ __device__ __forceinline__ bool run_stopped(const int* __restrict__ active, cons
     return true;
 }
 
-// Children's sums of a level, one thread per row: t = b - sum at its columns (held in z until the
-// backward pass), the sum itself at its boundary rows (in c, where the forward product adds to it).
+// Children's sums of a level, one thread per row: t = b - sum at its columns,
+// the sum itself at its boundary rows (in c, where the forward product adds to it).
 // On its own because a node's row tiles go to several workgroups, which all need every t of the node:
 // with the sums inside the forward kernel, its gather was 3 times its product on the 256^3 level-0
 // interiors (171 us against 49 us for the backward pass of the same level).
@@ -151,15 +151,25 @@ __device__ __forceinline__ void row_tiles(int split, int rt0, int rt1, f32x4 (*r
     row_tiles<NW, 4>(rt0, rt1, red, where, gather, out);
 }
 
-// Forward pass of a level: t into LDS, then the row tiles of [I + S; W] t. NW waves per workgroup;
-// INC: the nodes have children (t and the boundary rows' sums from k_node_children).
+__device__ __forceinline__ void store_rows(const int* __restrict__ orig, int i, f32x4 d, float* __restrict__ x) {
+    const int4 o = *reinterpret_cast<const int4*>(orig + i);
+    if (o.x >= 0) x[o.x] = d[0];
+    if (o.y >= 0) x[o.y] = d[1];
+    if (o.z >= 0) x[o.z] = d[2];
+    if (o.w >= 0) x[o.w] = d[3];
+}
+
+// Forward pass of a level: t into LDS, then the row tiles of [I + S; W] t, or of a closed node's whole
+// result (the inverse's diagonal apart as well: its row's largest term is added once, after the others).
+// NW waves per workgroup; INC: the nodes have children (t and the boundary rows' sums from k_node_children).
 template <int NW, bool INC>
 __global__ void __launch_bounds__(NW * 64) k_node_fwd(const NodeItem* __restrict__ items, const int* __restrict__ inst_y,
                                                       const int* __restrict__ inst_c, const int* __restrict__ inst_prob,
                                                       const int* __restrict__ active, const int* __restrict__ orig,
                                                       const float* __restrict__ t, const float* __restrict__ tiles,
                                                       const float* __restrict__ scale, const float* __restrict__ b,
-                                                      float* __restrict__ y, float* __restrict__ c) {
+                                                      float* __restrict__ y, float* __restrict__ c, float* __restrict__ z,
+                                                      float* __restrict__ x) {
     extern __shared__ f32x4 lds[];
     __shared__ f32x4 red[NW][64];
     const NodeItem it = items[blockIdx.x];
@@ -170,9 +180,9 @@ __global__ void __launch_bounds__(NW * 64) k_node_fwd(const NodeItem* __restrict
     const f32x4* base = reinterpret_cast<const f32x4*>(tiles) + (size_t)it.tile * 64 + lane;
     const f32x4* tcol = lds + (my_col * ld) / 4 + q;
     auto where = [&](int rt, const f32x4*& A, const f32x4*& tp, int& nt) {
-        A = base + (size_t)fwd_row(rt, it.nk) * 64;
+        A = base + (size_t)(it.nrk ? fwd_row(rt, it.nk) : (long long)rt * it.nk) * 64;
         tp = tcol;
-        nt = rt < it.nk ? rt + 1 : it.nk;
+        nt = it.nrk && rt < it.nk ? rt + 1 : it.nk;
     };
     auto gather = [&]() {
         for (int idx = threadIdx.x; idx < it.cnt * np / 4; idx += NW * 64) {
@@ -191,7 +201,12 @@ __global__ void __launch_bounds__(NW * 64) k_node_fwd(const NodeItem* __restrict
     };
     auto out = [&](int rt, f32x4 d) {
         if (col >= it.cnt) return;
-        if (rt < it.nk) {
+        if (!it.nrk) {
+            d += tcol[rt * 4] * *reinterpret_cast<const f32x4*>(scale + it.scale + rt * T + 4 * q);
+            const int i = yb + rt * T + 4 * q;
+            *reinterpret_cast<f32x4*>(z + i) = d;
+            store_rows(orig, i, d, x);
+        } else if (rt < it.nk) {
             d += tcol[rt * 4];  // the unit diagonal
             d *= *reinterpret_cast<const f32x4*>(scale + it.scale + rt * T + 4 * q);
             *reinterpret_cast<f32x4*>(y + yb + rt * T + 4 * q) = d;
@@ -244,11 +259,7 @@ __global__ void __launch_bounds__(NW * 64) k_node_bwd(const NodeItem* __restrict
         d += tcol[rt * 4];
         const int i = yb + rt * T + 4 * q;
         *reinterpret_cast<f32x4*>(z + i) = d;
-        const int4 o = *reinterpret_cast<const int4*>(orig + i);
-        if (o.x >= 0) x[o.x] = d[0];
-        if (o.y >= 0) x[o.y] = d[1];
-        if (o.z >= 0) x[o.z] = d[2];
-        if (o.w >= 0) x[o.w] = d[3];
+        store_rows(orig, i, d, x);
     };
     row_tiles<NW>(it.split, it.rt0, it.rt1, red, where, gather, out);
 }
@@ -291,7 +302,9 @@ __global__ void __launch_bounds__(256) k_node_columns(const SetupSupernode* __re
 // A's tiles along a row at a + 16 k and B's down a column at b + 16 k * ld. Four tile pairs go through
 // LDS at a time and the next four load meanwhile: one at a time, the wait for each pair made the
 // inverse of a 2080-row block take 30 ms.
+// With kAT, A is the transpose of what `a` points to: its tiles go down a column at a + 16 k * ld.
 constexpr int kPairs = 4;
+template <bool kAT = false>
 __device__ __forceinline__ double tile_products(double s, double sign, const double* __restrict__ a, const double* b, long long ld, int k0,
                                                 int k1, double (*as)[T][T + 1], double (*bs)[T][T + 1]) {
     const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
@@ -300,14 +313,14 @@ __device__ __forceinline__ double tile_products(double s, double sign, const dou
 #pragma unroll
         for (int u = 0; u < kPairs; ++u) {
             const bool in = k + u < k1;
-            an[u] = in ? a[r * ld + (long long)(k + u) * T + c] : 0.0;
+            an[u] = in ? (kAT ? a[((long long)(k + u) * T + r) * ld + c] : a[r * ld + (long long)(k + u) * T + c]) : 0.0;
             bn[u] = in ? b[((long long)(k + u) * T + r) * ld + c] : 0.0;
         }
     };
     if (k0 < k1) fetch(k0);
     for (int k = k0; k < k1; k += kPairs) {
 #pragma unroll
-        for (int u = 0; u < kPairs; ++u) { as[u][r][c] = sign * an[u]; bs[u][r][c] = bn[u]; }
+        for (int u = 0; u < kPairs; ++u) { (kAT ? as[u][c][r] : as[u][r][c]) = sign * an[u]; bs[u][r][c] = bn[u]; }
         __syncthreads();
         if (k + kPairs < k1) fetch(k + kPairs);
 #pragma unroll
@@ -347,7 +360,8 @@ __global__ void __launch_bounds__(256) k_node_inverse(const SetupBlock* __restri
     }
 }
 
-// forward operator, one workgroup per row tile: S = D Linv - I rounded to float (and D^-2), or W = L21 Linv (double sums)
+// forward operator, one workgroup per row tile: S = D Linv - I rounded to float (and D^-2), or W = L21 Linv (double sums);
+// of a closed block the inverse Linv^T Linv (double sums), a tile and its mirror image from the same sums
 __global__ void __launch_bounds__(256) k_node_forward_tiles(const SetupBlock* __restrict__ blocks, const int2* __restrict__ rows,
                                                             const double* __restrict__ L, const double* __restrict__ X,
                                                             float* __restrict__ tiles, float* __restrict__ scale) {
@@ -357,6 +371,19 @@ __global__ void __launch_bounds__(256) k_node_forward_tiles(const SetupBlock* __
     const int r = threadIdx.x >> 4, c = threadIdx.x & 15, rt = rw.y;
     const long long np = (long long)B.nk * T;
     const double* Xb = X + B.x;
+    if (!B.nrk) {
+        const int at = ((c >> 2) * 16 + r) * 4 + (c & 3), mirror = ((r >> 2) * 16 + c) * 4 + (r & 3);
+        float* M = tiles + (size_t)B.fwd * 256;
+        for (int j = 0; j <= rt; ++j) {
+            const double v = tile_products<true>(0.0, 1.0, Xb + rt * T, Xb + j * T, np, rt, B.nk, ls, xs);
+            const bool diag = j == rt && r == c;
+            const float f = diag ? 0.f : (float)v;
+            if (diag) scale[B.scale + rt * T + r] = (float)v;
+            M[((size_t)rt * B.nk + j) * 256 + at] = f;
+            if (j < rt) M[((size_t)j * B.nk + rt) * 256 + mirror] = f;
+        }
+        return;
+    }
     float* out = tiles + ((size_t)B.fwd + fwd_row(rt, B.nk)) * 256 + ((c >> 2) * 16 + r) * 4 + (c & 3);
     if (rt < B.nk) {
         const double d = L[B.l + (rt * T + r) * np + rt * T + r];
@@ -423,7 +450,7 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
     P.pos_c.resize(std::max<size_t>(1, P.pos_c.size()), NodePos{P.csize, P.csize});
     pos_y.upload(P.pos_y); pos_c.upload(P.pos_c);
     tiles.alloc((size_t)P.tiles * 256); scale.alloc(P.scales);
-    y.alloc(P.ysize); z.alloc((size_t)P.ysize + 1); c.alloc((size_t)P.csize + 1);
+    t.alloc(P.ysize); y.alloc(P.ysize); z.alloc((size_t)P.ysize + 1); c.alloc((size_t)P.csize + 1);
     // the blocks in chunks: their supernodes' columns uploaded and put in place, inverted and packed
     constexpr size_t kChunk = size_t(24) << 20;  // doubles per chunk, unless one block needs more
     auto doubles = [](const NodePlanHost::Block& B) { return (size_t)(B.nk + B.nrk) * T * B.nk * T; };
@@ -456,7 +483,10 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
             sb.push_back({l, xo, B.nk, B.nrk, B.fwd, B.bwd, B.scale, 0});
             l += (long long)doubles(B);
             xo += (long long)B.nk * T * B.nk * T;
-            for (int r = 0; r < B.nk; ++r) { strips.push_back(make_int2(id, r)); brows.push_back(make_int2(id, r)); }
+            for (int r = 0; r < B.nk; ++r) {
+                strips.push_back(make_int2(id, r));
+                if (B.nrk) brows.push_back(make_int2(id, r));
+            }
             for (int r = 0; r < B.nk + B.nrk; ++r) rows.push_back(make_int2(id, r));
         }
         std::vector<SetupSupernode> ss;
@@ -486,7 +516,8 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
         }
         DBuf<SetupBlock> dsb; dsb.upload(sb);
         DBuf<int2> dst, drw, dbr;
-        dst.upload(strips); drw.upload(rows); dbr.upload(brows);
+        dst.upload(strips); drw.upload(rows);
+        if (!brows.empty()) dbr.upload(brows);
         DBuf<SetupSupernode> dss; dss.upload(ss);
         DBuf<int> dlist; dlist.upload(list.empty() ? std::vector<int>(1, 0) : list);
         DBuf<double> dsrc; dsrc.upload(host);
@@ -495,7 +526,8 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
         launch(k_node_inverse, (int)strips.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)dst.p, (const double*)dL.p, dX.p);
         launch(k_node_forward_tiles, (int)rows.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)drw.p, (const double*)dL.p,
                (const double*)dX.p, tiles.p, scale.p);
-        launch(k_node_backward_tiles, (int)brows.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)dbr.p, tiles.p);
+        if (!brows.empty())
+            launch(k_node_backward_tiles, (int)brows.size(), 4, 0, nullptr, (const SetupBlock*)dsb.p, (const int2*)dbr.p, tiles.p);
         hdd_check(hipGetLastError(), "node blocks");
         hdd_check(hipStreamSynchronize(nullptr), "node blocks");
     }
@@ -504,18 +536,18 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
 
 size_t NodePlan::bytes() const {
     return (fwd.n + bwd.n) * sizeof(NodeItem) + (inst_y.n + inst_c.n + inst_prob.n + orig.n + zidx.n + more.n) * 4 +
-           (pos_y.n + pos_c.n) * 8 + (tiles.n + scale.n + y.n + z.n + c.n) * 4;
+           (pos_y.n + pos_c.n) * 8 + (tiles.n + scale.n + t.n + y.n + z.n + c.n) * 4;
 }
 
 void NodePlan::solve(const float* b, float* x, const int* active, hipStream_t s) {
     auto fwd_level = [&](const NodePlanHost::Level& L) {
         if (L.children)
             hipLaunchKernelGGL(k_node_children, dim3((unsigned)((L.y1 - L.y0 + L.c1 - L.c0 + 255) / 256)), dim3(256), 0, s, L.y0, L.y1, L.c0, L.c1,
-                               (const NodePos*)pos_y.p, (const NodePos*)pos_c.p, (const int*)more.p, (const int*)orig.p, b, z.p, c.p);
+                               (const NodePos*)pos_y.p, (const NodePos*)pos_c.p, (const int*)more.p, (const int*)orig.p, b, t.p, c.p);
         auto go = [&](auto kernel) {
             launch(kernel, L.fwd1 - L.fwd0, L.fwd_waves, L.fwd_lds * sizeof(float), s, (const NodeItem*)fwd.p + L.fwd0, (const int*)inst_y.p,
-                   (const int*)inst_c.p, (const int*)inst_prob.p, active, (const int*)orig.p, (const float*)z.p, (const float*)tiles.p,
-                   (const float*)scale.p, b, y.p, c.p);
+                   (const int*)inst_c.p, (const int*)inst_prob.p, active, (const int*)orig.p, (const float*)t.p, (const float*)tiles.p,
+                   (const float*)scale.p, b, y.p, c.p, z.p, x);
         };
         if (L.fwd_waves == 4) { if (L.children) go(k_node_fwd<4, true>); else go(k_node_fwd<4, false>); }
         else { if (L.children) go(k_node_fwd<16, true>); else go(k_node_fwd<16, false>); }

@@ -60,6 +60,10 @@ void check_indices(const NodePlanHost& P) {
         need((fwd ? L.fwd_lds : L.bwd_lds) <= NodePlanHost::kMaxLdsFloats, "LDS size");
         need(it.scale >= 0 && it.scale + T * it.nk <= P.scales && it.scale % 4 == 0, "scale");
         for (int r = it.rt0; r < it.rt1; ++r) {
+            if (fwd && !it.nrk) {
+                need(it.tile >= 0 && it.tile + (long long)(r + 1) * it.nk <= P.tiles, "tiles");
+                continue;
+            }
             const long long base = it.tile + (fwd ? (r < it.nk ? (long long)r * (r + 1) / 2 : (long long)it.nk * (it.nk + 1) / 2 + (long long)(r - it.nk) * it.nk)
                                                   : (long long)r * (it.nk + it.nrk) - (long long)r * (r - 1) / 2);
             const long long nt = fwd ? (r < it.nk ? r + 1 : it.nk) : it.nk + it.nrk - r;
@@ -69,6 +73,7 @@ void check_indices(const NodePlanHost& P) {
             const int y = P.inst_y[it.inst0 + j], c = P.inst_c[it.inst0 + j];
             need(y >= L.y0 && y % T == 0 && y + T * it.nk <= L.y1 && L.y1 <= P.ysize, "columns");
             need(c >= L.c0 && c % T == 0 && c + T * it.nrk <= L.c1 && L.c1 <= P.csize, "boundary rows");
+            if (fwd && !it.nrk) for (int r = it.rt0; r < it.rt1; ++r) ++bcount[y / T + r];  // the whole solve
             for (int r = it.rt0; r < it.rt1; ++r) ++(fwd ? (r < it.nk ? fcount[y / T + r] : ccount[c / T + r - it.nk]) : bcount[y / T + r]);
         }
     };
@@ -104,6 +109,13 @@ double emulate(const NodePlanHost& P, const std::vector<const SupernodalFactor*>
         for (int i = 0; i < np; ++i) for (int j = 0; j <= i; ++j) inv[(size_t)j * np + i] = L[(size_t)i * np + j];
         invert_lower(inv, np);
         S[k].assign((size_t)np * np, 0.0); W[k].assign((size_t)nr * np, 0.0); D2[k].resize(np);
+        if (!nr) {  // closed: the inverse
+            for (int i = 0; i < np; ++i)
+                for (int j = 0; j < np; ++j)
+                    for (int q = std::max(i, j); q < np; ++q) S[k][(size_t)i * np + j] += inv[(size_t)i * np + q] * inv[(size_t)j * np + q];
+            by_fwd[B.fwd] = (int)k;
+            continue;
+        }
         for (int i = 0; i < np; ++i) {
             const double d = L[(size_t)i * np + i];
             D2[k][i] = 1.0 / (d * d);
@@ -116,7 +128,7 @@ double emulate(const NodePlanHost& P, const std::vector<const SupernodalFactor*>
             }
         by_fwd[B.fwd] = (int)k; by_bwd[B.bwd] = (int)k;
     }
-    std::vector<double> b(P.n), x(P.n, 0.0), y(P.ysize, 0.0), z(P.ysize + 1, 0.0), c(P.csize + 1, 0.0);
+    std::vector<double> b(P.n), x(P.n, 0.0), t0(P.ysize, 0.0), y(P.ysize, 0.0), z(P.ysize + 1, 0.0), c(P.csize + 1, 0.0);
     uint32_t s = 7;
     for (auto& v : b) { s = s * 1664525u + 1013904223u; v = (s >> 8) / 16777216.0 - 0.5; }
     auto children = [&](const NodePos& q) {
@@ -128,7 +140,7 @@ double emulate(const NodePlanHost& P, const std::vector<const SupernodalFactor*>
     };
     for (const auto& L : P.levels) {
         if (L.children) {
-            for (int i = L.y0; i < L.y1; ++i) z[i] = (P.orig[i] >= 0 ? b[P.orig[i]] : 0.0) - children(P.pos_y[i]);
+            for (int i = L.y0; i < L.y1; ++i) t0[i] = (P.orig[i] >= 0 ? b[P.orig[i]] : 0.0) - children(P.pos_y[i]);
             for (int i = L.c0; i < L.c1; ++i) c[i] = children(P.pos_c[i]);
         }
         for (int i = L.fwd0; i < L.fwd1; ++i) {
@@ -137,10 +149,14 @@ double emulate(const NodePlanHost& P, const std::vector<const SupernodalFactor*>
             for (int j = 0; j < it.cnt; ++j) {
                 const int yb = P.inst_y[it.inst0 + j], cb = P.inst_c[it.inst0 + j];
                 std::vector<double> t(np);
-                for (int q = 0; q < np; ++q) t[q] = L.children ? z[yb + q] : (P.orig[yb + q] >= 0 ? b[P.orig[yb + q]] : 0.0);
+                for (int q = 0; q < np; ++q) t[q] = L.children ? t0[yb + q] : (P.orig[yb + q] >= 0 ? b[P.orig[yb + q]] : 0.0);
                 for (int r = it.rt0 * T; r < it.rt1 * T; ++r) {
                     double a = 0;
-                    if (r < np) {
+                    if (!it.nrk) {
+                        for (int q = 0; q < np; ++q) a += S[k][(size_t)r * np + q] * t[q];
+                        z[yb + r] = a;
+                        if (P.orig[yb + r] >= 0) x[P.orig[yb + r]] = a;
+                    } else if (r < np) {
                         for (int q = 0; q < r; ++q) a += S[k][(size_t)r * np + q] * t[q];
                         y[yb + r] = (a + t[r]) * D2[k][r];
                     } else {
