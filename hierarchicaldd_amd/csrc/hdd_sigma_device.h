@@ -22,6 +22,26 @@ struct CsrDev {
     size_t bytes() const { return p.n * 4 + ix.n * 4 + v.n * 4; }
 };
 
+// A sparse matrix in slices of 64 consecutive rows for products with one row per lane: entry k of
+// the slice's rows side by side, so a wavefront reads whole lines and all of a row's loads are in
+// flight at once. Rows without entries may be left out (`row`: the rows that are there).
+struct SlicedEntry { int ix; float v; };  // ix < 0: padding
+struct SlicedView {
+    int rows = 0, width = 0;            // rows held; entries per row where all slices have as many (0: `slice`)
+    const int2* slice = nullptr;        // first entry and entries per row of each slice
+    const int* row = nullptr;           // nullptr: row i is row i of the matrix
+    const SlicedEntry* e = nullptr;
+};
+struct SlicedDev {
+    int rows = 0, width = 0;
+    DBuf<int2> slice;
+    DBuf<int> row;
+    DBuf<SlicedEntry> e;
+    void upload(const Csr& m, bool skip_empty);
+    SlicedView view() const { return {rows, width, slice.p, row.p, e.p}; }
+    size_t bytes() const { return slice.n * 8 + row.n * 4 + e.n * 8; }
+};
+
 // Exact solve x = (A + eps I)^{-1} b for a batch of independent matrices,
 // from their supernodal factors: the dense-node form (hdd_nodeplan.h), or the
 // per-height form (layout in hdd_triplan.h) for refined solves, for batches
@@ -79,9 +99,9 @@ struct TriPlan {
 struct SigmaLevel {
     int n_if = 0, n_int = 0;
     int n_distinct = 0;  // distinct interior matrices (subdomains of the same shape share one factor)
-    CsrDev Air, AirT, Arr, P, PT;  // P: this level -> next coarser (rows = this level), PT its transpose
+    SlicedDev Air, AirT, Arr, P, PT;  // P: this level -> next coarser (rows = this level), PT its transpose; Air without its empty rows
     TriPlan Lii, Lrr;
-    DBuf<float> u, b, r, vb, vx, tmp;
+    DBuf<float> u, b, r, vb, vx, tmp;  // vb: zero at the rows Air leaves out
 };
 
 // Host factors of one problem's interface solver: the exact solves of
@@ -153,7 +173,7 @@ struct SigmaDevice {
     double factor_seconds = 0;
     size_t plan_bytes = 0;
     ~SigmaDevice();
-    void smooth(int l, hipStream_t s);
+    void smooth(int l, hipStream_t s, bool u_zero = false);  // u_zero: from u = 0 (and u is not read)
     void residual(int l, hipStream_t s);
     void vcycle(hipStream_t s, bool first);
     // per-problem flags of the batch PCG (device): exact solves skip stopped problems; nullptr: skip nothing
