@@ -35,13 +35,15 @@ void upload_constants();
 // V-cycle kernels, float storage and half (FP16) storage with float arithmetic
 void launch_smooth(const DevLevel& L, const float* u_in, float* u_out, const float* b, bool interior, bool boundary, hipStream_t s);
 void launch_smooth(const DevLevel& L, const __half* u_in, __half* u_out, const __half* b, bool interior, bool boundary, hipStream_t s);
-// Sweeps of a level whose Active cells couple only within small clusters of pages, several in one
-// launch (k_cluster_sweeps): workgroups of `slots` page slots hold whole clusters in LDS.
+// Sweeps of a level whose Active cells couple only within small clusters, several in one launch
+// (k_cluster_sweeps): workgroups of `slots` cells hold whole clusters in LDS.
 struct DevClusters {
-    int nwg = 0, slots = 0, entries = 0;       // workgroups, page slots each, LDS values (the slots' cells, then the halo)
-    const int* wg_page = nullptr;              // [nwg*slots] page of each slot, -1: empty
-    const uint16_t* nbr = nullptr;             // [nwg][6][slots*256] LDS value of each cell's face neighbour (its own where the face bit is not set)
-    const int *halo_ptr = nullptr, *halo_cell = nullptr;  // values past the slots' cells: cells of the level ([nwg+1], then the lists)
+    int nwg = 0, slots = 0, threads = 0;       // workgroups, cells each (a multiple of their threads)
+    int entries = 0;                           // LDS values (the slots, then the halo)
+    bool rest = false;                         // the residual also clears the cells that are not Active
+    const int* cell = nullptr;                 // [nwg*slots] Active cell of each slot, -1: empty
+    const uint16_t* nbr = nullptr;             // [nwg][6][slots] LDS value of each cell's face neighbour (its own where the face bit is not set)
+    const int *halo_ptr = nullptr, *halo_cell = nullptr;  // values past the slots: cells of the level ([nwg+1], then the lists)
 };
 // in turn: count[i] sweeps of the interior (kSweepInterior) and / or boundary (kSweepBoundary) cells
 enum { kSweepInterior = 1, kSweepBoundary = 2 };

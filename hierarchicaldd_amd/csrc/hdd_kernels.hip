@@ -159,40 +159,38 @@ __global__ void __launch_bounds__(64 * kSweepPages) k_smooth(DevLevel L, const S
 }
 
 // Several sweeps of a level in one launch, and the residual after them, where
-// its Active cells couple only within small clusters of pages (the coarse
-// levels: a cluster is the part of a subdomain, or of a few that meet inside an
-// obstacle). A workgroup holds whole clusters in LDS, C cells per thread
-// (cell i of thread t: i * blockDim + t of the workgroup's slots * 256), and
-// sweeps them with the operations of Stencil4 and k_smooth, keeping every
-// iterate in the level's storage type, so the result is bit-identical to one
-// launch per sweep. nbr gives each cell's face neighbours as LDS values; a
-// neighbour outside the workgroup is a cell no sweep writes, held in the halo
-// behind the slots' cells. Where a face bit is not set it names the cell itself,
-// whose difference is an exact zero. The cells ping-pong between two copies (the
-// halo is in both), one barrier per sweep. u is updated in place: no other
-// workgroup reads the Active cells of this one's pages.
+// its Active cells couple only within small clusters (the coarse levels: a
+// cluster is the part of a subdomain, or of a few that meet inside an obstacle).
+// A workgroup holds whole clusters in LDS, C cells per thread (cell i of thread
+// t: slot i * blockDim + t), and sweeps them with the operations of Stencil4 and
+// k_smooth, keeping every iterate in the level's storage type, so the result is
+// bit-identical to one launch per sweep. nbr gives each cell's face neighbours as
+// LDS values; a neighbour outside the workgroup is a cell no sweep writes, held
+// in the halo behind the slots. Where a face bit is not set it names the cell
+// itself, whose difference is an exact zero. The cells ping-pong between two
+// copies (the halo is in both), one barrier per sweep. u is updated in place: no
+// other workgroup reads the Active cells of this one's clusters.
 //
 // Bound by instruction issue and the barrier: a sweep is 6 LDS reads, about 25
 // operations and one write per cell, against a launch of 3.3-5 us per sweep of a
-// small level. The 200 sweeps of a V-cycle's bottom take 36 us where clusters are
-// single pages (71 with four pages to every workgroup, whose 16 waves share the
-// barrier), 51 us at up to four pages (200 launches: 650), 76 us at up to eight;
-// the seven sweeps and the residual of a small level 5-12 us instead of 35.
-// More than 32 pages would spill (68 us for the seven sweeps of 46-page clusters
-// at 100^3, 45 us as launches), so those levels keep one launch per sweep.
+// small level. The seven sweeps and the residual of a level take 4.7 us at 343 cells
+// a cluster, 13 us at 3375 to 4096 (eight launches: 35-46 us); 200 sweeps of clusters
+// of up to 343 cells 28 us. Cells, not pages, make up a cluster: by pages, the 16^3
+// clusters of a 100^3 domain's level 1 lie in 46 pages and did not fit, and its
+// bottom clusters filled 2048 slots (76 us for the 200 sweeps).
 template <class S, int C>
 __global__ void __launch_bounds__(1024) k_cluster_sweeps(DevLevel L, DevClusters W, S* u, const S* __restrict__ b, S* __restrict__ r,
                                                          SweepPhases ph, int u_zero) {
     extern __shared__ __align__(16) unsigned char cluster_lds[];
     S* us = reinterpret_cast<S*>(cluster_lds);
-    const int wg = blockIdx.x, nt = blockDim.x, cells = W.slots * kPageCells;
+    const int wg = blockIdx.x, nt = blockDim.x, cells = W.slots;
     float cur[C], bv[C], wgt[C];
     unsigned nb[C][3];    // LDS values of the six face neighbours, two per register
     unsigned kind = 0;    // two bits per cell: kSweepInterior, kSweepBoundary, 0 (never swept)
     // cell i's place in the level, -1 in an empty slot or a stopped problem's page
     auto place = [&](int i) {
-        const int ci = i * nt + (int)threadIdx.x, p = W.wg_page[wg * W.slots + (ci >> 8)];
-        return p >= 0 && !page_stopped(L, p) ? p * kPageCells + (ci & 255) : -1;
+        const int e = W.cell[wg * cells + i * nt + (int)threadIdx.x];
+        return e >= 0 && !page_stopped(L, e >> 8) ? e : -1;
     };
 #pragma unroll
     for (int i = 0; i < C; ++i) {
@@ -211,6 +209,12 @@ __global__ void __launch_bounds__(1024) k_cluster_sweeps(DevLevel L, DevClusters
         }
         st(us, ci, cur[i]);
         st(us, W.entries + ci, cur[i]);
+    }
+    if (r && W.rest) {  // a share of the level's cells
+        const int n = L.np * kPageCells, share = (n + W.nwg - 1) / W.nwg, end = min(n, (wg + 1) * share);
+#pragma unroll 8
+        for (int c = wg * share + (int)threadIdx.x; c < end; c += nt)
+            if (!(L.flags[c] & kActive) && !page_stopped(L, c >> 8)) st(r, c, 0.f);
     }
     const int h0 = W.halo_ptr[wg], nh = W.halo_ptr[wg + 1] - h0;
     for (int h = threadIdx.x; h < nh; h += nt) {
@@ -253,10 +257,56 @@ __global__ void __launch_bounds__(1024) k_cluster_sweeps(DevLevel L, DevClusters
     for (int i = 0; i < C; ++i) {
         const int e = place(i);
         if (e < 0) continue;
-        const bool act = ((kind >> (2 * i)) & 3u) != 0;
-        if (act) st(u, e, cur[i]);
-        if (r) st(r, e, act ? residual(i, from) : 0.f);
+        st(u, e, cur[i]);
+        if (r) st(r, e, residual(i, from));
     }
+}
+
+// k_cluster_sweeps where a workgroup is one wavefront with a cell per lane (clusters of up to 64 cells:
+// the bottom levels) and the cells around it hold zero: the neighbours come from the lanes' registers
+// (ds_bpermute), so a sweep has no LDS write and no barrier in its chain. The 200 sweeps of a bottom
+// level take 21 us instead of 28.
+template <class S>
+__global__ void __launch_bounds__(64) k_cluster_wave(DevLevel L, DevClusters W, S* u, const S* __restrict__ b, S* __restrict__ r, SweepPhases ph,
+                                                     int u_zero) {
+    const int wg = blockIdx.x, lane = threadIdx.x;
+    int e = W.cell[wg * 64 + lane];
+    int from[6], keep[6];  // the neighbour's lane as ds_bpermute wants it; 0 for a cell outside, whose value is zero
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+        const int v = W.nbr[(size_t)wg * 6 * 64 + f * 64 + lane];
+        from[f] = (v & 63) * 4;
+        keep[f] = v < 64 ? -1 : 0;
+    }
+    if (e >= 0 && page_stopped(L, e >> 8)) e = -1;
+    float cur = 0.f, bv = 0.f, wgt = 0.f;
+    int kind = 0;
+    if (e >= 0) {
+        const uint32_t fl = L.flags[e];
+        kind = fl & kBoundary ? kSweepBoundary : kSweepInterior;
+        wgt = c_omega_fc[__popc(fl & (0x3fu * kFaceMX))];
+        bv = ld(b, e);
+        if (!u_zero) cur = ld(u, e);
+    }
+    auto residual = [&]() {
+        float n[6], result = 0.f;
+#pragma unroll
+        for (int f = 0; f < 6; ++f) n[f] = __int_as_float(__builtin_amdgcn_ds_bpermute(from[f], __float_as_int(cur)) & keep[f]);
+#pragma unroll
+        for (int f = 0; f < 6; ++f) result -= (n[f] - cur);
+        return bv - result;
+    };
+    for (int k = 0; k < ph.n; ++k) {
+        const bool sel = (kind & ph.cells[k]) != 0;
+        for (int it = 0; it < ph.count[k]; ++it) {
+            const float v = stored(u, cur + wgt * residual());
+            cur = sel ? v : cur;
+        }
+    }
+    const float res = residual();
+    if (e < 0) return;
+    st(u, e, cur);
+    if (r) st(r, e, res);
 }
 
 // residual at Active cells; other cells of r are written 0 (the value they
@@ -751,20 +801,23 @@ template <class S, int C>
 static void cluster_sweeps_c(const DevLevel& L, const DevClusters& W, S* u, const S* b, S* r, const SweepPhases& ph, bool u_zero, hipStream_t s) {
     const size_t lds = 2 * (size_t)W.entries * sizeof(S);
     if (lds > 48 * 1024)
-        hdd_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cluster_sweeps<S, C>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+        hdd_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cluster_sweeps<S, C>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024),
                   "cluster sweeps' LDS");
-    hipLaunchKernelGGL((k_cluster_sweeps<S, C>), dim3(W.nwg), dim3(W.slots * kPageCells / C), lds, s, L, W, u, b, r, ph, (int)u_zero);
+    hipLaunchKernelGGL((k_cluster_sweeps<S, C>), dim3(W.nwg), dim3(W.threads), lds, s, L, W, u, b, r, ph, (int)u_zero);
 }
 template <class S>
 static void cluster_sweeps_t(const DevLevel& L, const DevClusters& W, S* u, const S* b, S* r, const SweepPhases& ph, bool u_zero, hipStream_t s) {
     if (!W.nwg) return;
-    // up to 1024 threads: one cell each up to four page slots, then C = slots / 4 cells each
-    switch (W.slots) {
-        case 1: case 2: case 4: cluster_sweeps_c<S, 1>(L, W, u, b, r, ph, u_zero, s); break;
-        case 8: cluster_sweeps_c<S, 2>(L, W, u, b, r, ph, u_zero, s); break;
-        case 16: cluster_sweeps_c<S, 4>(L, W, u, b, r, ph, u_zero, s); break;
-        case 32: cluster_sweeps_c<S, 8>(L, W, u, b, r, ph, u_zero, s); break;
-        default: throw std::runtime_error("cluster sweeps: slots must be a power of two up to 32");
+    if (W.slots == 64 && W.threads == 64 && !W.rest) {
+        hipLaunchKernelGGL(k_cluster_wave<S>, dim3(W.nwg), dim3(64), 0, s, L, W, u, b, r, ph, (int)u_zero);
+        return;
+    }
+    switch (W.slots / W.threads) {  // cells per thread
+        case 1: cluster_sweeps_c<S, 1>(L, W, u, b, r, ph, u_zero, s); break;
+        case 2: cluster_sweeps_c<S, 2>(L, W, u, b, r, ph, u_zero, s); break;
+        case 4: cluster_sweeps_c<S, 4>(L, W, u, b, r, ph, u_zero, s); break;
+        case 8: cluster_sweeps_c<S, 8>(L, W, u, b, r, ph, u_zero, s); break;
+        default: throw std::runtime_error("cluster sweeps: cells per thread");
     }
 }
 template <class S>

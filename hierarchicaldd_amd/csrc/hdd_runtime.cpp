@@ -262,32 +262,25 @@ void Solver::merge_levels() {
 DevClusters LevelBuffers::clusters() const {
     DevClusters c;
     c.slots = cl_slots; c.entries = cl_entries;
-    c.nwg = cl_slots ? (int)(cl_page.n / cl_slots) : 0;
-    c.wg_page = cl_page.p; c.nbr = cl_nbr.p; c.halo_ptr = cl_halo_ptr.p; c.halo_cell = cl_halo_cell.p;
+    c.nwg = cl_slots ? (int)(cl_cell.n / cl_slots) : 0;
+    c.threads = cl_threads; c.rest = cl_rest;
+    c.cell = cl_cell.p; c.nbr = cl_nbr.p; c.halo_ptr = cl_halo_ptr.p; c.halo_cell = cl_halo_cell.p;
     return c;
 }
 
-// Clusters of a level's pages: pages are linked when an Active cell of one has a
-// set face bit to an Active cell of the other; a sweep of one cluster reads no
-// cell that a sweep of another writes. Whole clusters are packed into workgroups
-// of `slots` page slots (the largest cluster, rounded up to a power of two;
-// one cluster each while there are no more than kSpread, so that they run side
-// by side), each with the LDS value of every cell's face neighbours and the
-// list of cells outside the workgroup that its faces read. zero_outside: cells
-// that are not Active hold zero on this level (every level but 0), so that
-// list is one of them. False when a cluster is larger than kMaxSlots pages or
-// a workgroup's two copies exceed the LDS.
+// Clusters of a level's Active cells: cells are linked across set face bits, so a sweep of one cluster
+// reads no cell that a sweep of another writes. A workgroup holds whole clusters, one per workgroup
+// while there are no more than kSpread (they run side by side), packed beyond that; `slots` cells per
+// workgroup, the largest cluster rounded up to whole wavefronts. Each has the LDS value of every cell's
+// face neighbours and the list of cells outside it that its faces read. zero_outside: cells that are not
+// Active hold zero on this level (every level but 0), so that list is one of them. False when a
+// cluster is larger than kMaxCells or a workgroup's two copies exceed the LDS.
 static bool plan_clusters(LevelBuffers& LB, bool zero_outside) {
-    constexpr int kMaxSlots = 32, kSpread = 512, kLdsBytes = 150 * 1024;
+    constexpr int kMaxCells = 8192, kSpread = 512, kLdsBytes = 150 * 1024;
     static const int d[6][3] = {{-1, 0, 0}, {1, 0, 0}, {0, -1, 0}, {0, 1, 0}, {0, 0, -1}, {0, 0, 1}};
     const PagedLevel& H = LB.host;
     const int np = H.npages();
     if (np == 0) return false;
-    std::vector<int> parent(np), size(np, 1), nbp((size_t)np * 6);
-    auto find = [&](int a) {
-        while (parent[a] != a) a = parent[a] = parent[parent[a]];
-        return a;
-    };
     // cell c's neighbour across face q: its cell in the page, or in the face's neighbour page (outside = true)
     auto step = [](int c, int q, bool& outside) {
         const int x = c >> 6, y = (c >> 3) & 7, z = c & 7;
@@ -295,86 +288,134 @@ static bool plan_clusters(LevelBuffers& LB, bool zero_outside) {
         outside = X < 0 || X >= kPX || Y < 0 || Y >= kPY || Z < 0 || Z >= kPZ;
         return page_cell(X + kPX, Y + kPY, Z + kPZ);
     };
-    for (int p = 0; p < np; ++p) parent[p] = p;
+    // the connected pieces of each page's Active cells
+    std::vector<uint8_t> piece((size_t)np * kPageCells);
+    std::vector<int> nbp((size_t)np * 6), first(np + 1, 0);
+#pragma omp parallel for schedule(static)
+    for (int p = 0; p < np; ++p) {
+        const Int3 o = H.page_base[p];
+        const uint32_t* fl = &H.flags[(size_t)p * kPageCells];
+        uint8_t* pc = &piece[(size_t)p * kPageCells];
+        for (int q = 0; q < 6; ++q) nbp[(size_t)p * 6 + q] = H.page_at(o.x + d[q][0] * kPX, o.y + d[q][1] * kPY, o.z + d[q][2] * kPZ);
+        bool seen[kPageCells] = {};
+        int todo[kPageCells], n = 0;
+        for (int c = 0; c < kPageCells; ++c) {
+            if (!(fl[c] & kActive) || seen[c]) continue;
+            int left = 0;
+            todo[left++] = c; seen[c] = true;
+            while (left) {
+                const int k = todo[--left];
+                pc[k] = (uint8_t)n;
+                for (int q = 0; q < 6; ++q) {
+                    if (!(fl[k] & (kFaceMX << q))) continue;
+                    bool out;
+                    const int m = step(k, q, out);
+                    if (!out && (fl[m] & kActive) && !seen[m]) { seen[m] = true; todo[left++] = m; }
+                }
+            }
+            ++n;
+        }
+        first[p + 1] = n;
+    }
+    for (int p = 0; p < np; ++p) first[p + 1] += first[p];
+    const int pieces = first[np];
+    // pieces joined across the pages' faces
+    std::vector<int> parent(pieces), size(pieces, 0);
+    for (int k = 0; k < pieces; ++k) parent[k] = k;
+    auto find = [&](int a) {
+        while (parent[a] != a) a = parent[a] = parent[parent[a]];
+        return a;
+    };
+    for (int p = 0; p < np; ++p)
+        for (int c = 0; c < kPageCells; ++c)
+            if (H.flags[(size_t)p * kPageCells + c] & kActive) ++size[first[p] + piece[(size_t)p * kPageCells + c]];
     constexpr int kBlock = 4096;  // pages whose links are found in parallel before they are joined
-    std::vector<char> link((size_t)kBlock * 6);
+    std::vector<std::vector<std::pair<int, int>>> links(kBlock);
     for (int p0 = 0; p0 < np; p0 += kBlock) {
         const int p1 = std::min(np, p0 + kBlock);
 #pragma omp parallel for schedule(static)
         for (int p = p0; p < p1; ++p) {
-            const Int3 o = H.page_base[p];
-            const uint32_t* fl = &H.flags[(size_t)p * kPageCells];
+            auto& to = links[p - p0];
+            to.clear();
             for (int q = 0; q < 6; ++q) {
-                const int pn = H.page_at(o.x + d[q][0] * kPX, o.y + d[q][1] * kPY, o.z + d[q][2] * kPZ);
-                nbp[(size_t)p * 6 + q] = pn;
-                bool linked = false;
-                for (int c = 0; pn >= 0 && c < kPageCells && !linked; ++c) {
+                const int pn = nbp[(size_t)p * 6 + q];
+                if (pn < 0) continue;
+                for (int c = 0; c < kPageCells; ++c) {
+                    const uint32_t f = H.flags[(size_t)p * kPageCells + c];
+                    if (!(f & kActive) || !(f & (kFaceMX << q))) continue;
                     bool out;
-                    if ((fl[c] & kActive) && (fl[c] & (kFaceMX << q))) {
-                        const int nc = step(c, q, out);
-                        linked = out && (H.flags[(size_t)pn * kPageCells + nc] & kActive);
-                    }
+                    const int m = step(c, q, out);
+                    if (!out || !(H.flags[(size_t)pn * kPageCells + m] & kActive)) continue;
+                    const std::pair<int, int> l = {first[p] + piece[(size_t)p * kPageCells + c], first[pn] + piece[(size_t)pn * kPageCells + m]};
+                    if (to.empty() || to.back() != l) to.push_back(l);
                 }
-                link[(size_t)(p - p0) * 6 + q] = linked;
             }
         }
         for (int p = p0; p < p1; ++p)
-            for (int q = 0; q < 6; ++q) {
-                if (!link[(size_t)(p - p0) * 6 + q]) continue;
-                const int a = find(p), b = find(nbp[(size_t)p * 6 + q]);
-                if (a == b) continue;
-                parent[b] = a;
-                if ((size[a] += size[b]) > kMaxSlots) return false;
+            for (auto& l : links[p - p0]) {
+                const int x = find(l.first), y = find(l.second);
+                if (x == y) continue;
+                parent[y] = x;
+                if ((size[x] += size[y]) > kMaxCells) return false;
             }
     }
-    std::vector<std::vector<int>> members(np);
-    for (int p = 0; p < np; ++p) members[find(p)].push_back(p);  // ascending pages per cluster
-    size_t largest = 0, count = 0;
-    for (auto& m : members) { largest = std::max(largest, m.size()); count += !m.empty(); }
-    int slots = 1;
-    while (slots < (int)largest) slots *= 2;
-    std::vector<int> wg_page, slot(np, -1), wg_of(np, -1);
-    int used = slots;
-    for (int p = 0; p < np; ++p) {
-        const std::vector<int>& m = members[find(p)];
-        if (m.front() != p) continue;  // clusters in the order of their first page (Morton order keeps them local)
-        if (used + (int)m.size() > slots || count <= (size_t)kSpread) { wg_page.insert(wg_page.end(), slots, -1); used = 0; }
-        for (int q : m) {
-            slot[q] = used;
-            wg_of[q] = (int)wg_page.size() / slots - 1;
-            wg_page[wg_page.size() - slots + used] = q;
-            ++used;
-        }
+    // clusters in the order of their first cell (Morton order of the pages keeps them local), each with its cells ascending
+    std::vector<int> cluster(pieces, -1), count;
+    for (int k = 0; k < pieces; ++k) {
+        const int root = find(k);
+        if (cluster[root] < 0) { cluster[root] = (int)count.size(); count.push_back(size[root]); }
+        cluster[k] = cluster[root];
     }
-    const int nwg = (int)wg_page.size() / slots, cells = slots * kPageCells;
-    std::vector<uint16_t> nbr((size_t)nwg * 6 * cells);
+    int largest = 0;
+    for (int n : count) largest = std::max(largest, n);
+    const int per = largest <= 1024 ? 1 : largest <= 2048 ? 2 : largest <= 4096 ? 4 : 8;  // cells per thread
+    const int threads = std::max(1, ((largest + per - 1) / per + 63) / 64) * 64, slots = threads * per;
+    std::vector<int> base(count.size());  // first slot of each cluster, over all workgroups
+    int nwg = count.empty() ? 1 : 0, used = slots;
+    for (size_t k = 0; k < count.size(); ++k) {
+        if (used + count[k] > slots || count.size() <= (size_t)kSpread) { ++nwg; used = 0; }
+        base[k] = (nwg - 1) * slots + used;
+        used += count[k];
+    }
+    if ((long long)nwg * slots * 6 > (1LL << 30)) return false;
+    // a cluster's cells in x, y, z order: the neighbours of consecutive lanes are consecutive LDS values
+    std::vector<int> cell((size_t)nwg * slots, -1), at((size_t)np * kPageCells, -1), fill = base;
+    for (int p = 0; p < np; ++p)
+        for (int c = 0; c < kPageCells; ++c)
+            if (H.flags[(size_t)p * kPageCells + c] & kActive) cell[fill[cluster[first[p] + piece[(size_t)p * kPageCells + c]]]++] = p * kPageCells + c;
+#pragma omp parallel for schedule(dynamic, 8)
+    for (size_t k = 0; k < count.size(); ++k) {
+        auto key = [&](int e) {
+            const Int3 o = H.page_base[e >> 8];
+            return ((uint64_t)(uint32_t)(o.x + ((e >> 6) & 3)) << 42) + ((uint64_t)(uint32_t)(o.y + ((e >> 3) & 7)) << 21) + (uint32_t)(o.z + (e & 7));
+        };
+        std::sort(cell.begin() + base[k], cell.begin() + base[k] + count[k], [&](int e, int f) { return key(e) < key(f); });
+        for (int i = base[k]; i < base[k] + count[k]; ++i) at[cell[i]] = i;
+    }
+    std::vector<uint16_t> nbr((size_t)nwg * 6 * slots);
     std::vector<std::vector<int>> halo(nwg);
     std::vector<char> wide(nwg, 0);
 #pragma omp parallel for schedule(static)
     for (int w = 0; w < nwg; ++w) {
         std::map<int, int> seen;  // cell outside the workgroup -> its halo value
-        for (int s = 0; s < slots; ++s) {
-            const int p = wg_page[(size_t)w * slots + s];
-            for (int c = 0; c < kPageCells; ++c) {
-                const int ci = s * kPageCells + c;
-                const uint32_t f = p < 0 ? 0u : H.flags[(size_t)p * kPageCells + c];
-                for (int q = 0; q < 6; ++q) {
-                    int v = ci;
-                    if ((f & kActive) && (f & (kFaceMX << q))) {
-                        bool out;
-                        const int nc = step(c, q, out), pn = out ? nbp[(size_t)p * 6 + q] : p;
-                        if (pn >= 0 && wg_of[pn] == w) {
-                            v = slot[pn] * kPageCells + nc;
-                        } else {
-                            const int cell = zero_outside || pn < 0 ? np * kPageCells : pn * kPageCells + nc;
-                            const auto at = seen.emplace(cell, (int)seen.size());
-                            if (at.second) halo[w].push_back(cell);
-                            v = cells + at.first->second;
-                        }
+        for (int i = 0; i < slots; ++i) {
+            const int e = cell[(size_t)w * slots + i], p = e >> 8;
+            for (int q = 0; q < 6; ++q) {
+                int v = i;
+                if (e >= 0 && (H.flags[e] & (kFaceMX << q))) {
+                    bool out;
+                    const int nc = step(e & 255, q, out), pn = out ? nbp[(size_t)p * 6 + q] : p;
+                    const int n = pn >= 0 ? pn * kPageCells + nc : np * kPageCells;
+                    if (pn >= 0 && at[n] >= 0 && at[n] / slots == w) {
+                        v = at[n] - w * slots;
+                    } else {
+                        const auto h = seen.emplace(zero_outside ? np * kPageCells : n, (int)seen.size());
+                        if (h.second) halo[w].push_back(h.first->first);
+                        v = slots + h.first->second;
                     }
-                    wide[w] = wide[w] || v > 0xffff;
-                    nbr[((size_t)w * 6 + q) * cells + ci] = (uint16_t)v;
                 }
+                wide[w] = wide[w] || v > 0xffff;
+                nbr[((size_t)w * 6 + q) * slots + i] = (uint16_t)v;
             }
         }
     }
@@ -386,11 +427,13 @@ static bool plan_clusters(LevelBuffers& LB, bool zero_outside) {
         halo_cell.insert(halo_cell.end(), halo[w].begin(), halo[w].end());
         halo_ptr.push_back((int)halo_cell.size());
     }
-    if (2 * sizeof(float) * (size_t)(cells + most) > (size_t)kLdsBytes) return false;
+    if (2 * sizeof(float) * (size_t)(slots + most) > (size_t)kLdsBytes) return false;
     LB.cl_slots = slots;
-    LB.cl_entries = (cells + most + 3) / 4 * 4;
+    LB.cl_threads = threads;
+    LB.cl_entries = (slots + most + 3) / 4 * 4;
+    LB.cl_rest = !zero_outside;
     halo_cell.push_back(np * kPageCells);  // never empty
-    LB.cl_page.upload(wg_page); LB.cl_nbr.upload(nbr);
+    LB.cl_cell.upload(cell); LB.cl_nbr.upload(nbr);
     LB.cl_halo_ptr.upload(halo_ptr); LB.cl_halo_cell.upload(halo_cell);
     return true;
 }

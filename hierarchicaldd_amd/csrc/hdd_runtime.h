@@ -100,9 +100,10 @@ struct LevelBuffers {
     DBuf<float> u[2], b, r;
     DBuf<__half> hu[2], hb, hr;     // FP16-storage variant of u, b, r (allocated when it is selected)
     int cur = 0;  // which u buffer holds the current iterate
-    // clusters of pages that its sweeps couple (empty: one launch per sweep)
-    int cl_slots = 0, cl_entries = 0;
-    DBuf<int> cl_page, cl_halo_ptr, cl_halo_cell;
+    // clusters of Active cells that its sweeps couple (empty: one launch per sweep)
+    int cl_slots = 0, cl_threads = 0, cl_entries = 0;
+    bool cl_rest = false;
+    DBuf<int> cl_cell, cl_halo_ptr, cl_halo_cell;
     DBuf<uint16_t> cl_nbr;
     DevClusters clusters() const;
     DevLevel view() const;

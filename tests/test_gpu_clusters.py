@@ -1,8 +1,9 @@
-"""Sweeps of whole page clusters in one launch (every V-cycle level whose clusters of coupled pages
-fit a workgroup) against one launch per sweep (HDD_BOTTOM_LOCAL=0): the same operations in the same
-order, so the bar is equal bits. The cases have clusters of one page up to 32 (one to eight cells per
-thread), a level 0 whose cluster edges read interface cells, a single-level V-cycle (200 sweeps of
-level 0 around nonzero interface values), and levels on both sides of the size limit."""
+"""Sweeps of whole clusters in one launch (every V-cycle level whose clusters of coupled cells fit a
+workgroup) against one launch per sweep (HDD_BOTTOM_LOCAL=0): the same operations in the same order,
+so the bar is equal bits. The cases have clusters from a few cells (one wavefront, neighbours in
+registers) to several per thread, one cluster per workgroup and packed ones, a level 0 whose cluster
+edges read interface cells, a single-level V-cycle (200 sweeps of level 0 around nonzero interface
+values), and levels on both sides of the size limit."""
 import os
 
 import numpy as np
@@ -23,8 +24,9 @@ def _blocked(n, sub, vlevels, seed, nV=1):
 
 CASES = {
     "box45_sub16": lambda: domain.small_box(45, 16, 3, seed=4),        # level 0 in clusters, odd edge
-    "blocked100_sub16": lambda: _blocked(100, 16, 3, 7),               # clusters of up to 13 pages at level 1
-    "blocked100_sub32": lambda: _blocked(100, 32, 4, 0),               # bottom clusters of up to 6 pages, level 0 too large
+    "blocked100_sub16": lambda: _blocked(100, 16, 3, 7),               # clusters that lie in up to 13 pages at level 1
+    "blocked100_sub32": lambda: _blocked(100, 32, 4, 0),               # level 0 too large, level 1 across page boundaries
+    "box136_sub16": lambda: domain.small_box(136, 16, 3, seed=9),      # more clusters than run side by side: packed
     "box33_one_level": lambda: domain.small_box(33, 16, 1, seed=6),    # the bottom is level 0
     "box40_two_cycles": lambda: _blocked(40, 16, 2, 11, nV=2),         # V-cycles that start from a nonzero iterate
 }
