@@ -245,7 +245,7 @@ void push_items(std::vector<NodeItem>& out, NodeItem it, int rows, int len, int 
     constexpr int kWaveTiles = 16, kWorkTiles = 24, kGroups = 1024, kMaxRows = 16;
     int split = waves == 16 ? 16 : 1;
     while (split < waves && (len > kWaveTiles * split || (len > 4 * split && level_rows * split < 2048))) split *= 2;
-    it.split = (short)split;
+    it.split = split;
     const long long step = waves / split, by_work = (long long)kWorkTiles * waves / std::max(1, len);
     const long long want = std::max(1LL, std::min({by_work, level_rows / kGroups, (long long)kMaxRows}));
     const int chunk = (int)((want + step - 1) / step * step);
@@ -368,26 +368,36 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
         if (B.nrk) B.bwd += (int)(t / 2);
         P.tiles += t;
     }
-    // instances: every node of every member, its padded columns and boundary rows
-    struct Inst { int y, c, prob, block; };
+    // instances: every node of every member, its padded columns and boundary rows. A level's rows are
+    // contiguous, largest blocks first, and the nodes that share a block follow each other.
+    struct Inst { int y, c, prob, block, m, k; };
     std::vector<std::vector<Inst>> at_level(NL);
     std::vector<std::vector<int>> ybase(F.size()), cbase(F.size());
-    for (size_t m = 0; m < F.size(); ++m) { ybase[m].resize(nodes[which[m]].v.size()); cbase[m].resize(nodes[which[m]].v.size()); }
+    for (size_t m = 0; m < F.size(); ++m) {
+        const size_t n = nodes[which[m]].v.size();
+        ybase[m].resize(n); cbase[m].resize(n);
+        for (size_t k = 0; k < n; ++k) {
+            const Node& nd = nodes[which[m]].v[k];
+            at_level[nd.level].push_back({0, 0, prob_of.empty() ? 0 : prob_of[m], nd.block, (int)m, (int)k});
+        }
+    }
     P.levels.resize(NL);
     long long ny = 0, nc = 0;
-    for (int l = 0; l < NL; ++l) {  // a level's rows are contiguous
+    for (int l = 0; l < NL; ++l) {
         P_::Level& L = P.levels[l];
+        std::stable_sort(at_level[l].begin(), at_level[l].end(), [&](const Inst& a, const Inst& b) {
+            if (a.block == b.block) return false;
+            const P_::Block &x = P.blocks[a.block], &y = P.blocks[b.block];
+            const long long s = block_tiles(x.nk, x.nrk), t = block_tiles(y.nk, y.nrk);
+            return s != t ? s > t : a.block < b.block;
+        });
         L.y0 = (int)ny; L.c0 = (int)nc;
-        for (size_t m = 0; m < F.size(); ++m)
-            for (size_t k = 0; k < nodes[which[m]].v.size(); ++k) {
-                const Node& nd = nodes[which[m]].v[k];
-                if (nd.level != l) continue;
-                ybase[m][k] = (int)ny; cbase[m][k] = (int)nc;
-                const P_::Block& B = P.blocks[nd.block];
-                ny += T * B.nk; nc += T * B.nrk;
-                if (ny > INT_MAX - 64 || nc > INT_MAX - 64) return false;
-                at_level[l].push_back({ybase[m][k], cbase[m][k], prob_of.empty() ? 0 : prob_of[m], nd.block});
-            }
+        for (Inst& i : at_level[l]) {
+            const P_::Block& B = P.blocks[i.block];
+            ybase[i.m][i.k] = i.y = (int)ny; cbase[i.m][i.k] = i.c = (int)nc;
+            ny += T * B.nk; nc += T * B.nrk;
+            if (ny > INT_MAX - 64 || nc > INT_MAX - 64) return false;
+        }
         L.y1 = (int)ny; L.c1 = (int)nc;
     }
     P.ysize = (int)ny; P.csize = (int)nc;
@@ -427,18 +437,13 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
             }
         }
     }
-    // per level: runs of instances that share a block, largest blocks first, and their work items
+    // per level: runs of instances that share a block, and their work items
     for (int l = 0; l < NL; ++l) {
         P_::Level& L = P.levels[l];
         L.children = l > 0;
-        auto& v = at_level[l];
-        std::stable_sort(v.begin(), v.end(), [&](const Inst& a, const Inst& b) {
-            if (a.block == b.block) return false;
-            const P_::Block &x = P.blocks[a.block], &y = P.blocks[b.block];
-            const long long s = block_tiles(x.nk, x.nrk), t = block_tiles(y.nk, y.nrk);
-            return s != t ? s > t : a.block < b.block;
-        });
-        struct Run { int i0, cnt, block; };
+        const auto& v = at_level[l];
+        struct Run { int i0, cnt, block, y, c; };
+        std::vector<int> longest(P.blocks.size(), 0);  // run of each block
         std::vector<Run> runs;
         long long frows = 0, brows = 0, ftiles = 0, btiles = 0;
         for (size_t i = 0; i < v.size();) {
@@ -446,8 +451,9 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
             const int lim = run_limit(T * (B.nk + B.nrk));
             int k = 1;
             while (k < lim && i + k < v.size() && v[i + k].block == v[i].block) ++k;
-            runs.push_back({(int)(P.inst_y.size()), k, v[i].block});
-            for (int j = 0; j < k; ++j) { P.inst_y.push_back(v[i + j].y); P.inst_c.push_back(v[i + j].c); P.inst_prob.push_back(v[i + j].prob); }
+            longest[v[i].block] = std::max(longest[v[i].block], k);
+            runs.push_back({(int)P.inst_prob.size(), k, v[i].block, v[i].y, v[i].c});
+            for (int j = 0; j < k; ++j) P.inst_prob.push_back(v[i + j].prob);
             frows += B.nk + B.nrk;
             ftiles += pass_tiles(B.nk, B.nrk);
             L.fwd_lds = std::max(L.fwd_lds, k * (T * B.nk + 4));
@@ -463,7 +469,7 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
         L.fwd0 = (int)P.fwd.size(); L.bwd0 = (int)P.bwd.size();
         for (const Run& r : runs) {
             const P_::Block& B = P.blocks[r.block];
-            NodeItem it = {B.fwd, r.i0, (short)r.cnt, 1, B.nk, B.nrk, 0, 0, B.scale};
+            NodeItem it = {B.fwd, r.i0, r.y, r.c, r.cnt, 1, B.nk, B.nrk, 0, 0, longest[r.block] == 1, B.scale};
             push_items(P.fwd, it, B.nk + B.nrk, B.nk, L.fwd_waves, frows);
             if (!B.nrk) continue;
             it.tile = B.bwd;

@@ -32,12 +32,14 @@
 namespace hdd {
 
 // One workgroup's work: row tiles [rt0, rt1) of a run of `cnt` nodes that share a block.
-struct NodeItem {
+struct alignas(16) NodeItem {
     int tile;            // first tile of the block's operator for this pass (forward of a closed block: its inverse)
     int inst0;           // the run: instances [inst0, inst0 + cnt)
-    short cnt, split;    // split: waves that share a row tile
+    int y0, c0;          // first column and boundary row of the first; the others follow, nk and nrk tiles each
+    int cnt, split;      // split: waves that share a row tile
     int nk, nrk;         // column and boundary tiles of the block
     int rt0, rt1;
+    int one;             // the block has runs of one node only: vector sums instead of matrix products
     int scale;           // first of the block's D^-2 (closed: of its inverse's diagonal)
 };
 
@@ -71,7 +73,7 @@ struct NodePlanHost {
     std::vector<Block> blocks;
     std::vector<Level> levels;
     std::vector<NodeItem> fwd, bwd;
-    std::vector<int> inst_y, inst_c, inst_prob;  // per instance: first column, first boundary row, problem
+    std::vector<int> inst_prob;   // problem of each instance
     std::vector<int> orig;        // padded column -> row of the batch (-1: padding)
     std::vector<int> zidx;        // padded boundary row -> padded column (ysize: the zero slot)
     std::vector<NodePos> pos_y, pos_c;  // child contributions of each padded column and boundary row

@@ -10,7 +10,7 @@ struct NodePlan {
     int n = 0;
     std::vector<NodePlanHost::Level> levels;
     DBuf<NodeItem> fwd, bwd;
-    DBuf<int> inst_y, inst_c, inst_prob, orig, zidx, more;
+    DBuf<int> inst_prob, orig, zidx, more;
     DBuf<NodePos> pos_y, pos_c;
     DBuf<float> tiles, scale;  // the blocks' operators, 256 floats per tile, and their D^-2
     DBuf<float> t, y, z, c;    // padded columns (b less the children's sums, D^-2 y, the result), boundary rows; a zero slot follows z and c

@@ -7,9 +7,17 @@
 // operand of four v_mfma_f32_16x16x4_f32 (instruction s takes the columns
 // 4q + s of the lanes' groups q; A and B agree on that order, so it only
 // permutes the summands). The B operand is the run's vectors, one node per
-// column, in LDS: a run of one node uses one column of the sixteen, which the
-// matrix unit can afford (it consumes tiles at about 20 TB/s over the chip, HBM
-// delivers 8). Forward tiles of a block: row tile rt < nk (Linv) has rt + 1 of
+// column, in LDS. Blocks of a single node, most of them above the first level,
+// would fill one of the sixteen columns: they take the same tiles through vector
+// FMAs (16 instead of 128 cycles a tile) and add across the lanes at the end of
+// a row (96^3 interfaces: 72.8 -> 67.5 us a solve; with such sums for runs of two
+// to four as well the registers cost more than the matrix unit's idle columns).
+// The rest of a launch is latency, so a kernel is kept short: the wave's number
+// and all loop control are scalars, a pass's first loads go out before its first
+// tiles and everything a row tile needs at its end beside them, and no load
+// waits at the end of a branch (67.5 -> 57.3 us).
+// (The matrix unit consumes tiles at about 20 TB/s over the chip, HBM
+// delivers 8.) Forward tiles of a block: row tile rt < nk (Linv) has rt + 1 of
 // them, row tile nk + a (W) has nk. Backward: row tile rt has nk - rt (Linv^T)
 // and nrk (-W^T). A closed block (nrk = 0): every row tile of its inverse has nk.
 #include <hip/hip_runtime.h>
@@ -40,7 +48,9 @@ __device__ __forceinline__ bool run_stopped(const int* __restrict__ active, cons
 // the sum itself at its boundary rows (in c, where the forward product adds to it).
 // On its own because a node's row tiles go to several workgroups, which all need every t of the node:
 // with the sums inside the forward kernel, its gather was 3 times its product on the 256^3 level-0
-// interiors (171 us against 49 us for the backward pass of the same level).
+// interiors (171 us against 49 us for the backward pass of the same level); and where the gather is
+// small beside the tiles (a tenth of their bytes), no faster: 96^3 level-0 interface 74.6 us with,
+// 71.8 us without it.
 __global__ void __launch_bounds__(256) k_node_children(int y0, int y1, int c0, int c1, const NodePos* __restrict__ pos_y,
                                                        const NodePos* __restrict__ pos_c, const int* __restrict__ more,
                                                        const int* __restrict__ orig, const float* __restrict__ b,
@@ -67,7 +77,7 @@ __global__ void __launch_bounds__(256) k_node_children(int y0, int y1, int c0, i
     else c[c0 + i - ny] = s;
 }
 
-// D (16 rows x 16 nodes) of one row tile: tiles [0, nt) at A against the operand vectors from tp on,
+// D (16 rows x 16 nodes, or x 1 with ONE, in the matrix unit's layout) of one row tile: tiles [0, nt) at A against the operand vectors from tp on,
 // every KS-th tile from kw. The tiles are loaded kAhead at a time, a group ahead of the products
 // (`a` holds the first group on entry); four independent sums (one per tile column mod 4) keep the
 // chains short.
@@ -78,8 +88,25 @@ __device__ __forceinline__ void load_group(const f32x4* __restrict__ A, int k, i
     for (int u = 0; u < kAhead; ++u)
         if (k + u * KS < nt) a[u] = A[(size_t)(k + u * KS) * 64];
 }
-template <int KS>
+template <int KS, bool ONE>
 __device__ __forceinline__ f32x4 row_tile(const f32x4* __restrict__ A, const f32x4* tp, int nt, int kw, f32x4 (&a)[kAhead]) {
+    if (ONE) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        for (int k = kw; k < nt; k += kAhead * KS) {
+            f32x4 nx[kAhead];
+            load_group<KS>(A, k + kAhead * KS, nt, nx);
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u)
+                if (k + u * KS < nt) s = __builtin_elementwise_fma(a[u], tp[(k + u * KS) * 4], s);
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) a[u] = nx[u];
+        }
+        float v = (s[0] + s[1]) + (s[2] + s[3]);  // the lane's columns of its row; then all columns
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+        const int r = (threadIdx.x & 48) >> 2;  // rows 4q .. 4q + 3, as the matrix unit leaves them
+        return f32x4{__shfl(v, r), __shfl(v, r + 1), __shfl(v, r + 2), __shfl(v, r + 3)};
+    }
     f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0, s2 = s0, s3 = s0;
     for (int k = kw; k < nt; k += kAhead * KS) {
         f32x4 nx[kAhead];
@@ -112,47 +139,98 @@ __device__ __forceinline__ f32x4 join(f32x4 d, f32x4 (*red)[64], int w, int lane
     return d;
 }
 
-// The row tiles [rt0, rt1) of a workgroup of NW waves, KS of them per row tile: gather() fills the
-// operand vectors in LDS (while the first tiles load), where(rt, &A, &tp, &nt) gives a row tile's
-// tiles and operand, out(rt, d) takes its 16x16 result from the lanes that hold it.
-template <int NW, int KS, class Where, class Gather, class Out>
-__device__ __forceinline__ void row_tiles(int rt0, int rt1, f32x4 (*red)[64], Where where, Gather gather, Out out) {
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// The row tiles [rt0, rt1) of a workgroup of NW waves, KS of them per row tile: gather fills the
+// operand vectors in LDS, its first loads ahead of the first tiles (a wait for a load is a wait for all
+// before it), the dependent ones beside them; where(rt, &A, &tp, &nt) gives a row tile's
+// tiles and operand, ahead(rt) loads beside the first tiles what out(rt, d, it) needs for the 16x16 result in
+// the lanes that hold it.
+struct Ahead { f32x4 v; int4 o; };
+template <int NW, int KS, bool ONE, class Where, class Gather, class Load, class Out>
+__device__ __forceinline__ void row_tiles(int rt0, int rt1, f32x4 (*red)[64], Where where, Gather gather, Load ahead, Out out) {
+    // the wave's number as a scalar: its row tiles and their loops stay on the scalar unit
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     constexpr int step = NW / KS;
-    int rt = rt0 + w / KS, nt = 0;
-    const f32x4* A = nullptr;
-    const f32x4* tp = nullptr;
+    int rt = rt0 + w / KS, nt;
+    const f32x4 *A, *tp;
     f32x4 a[kAhead];
-    if (rt < rt1) {
-        where(rt, A, tp, nt);
+    const f32x4 g = gather.first();
+    {   // (a wave without a row tile loads the last one: no wait at a branch's end)
+        const int rf = min(rt, rt1 - 1);
+        where(rf, A, tp, nt);
         load_group<KS>(A, w % KS, nt, a);
     }
-    gather();
+    Ahead add = ahead(min(rt, rt1 - 1));
+    if (!gather.fill(g)) return;
     __syncthreads();
     for (int r0 = rt0; r0 < rt1; r0 += step) {
         const bool live = rt < rt1;
         f32x4 d = {0.f, 0.f, 0.f, 0.f};
-        if (live) d = row_tile<KS>(A, tp, nt, w % KS, a);
+        if (live) d = row_tile<KS, ONE>(A, tp, nt, w % KS, a);
         const int rc = rt;
+        const Ahead ac = add;
         rt += step;
         if (rt < rt1) {  // the next row tile's first tiles load beside this one's results
             where(rt, A, tp, nt);
             load_group<KS>(A, w % KS, nt, a);
+            add = ahead(rt);
         }
         d = join<KS>(d, red, w, lane);
-        if (live && w % KS == 0) out(rc, d);
+        if (live && w % KS == 0) out(rc, d, ac);
     }
 }
-template <int NW, class Where, class Gather, class Out>
-__device__ __forceinline__ void row_tiles(int split, int rt0, int rt1, f32x4 (*red)[64], Where where, Gather gather, Out out) {
-    if (NW == 16) return row_tiles<NW, 16>(rt0, rt1, red, where, gather, out);
-    if (split == 1) return row_tiles<NW, 1>(rt0, rt1, red, where, gather, out);
-    if (split == 2) return row_tiles<NW, 2>(rt0, rt1, red, where, gather, out);
-    row_tiles<NW, 4>(rt0, rt1, red, where, gather, out);
+template <int NW, bool ONE, class Where, class Gather, class Load, class Out>
+__device__ __forceinline__ void row_tiles(int split, int rt0, int rt1, f32x4 (*red)[64], Where where, Gather gather, Load ahead, Out out) {
+    if (NW == 16) return row_tiles<NW, 16, ONE>(rt0, rt1, red, where, gather, ahead, out);
+    if (split == 1) return row_tiles<NW, 1, ONE>(rt0, rt1, red, where, gather, ahead, out);
+    if (split == 2) return row_tiles<NW, 2, ONE>(rt0, rt1, red, where, gather, ahead, out);
+    row_tiles<NW, 4, ONE>(rt0, rt1, red, where, gather, ahead, out);
 }
 
-__device__ __forceinline__ void store_rows(const int* __restrict__ orig, int i, f32x4 d, float* __restrict__ x) {
-    const int4 o = *reinterpret_cast<const int4*>(orig + i);
+template <int NW, class Where, class Gather, class Load, class Out>
+__device__ __forceinline__ void run_tiles(const NodeItem& it, f32x4 (*red)[64], Where where, Gather gather, Load ahead, Out out) {
+    if (it.one) return row_tiles<NW, true>(it.split, it.rt0, it.rt1, red, where, gather, ahead, out);
+    row_tiles<NW, false>(it.split, it.rt0, it.rt1, red, where, gather, ahead, out);
+}
+
+// 16 bytes, of floats or of indices (through HIP's int4 instead, the compiler put the LDS address of the
+// operand's store into one of its data registers)
+__device__ __forceinline__ f32x4 load4(const void* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+// Operand vectors of a run, `rows` of each node: four rows from load(i, j, k) (row k of node j, i in all),
+// whose values (a vector, or where to find it) go through value(v, k) to LDS. fill() is false for a run
+// of stopped problems.
+template <int NW, class Load, class Value>
+struct Operands {
+    const NodeItem& it;
+    int rows;
+    const int *active, *prob;
+    f32x4* lds;
+    Load load;
+    Value value;
+    __device__ __forceinline__ f32x4 at(int idx) const {
+        const int j = it.cnt == 1 ? 0 : idx / (rows / 4);
+        return load(4 * idx, j, 4 * idx - j * rows);
+    }
+    __device__ __forceinline__ f32x4 first() const { return at(min((int)threadIdx.x, it.cnt * rows / 4 - 1)); }
+    __device__ __forceinline__ bool fill(f32x4 v) const {
+        if (run_stopped(active, prob, it.inst0, it.cnt)) return false;
+        const int n = it.cnt * rows / 4;
+        for (int idx = threadIdx.x; idx < n;) {
+            const int j = it.cnt == 1 ? 0 : idx / (rows / 4);
+            lds[idx + j] = value(v, 4 * idx - j * rows);
+            idx += NW * 64;
+            if (idx < n) v = at(idx);
+        }
+        return true;
+    }
+};
+template <int NW, class Load, class Value>
+__device__ __forceinline__ Operands<NW, Load, Value> operands(const NodeItem& it, int rows, const int* active, const int* prob, f32x4* lds,
+                                                              Load load, Value value) {
+    return {it, rows, active, prob, lds, load, value};
+}
+
+__device__ __forceinline__ void store_rows(int4 o, f32x4 d, float* __restrict__ x) {
     if (o.x >= 0) x[o.x] = d[0];
     if (o.y >= 0) x[o.y] = d[1];
     if (o.z >= 0) x[o.z] = d[2];
@@ -163,8 +241,7 @@ __device__ __forceinline__ void store_rows(const int* __restrict__ orig, int i, 
 // result (the inverse's diagonal apart as well: its row's largest term is added once, after the others).
 // NW waves per workgroup; INC: the nodes have children (t and the boundary rows' sums from k_node_children).
 template <int NW, bool INC>
-__global__ void __launch_bounds__(NW * 64) k_node_fwd(const NodeItem* __restrict__ items, const int* __restrict__ inst_y,
-                                                      const int* __restrict__ inst_c, const int* __restrict__ inst_prob,
+__global__ void __launch_bounds__(NW * 64) k_node_fwd(const NodeItem* __restrict__ items, const int* __restrict__ inst_prob,
                                                       const int* __restrict__ active, const int* __restrict__ orig,
                                                       const float* __restrict__ t, const float* __restrict__ tiles,
                                                       const float* __restrict__ scale, const float* __restrict__ b,
@@ -173,10 +250,9 @@ __global__ void __launch_bounds__(NW * 64) k_node_fwd(const NodeItem* __restrict
     extern __shared__ f32x4 lds[];
     __shared__ f32x4 red[NW][64];
     const NodeItem it = items[blockIdx.x];
-    if (run_stopped(active, inst_prob, it.inst0, it.cnt)) return;
     const int lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
     const int np = it.nk * T, ld = np + 4, my_col = min(col, it.cnt - 1);
-    const int yb = inst_y[it.inst0 + my_col], cb = inst_c[it.inst0 + my_col];
+    const int yb = it.y0 + my_col * np, cb = it.c0 + my_col * it.nrk * T;
     const f32x4* base = reinterpret_cast<const f32x4*>(tiles) + (size_t)it.tile * 64 + lane;
     const f32x4* tcol = lds + (my_col * ld) / 4 + q;
     auto where = [&](int rt, const f32x4*& A, const f32x4*& tp, int& nt) {
@@ -184,56 +260,58 @@ __global__ void __launch_bounds__(NW * 64) k_node_fwd(const NodeItem* __restrict
         tp = tcol;
         nt = it.nrk && rt < it.nk ? rt + 1 : it.nk;
     };
-    auto gather = [&]() {
-        for (int idx = threadIdx.x; idx < it.cnt * np / 4; idx += NW * 64) {
-            const int j = idx / (np / 4), k = idx - j * (np / 4);
-            const int i = inst_y[it.inst0 + j] + 4 * k;
-            f32x4 v;
-            if (INC) {
-                v = *reinterpret_cast<const f32x4*>(t + i);
-            } else {
-                const int4 o = *reinterpret_cast<const int4*>(orig + i);
-                v[0] = o.x >= 0 ? b[o.x] : 0.f; v[1] = o.y >= 0 ? b[o.y] : 0.f;
-                v[2] = o.z >= 0 ? b[o.z] : 0.f; v[3] = o.w >= 0 ? b[o.w] : 0.f;
+    auto gather = operands<NW>(
+        it, np, active, inst_prob, lds,
+        [&](int i, int, int) { return INC ? load4(t + it.y0 + i) : load4(orig + it.y0 + i); },
+        [&](f32x4 v, int) {
+            if (INC) return v;
+            f32x4 r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int o = __float_as_int(v[e]);
+                r[e] = o >= 0 ? b[o] : 0.f;
             }
-            lds[(j * ld) / 4 + k] = v;
-        }
+            return r;
+        });
+    auto ahead = [&](int rt) {  // the row tile's D^-2 or inverse diagonal, or its children's sums; rows of x
+        // (lanes beyond the run load the last node's, so that no load waits behind a branch)
+        Ahead h;
+        const int r = INC && rt >= it.nk ? cb + (rt - it.nk) * T : it.scale + min(rt, it.nk - 1) * T;
+        h.v = *reinterpret_cast<const f32x4*>((INC && rt >= it.nk ? c : scale) + r + 4 * q);
+        h.o = *reinterpret_cast<const int4*>(orig + yb + min(rt, it.nk - 1) * T + 4 * q);
+        return h;
     };
-    auto out = [&](int rt, f32x4 d) {
+    auto out = [&](int rt, f32x4 d, const Ahead& h) {
         if (col >= it.cnt) return;
         if (!it.nrk) {
-            d += tcol[rt * 4] * *reinterpret_cast<const f32x4*>(scale + it.scale + rt * T + 4 * q);
-            const int i = yb + rt * T + 4 * q;
-            *reinterpret_cast<f32x4*>(z + i) = d;
-            store_rows(orig, i, d, x);
+            d += tcol[rt * 4] * h.v;
+            *reinterpret_cast<f32x4*>(z + yb + rt * T + 4 * q) = d;
+            store_rows(h.o, d, x);
         } else if (rt < it.nk) {
             d += tcol[rt * 4];  // the unit diagonal
-            d *= *reinterpret_cast<const f32x4*>(scale + it.scale + rt * T + 4 * q);
+            d *= h.v;
             *reinterpret_cast<f32x4*>(y + yb + rt * T + 4 * q) = d;
         } else {
-            f32x4* ca = reinterpret_cast<f32x4*>(c + cb + (rt - it.nk) * T + 4 * q);
-            if (INC) d += *ca;
-            *ca = d;
+            if (INC) d += h.v;
+            *reinterpret_cast<f32x4*>(c + cb + (rt - it.nk) * T + 4 * q) = d;
         }
     };
-    row_tiles<NW>(it.split, it.rt0, it.rt1, red, where, gather, out);
+    run_tiles<NW>(it, red, where, gather, ahead, out);
 }
 
 // Backward pass of a level: [D^-2 y; z of the boundary rows] into LDS, then the row tiles of
 // [I + S^T | -W^T]; the result goes to z and, in the original numbering, to x.
 template <int NW>
-__global__ void __launch_bounds__(NW * 64) k_node_bwd(const NodeItem* __restrict__ items, const int* __restrict__ inst_y,
-                                                      const int* __restrict__ inst_c, const int* __restrict__ inst_prob,
+__global__ void __launch_bounds__(NW * 64) k_node_bwd(const NodeItem* __restrict__ items, const int* __restrict__ inst_prob,
                                                       const int* __restrict__ active, const int* __restrict__ orig,
                                                       const int* __restrict__ zidx, const float* __restrict__ tiles,
                                                       const float* __restrict__ y, float* __restrict__ z, float* __restrict__ x) {
     extern __shared__ f32x4 lds[];
     __shared__ f32x4 red[NW][64];
     const NodeItem it = items[blockIdx.x];
-    if (run_stopped(active, inst_prob, it.inst0, it.cnt)) return;
     const int lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
     const int np = it.nk * T, nz = np + it.nrk * T, ld = nz + 4, my_col = min(col, it.cnt - 1);
-    const int yb = inst_y[it.inst0 + my_col];
+    const int yb = it.y0 + my_col * np;
     const f32x4* base = reinterpret_cast<const f32x4*>(tiles) + (size_t)it.tile * 64 + lane;
     const f32x4* tcol = lds + (my_col * ld) / 4 + q;
     auto where = [&](int rt, const f32x4*& A, const f32x4*& tp, int& nt) {
@@ -241,27 +319,26 @@ __global__ void __launch_bounds__(NW * 64) k_node_bwd(const NodeItem* __restrict
         tp = tcol + rt * 4;
         nt = it.nk + it.nrk - rt;
     };
-    auto gather = [&]() {
-        for (int idx = threadIdx.x; idx < it.cnt * nz / 4; idx += NW * 64) {
-            const int j = idx / (nz / 4), k = 4 * (idx - j * (nz / 4));
-            f32x4 v;
-            if (k < np) {
-                v = *reinterpret_cast<const f32x4*>(y + inst_y[it.inst0 + j] + k);
-            } else {
-                const int4 o = *reinterpret_cast<const int4*>(zidx + inst_c[it.inst0 + j] + k - np);
-                v[0] = z[o.x]; v[1] = z[o.y]; v[2] = z[o.z]; v[3] = z[o.w];
+    auto gather = operands<NW>(
+        it, nz, active, inst_prob, lds,
+        [&](int, int j, int k) {
+            return load4(k < np ? reinterpret_cast<const int*>(y) + it.y0 + j * np + k : zidx + it.c0 + j * (nz - np) + k - np);
+        },
+        [&](f32x4 v, int k) {
+            if (k >= np) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = z[__float_as_int(v[e])];
             }
-            lds[(j * ld + k) / 4] = v;
-        }
-    };
-    auto out = [&](int rt, f32x4 d) {
+            return v;
+        });
+    auto ahead = [&](int rt) { return Ahead{{}, *reinterpret_cast<const int4*>(orig + yb + rt * T + 4 * q)}; };
+    auto out = [&](int rt, f32x4 d, const Ahead& h) {
         if (col >= it.cnt) return;
         d += tcol[rt * 4];
-        const int i = yb + rt * T + 4 * q;
-        *reinterpret_cast<f32x4*>(z + i) = d;
-        store_rows(orig, i, d, x);
+        *reinterpret_cast<f32x4*>(z + yb + rt * T + 4 * q) = d;
+        store_rows(h.o, d, x);
     };
-    row_tiles<NW>(it.split, it.rt0, it.rt1, red, where, gather, out);
+    run_tiles<NW>(it, red, where, gather, ahead, out);
 }
 
 // ---- set-up: the operators from the factor columns, in double -----------------------------------
@@ -443,7 +520,7 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
     n = P.n;
     levels = P.levels;
     fwd.upload(P.fwd); bwd.upload(P.bwd);
-    inst_y.upload(P.inst_y); inst_c.upload(P.inst_c); inst_prob.upload(P.inst_prob);
+    inst_prob.upload(P.inst_prob);
     orig.upload(P.orig);
     P.zidx.resize(std::max<size_t>(1, P.zidx.size()), P.ysize); zidx.upload(P.zidx);
     P.more.resize(std::max<size_t>(1, P.more.size()), 0); more.upload(P.more);
@@ -535,7 +612,7 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
 }
 
 size_t NodePlan::bytes() const {
-    return (fwd.n + bwd.n) * sizeof(NodeItem) + (inst_y.n + inst_c.n + inst_prob.n + orig.n + zidx.n + more.n) * 4 +
+    return (fwd.n + bwd.n) * sizeof(NodeItem) + (inst_prob.n + orig.n + zidx.n + more.n) * 4 +
            (pos_y.n + pos_c.n) * 8 + (tiles.n + scale.n + t.n + y.n + z.n + c.n) * 4;
 }
 
@@ -545,17 +622,17 @@ void NodePlan::solve(const float* b, float* x, const int* active, hipStream_t s)
             hipLaunchKernelGGL(k_node_children, dim3((unsigned)((L.y1 - L.y0 + L.c1 - L.c0 + 255) / 256)), dim3(256), 0, s, L.y0, L.y1, L.c0, L.c1,
                                (const NodePos*)pos_y.p, (const NodePos*)pos_c.p, (const int*)more.p, (const int*)orig.p, b, t.p, c.p);
         auto go = [&](auto kernel) {
-            launch(kernel, L.fwd1 - L.fwd0, L.fwd_waves, L.fwd_lds * sizeof(float), s, (const NodeItem*)fwd.p + L.fwd0, (const int*)inst_y.p,
-                   (const int*)inst_c.p, (const int*)inst_prob.p, active, (const int*)orig.p, (const float*)t.p, (const float*)tiles.p,
-                   (const float*)scale.p, b, y.p, c.p, z.p, x);
+            launch(kernel, L.fwd1 - L.fwd0, L.fwd_waves, L.fwd_lds * sizeof(float), s, (const NodeItem*)fwd.p + L.fwd0, (const int*)inst_prob.p,
+                   active, (const int*)orig.p, (const float*)t.p,
+                   (const float*)tiles.p, (const float*)scale.p, b, y.p, c.p, z.p, x);
         };
         if (L.fwd_waves == 4) { if (L.children) go(k_node_fwd<4, true>); else go(k_node_fwd<4, false>); }
         else { if (L.children) go(k_node_fwd<16, true>); else go(k_node_fwd<16, false>); }
     };
     auto bwd_level = [&](const NodePlanHost::Level& L) {
         auto go = [&](auto kernel) {
-            launch(kernel, L.bwd1 - L.bwd0, L.bwd_waves, L.bwd_lds * sizeof(float), s, (const NodeItem*)bwd.p + L.bwd0, (const int*)inst_y.p,
-                   (const int*)inst_c.p, (const int*)inst_prob.p, active, (const int*)orig.p, (const int*)zidx.p, (const float*)tiles.p,
+            launch(kernel, L.bwd1 - L.bwd0, L.bwd_waves, L.bwd_lds * sizeof(float), s, (const NodeItem*)bwd.p + L.bwd0, (const int*)inst_prob.p,
+                   active, (const int*)orig.p, (const int*)zidx.p, (const float*)tiles.p,
                    (const float*)y.p, z.p, x);
         };
         if (L.bwd_waves == 4) go(k_node_bwd<4>);

@@ -49,7 +49,7 @@ void box_matrix(int nx, int ny, int nz, int hole, unsigned seed, Csr& A, std::ve
 }
 
 void check_indices(const NodePlanHost& P) {
-    const int ni = (int)P.inst_y.size();
+    const int ni = (int)P.inst_prob.size();
     std::vector<int> fcount(P.ysize / T + 1, 0), ccount(P.csize / T + 1, 0), bcount(P.ysize / T + 1, 0);
     auto item = [&](const NodeItem& it, bool fwd, const NodePlanHost::Level& L) {
         const int waves = fwd ? L.fwd_waves : L.bwd_waves;
@@ -70,7 +70,7 @@ void check_indices(const NodePlanHost& P) {
             need(base >= 0 && base + nt <= P.tiles, "tiles");
         }
         for (int j = 0; j < it.cnt; ++j) {
-            const int y = P.inst_y[it.inst0 + j], c = P.inst_c[it.inst0 + j];
+            const int y = it.y0 + j * T * it.nk, c = it.c0 + j * T * it.nrk;
             need(y >= L.y0 && y % T == 0 && y + T * it.nk <= L.y1 && L.y1 <= P.ysize, "columns");
             need(c >= L.c0 && c % T == 0 && c + T * it.nrk <= L.c1 && L.c1 <= P.csize, "boundary rows");
             if (fwd && !it.nrk) for (int r = it.rt0; r < it.rt1; ++r) ++bcount[y / T + r];  // the whole solve
@@ -147,7 +147,7 @@ double emulate(const NodePlanHost& P, const std::vector<const SupernodalFactor*>
             const NodeItem& it = P.fwd[i];
             const int k = by_fwd.at(it.tile), np = T * it.nk;
             for (int j = 0; j < it.cnt; ++j) {
-                const int yb = P.inst_y[it.inst0 + j], cb = P.inst_c[it.inst0 + j];
+                const int yb = it.y0 + j * np, cb = it.c0 + j * T * it.nrk;
                 std::vector<double> t(np);
                 for (int q = 0; q < np; ++q) t[q] = L.children ? t0[yb + q] : (P.orig[yb + q] >= 0 ? b[P.orig[yb + q]] : 0.0);
                 for (int r = it.rt0 * T; r < it.rt1 * T; ++r) {
@@ -173,7 +173,7 @@ double emulate(const NodePlanHost& P, const std::vector<const SupernodalFactor*>
             const NodeItem& it = P.bwd[i];
             const int k = by_bwd.at(it.tile), np = T * it.nk, nr = T * it.nrk;
             for (int j = 0; j < it.cnt; ++j) {
-                const int yb = P.inst_y[it.inst0 + j], cb = P.inst_c[it.inst0 + j];
+                const int yb = it.y0 + j * np, cb = it.c0 + j * T * it.nrk;
                 for (int r = it.rt0 * T; r < it.rt1 * T; ++r) {
                     double a = 0;
                     for (int q = r + 1; q < np; ++q) a += S[k][(size_t)q * np + r] * y[yb + q];
@@ -221,7 +221,7 @@ extern "C" int nodeplan_check(int nx, int ny, int nz, int hole, int copies, int 
         need(P.n == n, "rows");
         check_indices(P);
         out[0] = emulate(P, F, off);
-        out[1] = (double)P.levels.size(); out[2] = (double)P.blocks.size(); out[3] = (double)P.inst_y.size();
+        out[1] = (double)P.levels.size(); out[2] = (double)P.blocks.size(); out[3] = (double)P.inst_prob.size();
         out[4] = 0;
         for (auto& B : P.blocks) out[4] = std::max(out[4], (double)B.n);
         return 0;
