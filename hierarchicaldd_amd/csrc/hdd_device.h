@@ -13,15 +13,18 @@ inline void hdd_check(hipError_t e, const char* what = "HIP call") {
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// One paged level on the device. flags has (np+1)*256 entries (zero page last),
+// One paged level on the device. flags has (np+1)*256 entries (zero page last), kinds the
+// bits of them that a sweep needs (bits 0-5 the face bits, kKindActive, kKindBoundary),
 // nbr np*6 face-neighbour pages (np = zero page), base np*3 cell origins,
 // lut the block lookup table over nbx*nby*nbz blocks (-1 = unallocated).
 // A stopped problem's pages keep stale values: no kernel reads them for another
 // problem (no stencil crosses problems), and the problem's result is final.
+enum : uint32_t { kKindFaces = 0x3fu, kKindActive = 0x40u, kKindBoundary = 0x80u };
 struct DevLevel {
     int np = 0;
     int nbx = 0, nby = 0, nbz = 0;
     const uint32_t* flags = nullptr;
+    const uint8_t* kinds = nullptr;
     const int* nbr = nullptr;
     const int* base = nullptr;
     const int* lut = nullptr;
@@ -33,8 +36,10 @@ struct DevLevel {
 
 void upload_constants();
 // V-cycle kernels, float storage and half (FP16) storage with float arithmetic
-void launch_smooth(const DevLevel& L, const float* u_in, float* u_out, const float* b, bool interior, bool boundary, hipStream_t s);
-void launch_smooth(const DevLevel& L, const __half* u_in, __half* u_out, const __half* b, bool interior, bool boundary, hipStream_t s);
+// again: u_out holds the iterate before u_in, which a sweep of the same cells made from it, so only those are written
+void launch_smooth(const DevLevel& L, const float* u_in, float* u_out, const float* b, bool interior, bool boundary, bool again, hipStream_t s);
+void launch_smooth(const DevLevel& L, const __half* u_in, __half* u_out, const __half* b, bool interior, bool boundary, bool again,
+                   hipStream_t s);
 // Sweeps of a level whose Active cells couple only within small clusters, several in one launch
 // (k_cluster_sweeps): workgroups of `slots` cells hold whole clusters in LDS.
 struct DevClusters {

@@ -103,13 +103,14 @@ __device__ __forceinline__ void st4(__half* __restrict__ p, size_t i4, const V4&
 template <class S>
 struct Stencil4 {
     V4 uc, r;
-    uint32_t f[4];
+    uint32_t f[4];  // DevLevel::kinds
     __device__ __forceinline__ Stencil4(const DevLevel& L, int p, int l, const S* __restrict__ u, const S* __restrict__ b) {
         const int x = l >> 4, y = (l >> 1) & 7, zh = l & 1;
         const int* nb = L.nbr + p * 6;
         const size_t base = (size_t)p * 64;
-        const uint4 fv = reinterpret_cast<const uint4*>(L.flags)[base + l];
-        f[0] = fv.x; f[1] = fv.y; f[2] = fv.z; f[3] = fv.w;
+        const uint32_t fv = reinterpret_cast<const uint32_t*>(L.kinds)[base + l];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f[k] = fv >> (8 * k) & 0xffu;
         uc = ld4(u, base + l);
         const V4 xm = ld4(u, x > 0 ? base + l - 16 : (size_t)nb[0] * 64 + l + 48);
         const V4 xp = ld4(u, x < 3 ? base + l + 16 : (size_t)nb[1] * 64 + l - 48);
@@ -125,7 +126,7 @@ struct Stencil4 {
             float result = 0.f;
 #pragma unroll
             for (int q = 0; q < 6; ++q)
-                if (f[k] & (kFaceMX << q)) result -= (nv[q] - cv);
+                if (f[k] >> q & 1u) result -= (nv[q] - cv);
             r.v[k] = bv.v[k] - result;
         }
     }
@@ -139,20 +140,33 @@ __host__ __device__ inline int sweep_groups(int np) { return (np + kSweepPages -
 // One damped-Jacobi sweep (residual + correction fused, ping-pong buffers);
 // u += (omega / face count) r on the selected cells
 // (LIB/SPGrid_Correction_Legacy.h:60-77), other cells copied unchanged.
-template <class S>
+// kAgain: u_out already holds the cells that this kind of sweep leaves alone (it is
+// the iterate before u_in), so lanes without a cell to write are done: at 32^3
+// subdomains a third of the lines. Bound by memory: 13 bytes a cell, of which one is
+// the kinds (the flags' four made it 16). 256^3: 55 us a sweep with flags, 46 with
+// kinds, 37 again (the same card).
+template <class S, bool kAgain>
 __global__ void __launch_bounds__(64 * kSweepPages) k_smooth(DevLevel L, const S* __restrict__ u_in, S* __restrict__ u_out,
-                                                             const S* __restrict__ b, int write_interior, int write_boundary) {
+                                                             const S* __restrict__ b, uint32_t interior, uint32_t boundary) {
     const int ng = sweep_groups(L.np), gi = xcd_page(ng), l = threadIdx.x & 63;
     const int p = gi * kSweepPages + (int)(threadIdx.x >> 6);
     if (gi >= ng || p >= L.np || page_stopped(L, p)) return;
+    // a kind is written when its Active and Boundary bits are `interior` or `boundary` (0: none)
+    auto written = [&](uint32_t f) {
+        const uint32_t sel = f & (kKindActive | kKindBoundary);
+        return sel && (sel == interior || sel == boundary);
+    };
+    if (kAgain) {
+        const uint32_t fv = reinterpret_cast<const uint32_t*>(L.kinds)[(size_t)p * 64 + l];
+        if (!written(fv & 0xffu) && !written(fv >> 8 & 0xffu) && !written(fv >> 16 & 0xffu) && !written(fv >> 24)) return;
+    }
     const Stencil4<S> st(L, p, l, u_in, b);
     V4 out;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        const uint32_t f = st.f[k], sel = f & (kActive | kBoundary);
-        const bool w = (sel == kActive && write_interior) || (sel == (kActive | kBoundary) && write_boundary);
+        const uint32_t f = st.f[k];
         float u = st.uc.v[k];
-        if (w) u += c_omega_fc[__popc(f & (0x3fu * kFaceMX))] * st.r.v[k];
+        if (written(f)) u += c_omega_fc[__popc(f & kKindFaces)] * st.r.v[k];
         out.v[k] = u;
     }
     st4(u_out, (size_t)p * 64 + l, out);
@@ -321,7 +335,7 @@ __global__ void __launch_bounds__(256) k_residual(DevLevel L, const S* __restric
     const Stencil4<S> st(L, p, l, u, b);
     V4 out;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) out.v[k] = (st.f[k] & kActive) ? st.r.v[k] : 0.f;
+    for (int k = 0; k < 4; ++k) out.v[k] = (st.f[k] & kKindActive) ? st.r.v[k] : 0.f;
     st4(r, (size_t)p * 64 + l, out);
 }
 
@@ -793,9 +807,10 @@ void upload_constants() {
 }
 
 template <class S>
-static void smooth_t(const DevLevel& L, const S* u_in, S* u_out, const S* b, bool interior, bool boundary, hipStream_t s) {
-    if (L.np) hipLaunchKernelGGL(k_smooth<S>, dim3(kXcds * xcd_chunk(sweep_groups(L.np))), dim3(64 * kSweepPages), 0, s, L, u_in, u_out, b, (int)interior,
-                                 (int)boundary);
+static void smooth_t(const DevLevel& L, const S* u_in, S* u_out, const S* b, bool interior, bool boundary, bool again, hipStream_t s) {
+    if (!L.np) return;
+    hipLaunchKernelGGL((again ? k_smooth<S, true> : k_smooth<S, false>), dim3(kXcds * xcd_chunk(sweep_groups(L.np))), dim3(64 * kSweepPages), 0, s,
+                       L, u_in, u_out, b, interior ? kKindActive : 0u, boundary ? kKindActive | kKindBoundary : 0u);
 }
 template <class S, int C>
 static void cluster_sweeps_c(const DevLevel& L, const DevClusters& W, S* u, const S* b, S* r, const SweepPhases& ph, bool u_zero, hipStream_t s) {
@@ -836,11 +851,11 @@ template <class S>
 static void prolong_t(const DevLevel& F, const DevLevel& C, S* u_f, const S* u_c, hipStream_t s) {
     if (F.np) hipLaunchKernelGGL(k_prolong<S>, dim3(kXcds * xcd_chunk(F.np)), dim3(256), 0, s, F, C, u_f, u_c);
 }
-void launch_smooth(const DevLevel& L, const float* u_in, float* u_out, const float* b, bool interior, bool boundary, hipStream_t s) {
-    smooth_t(L, u_in, u_out, b, interior, boundary, s);
+void launch_smooth(const DevLevel& L, const float* u_in, float* u_out, const float* b, bool interior, bool boundary, bool again, hipStream_t s) {
+    smooth_t(L, u_in, u_out, b, interior, boundary, again, s);
 }
-void launch_smooth(const DevLevel& L, const __half* u_in, __half* u_out, const __half* b, bool interior, bool boundary, hipStream_t s) {
-    smooth_t(L, u_in, u_out, b, interior, boundary, s);
+void launch_smooth(const DevLevel& L, const __half* u_in, __half* u_out, const __half* b, bool interior, bool boundary, bool again, hipStream_t s) {
+    smooth_t(L, u_in, u_out, b, interior, boundary, again, s);
 }
 void launch_cluster_sweeps(const DevLevel& L, const DevClusters& C, float* u, const float* b, float* r, const SweepPhases& ph, bool u_zero,
                            hipStream_t s) {

@@ -83,7 +83,7 @@ DevLevel LevelBuffers::view() const {
     DevLevel v;
     v.np = host.npages();
     v.nbx = host.nbx; v.nby = host.nby; v.nbz = host.nbz;
-    v.flags = flags.p; v.nbr = nbr.p; v.base = base.p; v.lut = lut.p;
+    v.flags = flags.p; v.kinds = kinds.p; v.nbr = nbr.p; v.base = base.p; v.lut = lut.p;
     v.prob = prob.p; v.active = active;
     return v;
 }
@@ -172,9 +172,9 @@ void ProblemHost::factorize(bool wait) {
 }
 
 size_t ProblemHost::device_bytes() const {
-    // every level: flags, two smoothing buffers, b, r (4 B each per slot), neighbour and origin tables
+    // every level: flags (5 B), two smoothing buffers, b, r (4 B each per slot), neighbour and origin tables
     double bytes = 0;
-    for (const PagedLevel& L : lv) bytes += (L.npages() + 1.0) * kPageCells * 20.0 + L.npages() * 36.0;
+    for (const PagedLevel& L : lv) bytes += (L.npages() + 1.0) * kPageCells * 21.0 + L.npages() * 36.0;
     bytes += (lv[0].npages() + 1.0) * kPageCells * 16.0;  // x, b, q, s
     // interface solver: dense-node plans of the factors, operators, vectors
     for (int l = 0; l < sigma.levels; ++l) {
@@ -530,6 +530,10 @@ static void upload_level(LevelBuffers& L) {
         std::vector<uint32_t> f(H.flags);
         f.resize((size_t)(np + 1) * kPageCells, 0u);
         L.flags.upload(f);
+        std::vector<uint8_t> k(f.size());
+        for (size_t i = 0; i < f.size(); ++i)
+            k[i] = (uint8_t)((f[i] / kFaceMX & kKindFaces) | (f[i] & kActive ? kKindActive : 0u) | (f[i] & kBoundary ? kKindBoundary : 0u));
+        L.kinds.upload(k);
         std::vector<int> nb((size_t)np * 6), base((size_t)np * 3);
         for (int p = 0; p < np; ++p) {
             const Int3 o = H.page_base[p];
@@ -573,9 +577,9 @@ double profile_sweep_pages(Int3 size, int n_pages, const uint64_t* page_offsets,
         hdd_check(hipEventCreate(&a), "hipEventCreate");
         hdd_check(hipEventCreate(&b), "hipEventCreate");
         const DevLevel v = L.view();
-        launch_smooth(v, L.u[0].p, L.u[1].p, L.b.p, true, true, s);  // warm
+        launch_smooth(v, L.u[0].p, L.u[1].p, L.b.p, true, true, false, s);  // warm
         hdd_check(hipEventRecord(a, s), "hipEventRecord");
-        for (int i = 0; i < reps; ++i) launch_smooth(v, L.u[i & 1].p, L.u[1 - (i & 1)].p, L.b.p, true, true, s);
+        for (int i = 0; i < reps; ++i) launch_smooth(v, L.u[i & 1].p, L.u[1 - (i & 1)].p, L.b.p, true, true, false, s);
         hdd_check(hipEventRecord(b, s), "hipEventRecord");
         hdd_check(hipEventSynchronize(b), "hipEventSynchronize");
         hdd_check(hipEventElapsedTime(&ms, a, b), "hipEventElapsedTime");
@@ -625,7 +629,7 @@ void Solver::sweeps_t(int l, int count, bool interior, bool boundary) {
     LevelBuffers& L = lv[l];
     const DevLevel v = L.view();
     for (int i = 0; i < count; ++i) {
-        launch_smooth(v, VStore<S>::u(L, L.cur), VStore<S>::u(L, 1 - L.cur), VStore<S>::b(L), interior, boundary, stream);
+        launch_smooth(v, VStore<S>::u(L, L.cur), VStore<S>::u(L, 1 - L.cur), VStore<S>::b(L), interior, boundary, i > 0 && interior != boundary, stream);
         L.cur = 1 - L.cur;
     }
 }

@@ -94,6 +94,7 @@ struct ProblemHost {
 struct LevelBuffers {
     PagedLevel host;
     DBuf<uint32_t> flags;
+    DBuf<uint8_t> kinds;
     DBuf<int> nbr, base, lut;
     DBuf<int> prob;                 // problem of each page (zero page: -1)
     const int* active = nullptr;    // set while a batch PCG runs: its per-problem flags

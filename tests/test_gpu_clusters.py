@@ -1,6 +1,7 @@
 """Sweeps of whole clusters in one launch (every V-cycle level whose clusters of coupled cells fit a
 workgroup) against one launch per sweep (HDD_BOTTOM_LOCAL=0): the same operations in the same order,
-so the bar is equal bits. The cases have clusters from a few cells (one wavefront, neighbours in
+so the bar is equal bits (which also holds the single sweeps that skip what the sweep before left in place
+against sweeps that write every cell). The cases have clusters from a few cells (one wavefront, neighbours in
 registers) to several per thread, one cluster per workgroup and packed ones, a level 0 whose cluster
 edges read interface cells, a single-level V-cycle (200 sweeps of level 0 around nonzero interface
 values), and levels on both sides of the size limit."""
