@@ -204,7 +204,7 @@ def main():
     fp16 = {"time_to_tolerance_s": float(np.mean(t16)), "solves_per_s": 1.0 / float(np.mean(t16)), "iterations": int(np.median(it16)),
             "sweep_us": h_ms * 1e3, "sweep_achieved_GBs": h_bytes / (h_ms * 1e-3) / 1e9,
             "sweep_frac": h_bytes / (h_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "sweep_bytes_per_slot": 10}
-    fp16["traffic"] = counter_traffic(dom.n_pages, "k_smooth<__half>") if args.config == "sphere256" else None
+    fp16["traffic"] = counter_traffic(dom.n_pages, "k_smooth<__half, false>") if args.config == "sphere256" else None
     log(f"[bench] fp16-storage V-cycles: {fp16['iterations']} iterations, {fp16['time_to_tolerance_s']:.3f}s; "
         f"level-0 sweep {h_ms * 1e3:.1f} us ({fp16['sweep_achieved_GBs']:.0f} GB/s algorithmic at 10 B/slot)")
     solver.close()
@@ -232,7 +232,7 @@ def main():
                    "sub_size": cfg.sub_size, "vlevels": cfg.vlevels, "sigma_levels": cfg.sigma_levels,
                    "tolerance": "max|r| <= 1e-6 max|b|", "iterations": int(np.median(iters)),
                    "time_to_tolerance_s": float(np.mean(times)), "setup_s": st["setup_s"], "factor_s": st["factor_s"]},
-        "roofline": {"kernel": f"level-{dom_plan['level']} {dom_plan['plan']} triangular-solve plan (k_tri_* / k_top_* chain, "
+        "roofline": {"kernel": f"level-{dom_plan['level']} {dom_plan['plan']} triangular-solve plan (k_node_* chain, "
                                f"{100 * dom_plan['share_of_iteration']:.0f}% of a PCG iteration)",
                      "bound": "hbm", "achieved": dom_plan["achieved_GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": dom_plan["achieved_GBs"] / HBM_PEAK_GBS,
@@ -315,7 +315,7 @@ def sweep_grid_threads(pages):
     return 8 * ((groups + 7) // 8) * 512
 
 
-def counter_traffic(pages, kernel="k_smooth<float>"):
+def counter_traffic(pages, kernel="k_smooth<float, false>"):
     """HBM bytes of one level-0 sweep from the committed rocprofv3 counter summaries.
 
     FETCH_SIZE and WRITE_SIZE (KiB per dispatch) of the sweep kernel at its

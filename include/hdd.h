@@ -261,8 +261,9 @@ hdd_status hdd_inner_product(hdd_ctx* ctx, int ch_a, int ch_b, double* out);
  * every cell of (float)(a*b), summed in double, with the bits hdd_inner_product
  * gives on a one-problem context holding the same pages. Enqueued on `stream`
  * (a hipStream_t; NULL: the null stream) and returns before it runs. The
- * partial sums live in a file-scope device array of 1024 doubles (8 KiB), one
- * per device, held until the process ends; nothing is allocated or freed.
+ * partial sums live in a file-scope device array of 1024 doubles (8 KiB, and
+ * 64 tickets), one per device, held until the process ends; nothing is
+ * allocated or freed.
  * Calls that overlap on one device race on that array. n_pages must be in
  * [1, HDD_NOALLOC_MAX_PAGES]; hdd_last_error(NULL) gives the message of a
  * failure. */
