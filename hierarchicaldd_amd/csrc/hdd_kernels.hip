@@ -401,38 +401,53 @@ __global__ void __launch_bounds__(256) k_restrict(DevLevel F, DevLevel C, const 
 // fine u += sum_{2x2x2} w u_coarse (Active fine cells only). The coarse cells
 // a fine page (origin o) reads form the region o/2 .. o/2+2 (x) and
 // o/2 .. o/2+4 (y, z), 3 x 5 x 5 cells in 2 x 2 x 2 coarse blocks: its pages
-// are looked up once and the region is staged in LDS once per workgroup.
+// are looked up once and the region is staged in LDS once per page. A wavefront
+// per page, four cells per lane as in the sweeps, and no workgroup barrier:
+// bound by the chain origin, page, coarse value, so by the pages in flight (a
+// workgroup per page, a cell per thread: 85 us at 256^3, now 47).
 template <class S>
 __global__ void __launch_bounds__(256) k_prolong(DevLevel F, DevLevel C, S* __restrict__ u_f, const S* __restrict__ u_c) {
     constexpr int RX = 3, RY = 5, RZ = 5;
-    __shared__ int tab[8];
-    __shared__ float su[RX * RY * RZ];
-    const int p = xcd_page(F.np), c = threadIdx.x, e = p * 256 + c;
-    if (p >= F.np || page_stopped(F, p)) return;  // uniform over the workgroup
-    const uint32_t fl = F.flags[e];  // the cell's own loads go out before the staging's
-    float u = ld(u_f, e);
+    __shared__ float staged[4][RX * RY * RZ + 1];
+    const int ng = page_groups(F.np), gi = xcd_page(ng), l = threadIdx.x & 63;
+    const int p = gi * 4 + (int)(threadIdx.x >> 6);
+    if (gi >= ng || p >= F.np || page_stopped(F, p)) return;
+    float* su = staged[threadIdx.x >> 6];
+    const size_t at = (size_t)p * 64 + l;
+    const uint32_t fl = reinterpret_cast<const uint32_t*>(F.kinds)[at];  // the cells' own loads go out before the staging's
+    V4 u = ld4(u_f, at);
     const int ox = F.base[p * 3 + 0], oy = F.base[p * 3 + 1], oz = F.base[p * 3 + 2];
     const int X0 = ox >> 1, Y0 = oy >> 1, Z0 = oz >> 1;
     const int bx0 = X0 >> 2, by0 = Y0 >> 3, bz0 = Z0 >> 3;
-    if (c < 8) tab[c] = lut_block(C, bx0 + (c >> 2), by0 + ((c >> 1) & 1), bz0 + (c & 1));
-    __syncthreads();
-    if (c < RX * RY * RZ) {
-        const int X = X0 + c / (RY * RZ), Y = Y0 + (c / RZ) % RY, Z = Z0 + c % RZ;
-        const int q = tab[((X >> 2) - bx0) * 4 + ((Y >> 3) - by0) * 2 + ((Z >> 3) - bz0)];
-        su[c] = ld(u_c, q * 256 + ((X & 3) << 6 | (Y & 7) << 3 | (Z & 7)));
+    const int block = lut_block(C, bx0 + (l >> 2 & 1), by0 + (l >> 1 & 1), bz0 + (l & 1));  // lane q (and q + 8, ..): block q
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int t = min(l + 64 * i, RX * RY * RZ - 1);
+        const int X = X0 + t / (RY * RZ), Y = Y0 + (t / RZ) % RY, Z = Z0 + t % RZ;
+        const int q = __shfl(block, ((X >> 2) - bx0) * 4 + ((Y >> 3) - by0) * 2 + ((Z >> 3) - bz0));
+        su[t] = ld(u_c, q * 256 + ((X & 3) << 6 | (Y & 7) << 3 | (Z & 7)));
     }
-    __syncthreads();
-    if (!(fl & kActive)) return;
-    const int x = ox + (c >> 6), y = oy + ((c >> 3) & 7), z = oz + (c & 7);
-    const int cx = (x + 1) >> 1, cy = (y + 1) >> 1, cz = (z + 1) >> 1;
-    const int px = 1 - (x - (2 * cx - 1)), py = 1 - (y - (2 * cy - 1)), pz = 1 - (z - (2 * cz - 1));
-    for (int i = 0; i < 2; ++i)
-        for (int j = 0; j < 2; ++j)
-            for (int k = 0; k < 2; ++k) {
-                const int X = cx + i - px, Y = cy + j - py, Z = cz + k - pz;
-                u += c_pweights[((i ^ px) << 2) | ((j ^ py) << 1) | (k ^ pz)] * su[((X - X0) * RY + (Y - Y0)) * RZ + (Z - Z0)];
-            }
-    st(u_f, e, u);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int x = ox + (l >> 4), y = oy + (l >> 1 & 7);
+    const int cx = (x + 1) >> 1, cy = (y + 1) >> 1;
+    const int px = 1 - (x - (2 * cx - 1)), py = 1 - (y - (2 * cy - 1));
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        if (!(fl >> (8 * n) & kKindActive)) continue;
+        const int z = oz + 4 * (l & 1) + n;
+        const int cz = (z + 1) >> 1, pz = 1 - (z - (2 * cz - 1));
+        float v = u.v[n];
+        for (int i = 0; i < 2; ++i)
+            for (int j = 0; j < 2; ++j)
+                for (int k = 0; k < 2; ++k) {
+                    const int X = cx + i - px, Y = cy + j - py, Z = cz + k - pz;
+                    v += c_pweights[((i ^ px) << 2) | ((j ^ py) << 1) | (k ^ pz)] * su[((X - X0) * RY + (Y - Y0)) * RZ + (Z - Z0)];
+                }
+        u.v[n] = v;
+    }
+    st4(u_f, at, u);
 }
 
 // PCG operator: out = L v on Active|Interface cells (double accumulation); kZero: 0 elsewhere
@@ -856,7 +871,7 @@ static void restrict_t(const DevLevel& F, const DevLevel& C, const S* r_f, S* b_
 }
 template <class S>
 static void prolong_t(const DevLevel& F, const DevLevel& C, S* u_f, const S* u_c, hipStream_t s) {
-    if (F.np) hipLaunchKernelGGL(k_prolong<S>, dim3(kXcds * xcd_chunk(F.np)), dim3(256), 0, s, F, C, u_f, u_c);
+    if (F.np) hipLaunchKernelGGL(k_prolong<S>, dim3(kXcds * xcd_chunk(page_groups(F.np))), dim3(256), 0, s, F, C, u_f, u_c);
 }
 void launch_smooth(const DevLevel& L, const float* u_in, float* u_out, const float* b, bool interior, bool boundary, bool again, hipStream_t s) {
     smooth_t(L, u_in, u_out, b, interior, boundary, again, s);
