@@ -10,7 +10,9 @@
 namespace hdd {
 
 inline void hdd_check(hipError_t e, const char* what = "HIP call") {
-    if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
+    if (e == hipSuccess) return;
+    (void)hipGetLastError();  // reported here: the checks after later launches report their own
+    throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
 // One paged level on the device. flags has (np+1)*256 entries (zero page last), kinds the

@@ -20,6 +20,7 @@
 #include <chrono>
 #include <functional>
 #include <memory>
+#include <utility>
 #include <vector>
 #include "hdd_device.h"
 #include "hdd_setup.h"
@@ -40,14 +41,20 @@ struct DBuf {
     DBuf(const DBuf&) = delete;
     DBuf& operator=(const DBuf&) = delete;
     DBuf(DBuf&& o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+    DBuf& operator=(DBuf&& o) noexcept {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+        return *this;
+    }
     ~DBuf() { if (p) (void)hipFree(p); }
     // The clear and the upload go through the null stream, which does not order
     // the contexts' non-blocking streams: both wait for completion before returning.
     void alloc(size_t count) {
         if (p) { (void)hipFree(p); p = nullptr; }
-        n = count;
+        n = 0;
         if (count) {
             hdd_check(hipMalloc(&p, count * sizeof(T)), "hipMalloc");
+            n = count;
             hdd_check(hipMemset(p, 0, count * sizeof(T)), "hipMemset");
             hdd_check(hipStreamSynchronize(nullptr), "hipMemset");
         }

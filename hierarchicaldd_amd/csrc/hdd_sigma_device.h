@@ -46,15 +46,8 @@ struct SlicedDev {
 // from their supernodal factors: the dense-node form (hdd_nodeplan.h), or the
 // per-height form (layout in hdd_triplan.h) for refined solves, for batches
 // outside the dense-node form's limits, and where the environment asks for it.
-struct TriPlan {
-    int n = 0, H = -1;      // H: tree heights of the per-height form, -1 until it is built
-    bool use_nodes = false;
-    NodePlan nodes;
-    // the factors outlive the plan (the problems a solver holds own them)
-    std::vector<const SupernodalFactor*> F;
-    std::vector<int> offsets, prob_of;
-    void build_heights();
-    size_t factor_nnz = 0;
+struct TriHeights {          // the per-height form
+    int H = -1;              // tree heights; -1 until every part of the form is there
     // per-height ranges and launch parameters (host copies)
     std::vector<int> sn_begin, sl_begin, sl_rows, row_begin, ci_begin, bi_begin, max_sz, big, fused, G, Gc, Gf, Gb, run_begin, run_max;
     std::vector<int> wave;  // per fused height: 1 = a wavefront per run (k_tri_*_wave), 0 = a workgroup per run (same results)
@@ -62,10 +55,30 @@ struct TriPlan {
     // per fused height: a cap on the workgroups of its launch, each looping over runs (default:
     // no cap, a workgroup per run; the tuner tries caps; results do not depend on it)
     std::vector<int> pgrid;
-    static constexpr int kFusedGroups = 1 << 30;
     DBuf<int> run_q, run_n, orig_of, s0, sz, nr, roff, srows, sn_of, sn_prob, sn_list, sl_sn, sl_r0, rowlist, inc_ptr, ci_sn, ci_a0, ci_a1, bi_sn, bi_c, bi_j0;
     DBuf<long long> loff, doff, cofs, cpos, bofs;
     DBuf<float> diag, diagT, l21, c, bpart, t, y;
+    std::vector<int> ci_entries, h_sn_list, h_sz, h_nr;  // host copies the tuner rebuilds the lists from
+    // dense tops (hdd_triplan.h): padded top rows, their tops, the Linv blocks
+    int top_nq = 0, Gt = 4;
+    long long top_dense_rows = 0;                        // rows of the distinct dense blocks
+    DBuf<int> top_rows, top_of, top_inc_ptr, top_base, top_ld;
+    DBuf<long long> top_cpos, top_woff;
+    DBuf<float> top_W, top_t;
+};
+
+struct TriPlan : TriHeights {
+    int n = 0;
+    bool use_nodes = false;
+    NodePlan nodes;
+    // the factors outlive the plan (the problems a solver holds own them)
+    std::vector<const SupernodalFactor*> F;
+    std::vector<int> offsets, prob_of;
+    // the per-height form; when it throws the plan has none, as before the call
+    void build_heights();
+    void drop_heights() { static_cast<TriHeights&>(*this) = TriHeights(); }
+    size_t factor_nnz = 0;
+    static constexpr int kFusedGroups = 1 << 30;
     // prob_of[m]: problem of factor m (empty: all problem 0)
     void build(const std::vector<const SupernodalFactor*>& factors, const std::vector<int>& offs, const std::vector<int>& probs = {});
     // per-problem flags (device, 1 = iterating): supernodes of stopped problems are skipped; nullptr: none skipped
@@ -84,15 +97,8 @@ struct TriPlan {
     // launch-shape autotuner (slice rows, contribution items per height); returns the choices changed
     int tune(hipStream_t s);
     size_t bytes() const;
-    std::vector<int> ci_entries, h_sn_list, h_sz, h_nr;  // host copies the tuner rebuilds the lists from
     static constexpr int kTuneMinRows = 20000;           // plans below this size keep their default shapes
     void rebuild_lists(hipStream_t s);
-    // dense tops (hdd_triplan.h): padded top rows, their tops, the Linv blocks
-    int top_nq = 0, Gt = 4;
-    long long top_dense_rows = 0;                        // rows of the distinct dense blocks
-    DBuf<int> top_rows, top_of, top_inc_ptr, top_base, top_ld;
-    DBuf<long long> top_cpos, top_woff;
-    DBuf<float> top_W, top_t;
     void top_solve(const float* b_orig, float* x_orig, hipStream_t s);
 };
 

@@ -1080,13 +1080,12 @@ void TriPlan::build(const std::vector<const SupernodalFactor*>& factors, const s
     if (!use_nodes) build_heights();
 }
 
-void TriPlan::build_heights() {
+void TriPlan::build_heights() try {
     if (n == 0 || H >= 0) return;
     TriPlanHost P;
     auto tp = std::chrono::steady_clock::now();
     build_triplan(F, offsets, P, dense_top_min_rows());
     setup_phase("  plan lists and float blocks", (int)F.size(), tp, "factors");
-    H = P.H;
     {
         // problem of each supernode (supernodes are numbered factor by factor, in order)
         std::vector<int> sp(P.s0.size(), 0);
@@ -1137,6 +1136,10 @@ void TriPlan::build_heights() {
         for (size_t k = 0; k < P.top_blocks.size(); ++k) dense_top_inverse(P.top_blocks[k], top_W.p + block_off[k]);
         setup_phase("  dense tops inverted", (int)P.top_blocks.size(), tp, "blocks");
     }
+    H = P.H;  // last: a solve, a retry and the tuner take the form to be there from now on
+} catch (...) {
+    drop_heights();
+    throw;
 }
 
 size_t TriPlan::bytes() const {
@@ -1888,10 +1891,15 @@ void SigmaDevice::set_refinement(const std::vector<const SigmaHost*>& hosts, int
         plans.push_back(&Lbottom);
         for (TriPlan* p : plans) {
             if (p->n == 0 || p->H >= 0) continue;
-            plan_bytes -= p->bytes();
+            const size_t before = p->bytes();
             p->build_heights();
-            if (autotune()) tuned_choices += p->tune(stream);
-            plan_bytes += p->bytes();
+            try {
+                if (autotune()) tuned_choices += p->tune(stream);
+            } catch (...) {
+                p->drop_heights();  // a half-tuned plan's lists may not fit its arrays
+                throw;
+            }
+            plan_bytes += p->bytes() - before;
             dense_top_rows += p->top_dense_rows;
         }
     }
