@@ -1,6 +1,7 @@
 #include "hdd_nodeplan.h"
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <map>
@@ -235,6 +236,55 @@ bool same_columns(const SupernodalFactor& fa, const std::vector<int>& a, const S
     return true;
 }
 
+// Share of the constant in the rows of a block's inverse, in units of the diagonal's: with m rows that are
+// coupled to each other, sum of all entries over sum of the diagonal q, and the constant nearly an
+// eigenvector, the inverse's rows have a part of 2-norm 1 / (q sqrt(m)) along it. Rounded to float, the
+// inverse leaves 0.3 * 2^-24 of that in every row, also where the right-hand side has no such part (a domain
+// without Dirichlet cells: its right-hand sides sum to zero, its operator annihilates the constant but for
+// the 1e-5 on the diagonal). The triangles leave their rounding in the constant itself, where the operator
+// does not see it. So a block beyond kMaxConstant keeps the two passes.
+// Measured as the error outside the smallest mode, inverse against two passes (blocks of 27 to 4129 columns,
+// in float): 0.2 to 4.8 times for shares below 1.2 (every block of the Dirichlet domains looked at, 32^3 to
+// 160^3, and of a channel of 3 x 3 x 126 cells), 3.3 times at 42 (four Dirichlet cells on a 32^3 box), 32 times at
+// 510 (one on a 64^3 box), 390 to 710 times at 13,000 to 23,000 (none on 32^3 to 64^3). At 100 it is 2e-6, what the
+// two passes have at the last of these.
+constexpr double kMaxConstant = 100;
+double constant_share(const P_::Block& B) {
+    const SupernodalFactor& f = *B.f;
+    std::vector<int> at, part(B.n);
+    local_rows(f, B.sns, B.n, at);
+    for (int i = 0; i < B.n; ++i) part[i] = i;
+    auto find = [&](int a) {
+        while (part[a] != a) a = part[a] = part[part[a]];
+        return a;
+    };
+    auto columns = [&](auto&& use) {  // use(column, row, entry) for the entries of the triangle, column after column
+        int col = 0;
+        const int* row = at.data();
+        for (int s : B.sns) {
+            const int n = f.sn[s].n, nr = (int)f.sn[s].rows.size();
+            for (int j = 0; j < n; ++j) {
+                for (int r = j; r < n; ++r) use(col + j, col + r, f.L11[s][(size_t)j * n + r]);
+                for (int a = 0; a < nr; ++a) use(col + j, row[a], f.L21[s][(size_t)j * nr + a]);
+            }
+            col += n;
+            row += nr;
+        }
+    };
+    columns([&](int j, int i, double l) { if (l != 0 && i != j) part[find(i)] = find(j); });
+    std::vector<double> sum(B.n, 0.0), all(B.n, 0.0), diag(B.n, 0.0);  // of a column; of a part's entries, of its diagonal
+    std::vector<int> m(B.n, 0);
+    columns([&](int j, int i, double l) {
+        sum[j] += l;
+        diag[find(i)] += l * l;
+    });
+    for (int j = 0; j < B.n; ++j) { const int p = find(j); all[p] += sum[j] * sum[j]; ++m[p]; }
+    double share = 0;
+    for (int p = 0; p < B.n; ++p)
+        if (m[p] > 1) share = std::max(share, diag[p] / (all[p] * std::sqrt((double)m[p])));
+    return share;
+}
+
 // Work items of one run in one pass: `rows` row tiles of up to `len` tiles, `level_rows` row tiles in
 // the level. A wave streams about four tiles per memory round trip, so the waves of a workgroup share
 // a row tile (split) until each has at most kWaveTiles of its tiles, or 4 where the chip has waves to
@@ -359,6 +409,19 @@ bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::ve
                 B.nk = tiles_of(nd.n); B.nrk = tiles_of(nd.nr);
                 P.blocks.push_back(B);
             }
+    }
+    // a nearly singular block without boundary rows gets a boundary tile of zeros, and with it the two passes
+    {
+        ParallelErrors errs;
+#pragma omp parallel for schedule(dynamic)
+        for (size_t k = 0; k < P.blocks.size(); ++k)
+            errs.run([&] {
+                P_::Block& B = P.blocks[k];
+                if (!B.nr && !(constant_share(B) <= kMaxConstant)) B.nrk = 1;
+            });
+        errs.rethrow();
+        for (const P_::Block& B : P.blocks)
+            if (T * (B.nk + B.nrk) + 4 > P_::kMaxLdsFloats) return false;
     }
     for (P_::Block& B : P.blocks) {
         const long long t = block_tiles(B.nk, B.nrk);

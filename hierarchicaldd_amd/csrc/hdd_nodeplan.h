@@ -13,7 +13,9 @@
 //   backward  z = [I + S^T | -W^T] [D^-2 y; z of the boundary rows]
 // A closed node (no boundary rows: the root of a tree) holds its inverse, z = Linv^T Linv t, in
 // place of the triangle and its transpose (the same number of elements in one launch instead of
-// two; a launch of a few us is most of a small solve) and has no backward pass. So a pass is one
+// two; a launch of a few us is most of a small solve) and has no backward pass, unless the block
+// is nearly singular (constant_share in hdd_nodeplan.cpp), when it keeps the two passes with a
+// boundary tile of zeros. So a pass is one
 // launch per band (level), less the last band's backward, and one more forward for the
 // children's sums where there are any. Blocks are formed in double on the
 // device at set-up and held in float, as the per-height plan holds its own. With
