@@ -76,13 +76,41 @@ struct Nodes {
     std::vector<int> ptr, child, row;
 };
 
-double estimate_level(const std::vector<const SupernodalFactor*>& distinct, const std::vector<int>& members,
-                      const std::vector<std::vector<Hash>>& sh, int H, int a, int b, bool* ok) {
-    std::unordered_map<Hash, std::pair<long long, double>, HashKey> seen;  // node content -> members, bytes
-    std::unordered_map<Hash, int, HashKey> limit;
-    *ok = true;
-    for (size_t d = 0; d < distinct.size(); ++d) {
-        const SupernodalFactor& f = *distinct[d];
+// The distinct factors of a batch, how often each is solved with, and the content of their supernodes
+struct Batch {
+    std::vector<const SupernodalFactor*> distinct;
+    std::vector<int> members, which;  // which: distinct factor of each one passed
+    std::vector<std::vector<Hash>> sh;
+    int H = -1;                       // tallest tree
+    explicit Batch(const std::vector<const SupernodalFactor*>& F) : which(F.size()) {
+        std::map<const SupernodalFactor*, int> id;
+        for (size_t m = 0; m < F.size(); ++m) {
+            if (F[m]->n) H = std::max(H, F[m]->max_height);
+            auto e = id.emplace(F[m], (int)distinct.size());
+            if (e.second) { distinct.push_back(F[m]); members.push_back(0); }
+            which[m] = e.first->second;
+            ++members[which[m]];
+        }
+        sh.resize(distinct.size());
+        std::vector<std::pair<int, int>> todo;
+        for (size_t d = 0; d < distinct.size(); ++d) {
+            sh[d].resize(distinct[d]->sn.size());
+            for (int s = 0; s < (int)sh[d].size(); ++s) todo.push_back({(int)d, s});
+        }
+        ParallelErrors errs;
+#pragma omp parallel for schedule(dynamic, 16)
+        for (size_t i = 0; i < todo.size(); ++i)
+            errs.run([&] { sh[todo[i].first][todo[i].second] = supernode_hash(*distinct[todo[i].first], todo[i].second); });
+        errs.rethrow();
+    }
+};
+
+// the nodes of a band of heights [a, b) by content; false when one is beyond the form's limits
+struct NodeKind { long long members = 0; int nk = 0, nrk = 0; };
+using NodeKinds = std::unordered_map<Hash, NodeKind, HashKey>;
+bool band_nodes(const Batch& B, int a, int b, NodeKinds& kinds) {
+    for (size_t d = 0; d < B.distinct.size(); ++d) {
+        const SupernodalFactor& f = *B.distinct[d];
         const int ns = (int)f.sn.size();
         std::vector<int> n(ns, 0);
         std::vector<Hash> h(ns);
@@ -90,37 +118,43 @@ double estimate_level(const std::vector<const SupernodalFactor*>& distinct, cons
             const Supernode& S = f.sn[s];
             if (S.height < a || S.height >= b) continue;
             n[s] += S.n;
-            h[s].word(sh[d][s].a);
+            h[s].word(B.sh[d][s].a);
             const int p = S.parent;
             if (p >= 0 && f.sn[p].height < b) {
                 n[p] += n[s];
                 h[p].word(h[s].a);
                 continue;
             }
-            const int nr = (int)S.rows.size(), nk = tiles_of(n[s]), nrk = tiles_of(nr);
-            if (T * (nk + nrk) + 4 > P_::kMaxLdsFloats || (b > a + 1 && n[s] > kMaxMergedColumns)) { *ok = false; return 0; }
-            auto& e = seen[h[s]];
-            e.first += members[d];
-            e.second = 1024.0 * (double)block_tiles(nk, nrk) * 1e-6;
-            limit[h[s]] = run_limit(T * (nk + nrk));
+            const int nk = tiles_of(n[s]), nrk = tiles_of((int)S.rows.size());
+            if (T * (nk + nrk) + 4 > P_::kMaxLdsFloats || (b > a + 1 && n[s] > kMaxMergedColumns)) return false;
+            NodeKind& k = kinds[h[s]];
+            k.members += B.members[d];
+            k.nk = nk; k.nrk = nrk;
         }
     }
-    if (seen.empty()) return 0;
+    return true;
+}
+
+double estimate_level(const Batch& B, int a, int b, bool* ok) {
+    NodeKinds kinds;
+    *ok = band_nodes(B, a, b, kinds);
+    if (!*ok || kinds.empty()) return 0;
     double distinct_mb = 0, again_mb = 0, runs = 0;
-    for (auto& e : seen) {
-        const int lim = limit[e.first];
-        const double r = (double)((e.second.first + lim - 1) / lim);
-        distinct_mb += e.second.second;
-        again_mb += (r - 1) * e.second.second;
+    for (auto& e : kinds) {
+        const NodeKind& k = e.second;
+        const int lim = run_limit(T * (k.nk + k.nrk));
+        const double r = (double)((k.members + lim - 1) / lim), mb = 1024.0 * (double)block_tiles(k.nk, k.nrk) * 1e-6;
+        distinct_mb += mb;
+        again_mb += (r - 1) * mb;
         runs += r;
     }
-    return kLaunchUs * (1 + (a > 0) + (b <= H)) + distinct_mb / kMemoryMBPerUs + again_mb / kCacheMBPerUs + runs * kRunUs;
+    return kLaunchUs * (1 + (a > 0) + (b <= B.H)) + distinct_mb / kMemoryMBPerUs + again_mb / kCacheMBPerUs + runs * kRunUs;
 }
 
 // band boundaries 0 = c_0 < c_1 < .. = H + 1 of least estimated time (empty: none is possible)
-std::vector<int> choose_cuts(const std::vector<const SupernodalFactor*>& distinct, const std::vector<int>& members,
-                             const std::vector<std::vector<Hash>>& sh, int H) {
+std::vector<int> choose_cuts(const Batch& B) {
     const double inf = 1e300;
+    const int H = B.H;
     struct Band { int a, b; double us; bool ok; };
     std::vector<Band> bands;
     for (int b = 1; b <= H + 1; ++b)
@@ -128,7 +162,7 @@ std::vector<int> choose_cuts(const std::vector<const SupernodalFactor*>& distinc
     ParallelErrors errs;
 #pragma omp parallel for schedule(dynamic)
     for (size_t i = 0; i < bands.size(); ++i)
-        errs.run([&] { bands[i].us = estimate_level(distinct, members, sh, H, bands[i].a, bands[i].b, &bands[i].ok); });
+        errs.run([&] { bands[i].us = estimate_level(B, bands[i].a, bands[i].b, &bands[i].ok); });
     errs.rethrow();
     std::vector<double> best(H + 2, inf);
     std::vector<int> from(H + 2, -1);
@@ -311,58 +345,44 @@ int level_waves(long long row_tiles, double mean_tiles) { return row_tiles < 640
 
 }  // namespace
 
-double nodeplan_bytes(const SupernodalFactor& f) {
-    if (f.n == 0 || f.sn.empty()) return 0;
-    std::vector<std::vector<Hash>> sh(1, std::vector<Hash>(f.sn.size()));
-    for (size_t s = 0; s < f.sn.size(); ++s) sh[0][s].word(s);  // nothing shared
-    const std::vector<int> cuts = choose_cuts({&f}, {1}, sh, f.max_height);
-    std::vector<int> level_of(f.max_height + 1, 0);
-    for (size_t l = 0; l + 1 < cuts.size(); ++l)
-        for (int h = cuts[l]; h < cuts[l + 1]; ++h) level_of[h] = (int)l;
-    std::vector<long long> n(f.sn.size(), 0);
-    double bytes = 0;
-    for (size_t s = 0; s < f.sn.size(); ++s) {
-        const Supernode& S = f.sn[s];
-        n[s] += S.n;
-        if (!cuts.empty() && S.parent >= 0 && level_of[f.sn[S.parent].height] == level_of[S.height]) { n[S.parent] += n[s]; continue; }
-        bytes += 1024.0 * block_tiles(tiles_of((int)n[s]), tiles_of((int)S.rows.size())) + 44.0 * (n[s] + S.rows.size());
+PlanBytes nodeplan_bytes(const std::vector<const SupernodalFactor*>& F) {
+    PlanBytes out;
+    const Batch B(F);
+    if (B.H < 0) return out;
+    const std::vector<int> cuts = choose_cuts(B);
+    out.planned = !cuts.empty();
+    double total = 0, largest = 0;
+    for (size_t l = 0; l + 1 < cuts.size(); ++l) {
+        NodeKinds kinds;
+        band_nodes(B, cuts[l], cuts[l + 1], kinds);
+        for (auto& e : kinds) {
+            const NodeKind& k = e.second;
+            const int lim = run_limit(T * (k.nk + k.nrk));
+            const double runs = (double)((k.members + lim - 1) / lim), doubles = 256.0 * (k.nk + k.nrk) * k.nk;
+            out.held += 1024.0 * (double)block_tiles(k.nk, k.nrk) + 4.0 * T * k.nk;
+            // per padded column t, y, z, its row and its children's positions; per boundary row c, its column and the
+            // same; a work item per row tile
+            out.held += k.members * (24.0 * T * k.nk + 20.0 * T * k.nrk + 4.0) + runs * 48.0 * (2.0 * k.nk + k.nrk);
+            total += doubles;
+            largest = std::max(largest, doubles);
+        }
     }
-    return bytes;
+    // set-up: a chunk of the blocks' columns, their inverses, and the factor columns on their way
+    out.setup = 8.0 * 2.5 * std::min(total, std::max(largest, (double)P_::kSetupChunk));
+    return out;
 }
 
 bool build_nodeplan(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, const std::vector<int>& prob_of,
                     NodePlanHost& P) {
     P = NodePlanHost();
-    int H = -1;
-    std::vector<const SupernodalFactor*> distinct;
-    std::vector<int> members, which(F.size());
-    {
-        std::map<const SupernodalFactor*, int> id;
-        for (size_t m = 0; m < F.size(); ++m) {
-            P.n = std::max(P.n, offsets[m] + F[m]->n);
-            if (F[m]->n) H = std::max(H, F[m]->max_height);
-            auto e = id.emplace(F[m], (int)distinct.size());
-            if (e.second) { distinct.push_back(F[m]); members.push_back(0); }
-            which[m] = e.first->second;
-            ++members[which[m]];
-        }
-    }
+    for (size_t m = 0; m < F.size(); ++m) P.n = std::max(P.n, offsets[m] + F[m]->n);
+    const Batch batch(F);
+    const std::vector<const SupernodalFactor*>& distinct = batch.distinct;
+    const std::vector<int>& which = batch.which;
+    const std::vector<std::vector<Hash>>& sh = batch.sh;
+    const int H = batch.H;
     if (P.n == 0 || H < 0) return false;
-    // content hash of every supernode
-    std::vector<std::vector<Hash>> sh(distinct.size());
-    {
-        std::vector<std::pair<int, int>> todo;
-        for (size_t d = 0; d < distinct.size(); ++d) {
-            sh[d].resize(distinct[d]->sn.size());
-            for (int s = 0; s < (int)sh[d].size(); ++s) todo.push_back({(int)d, s});
-        }
-        ParallelErrors errs;
-#pragma omp parallel for schedule(dynamic, 16)
-        for (size_t i = 0; i < todo.size(); ++i)
-            errs.run([&] { sh[todo[i].first][todo[i].second] = supernode_hash(*distinct[todo[i].first], todo[i].second); });
-        errs.rethrow();
-    }
-    const std::vector<int> cuts = choose_cuts(distinct, members, sh, H);
+    const std::vector<int> cuts = choose_cuts(batch);
     if (cuts.empty()) return false;
     const int NL = (int)cuts.size() - 1;
     std::vector<int> level_of(H + 1, 0);

@@ -54,6 +54,7 @@ struct NodePlanHost {
     static constexpr int kRun = 16;          // nodes per run at most (columns of an MFMA tile)
     static constexpr int kMaxLdsFloats = 36000;  // one node's operand vector (n + nr rows)
     static constexpr int kRunLdsFloats = 12288;  // operand vectors of a run of several nodes
+    static constexpr size_t kSetupChunk = size_t(24) << 20;  // doubles of blocks set up together, unless one needs more
     struct Block {
         const SupernodalFactor* f = nullptr;
         std::vector<int> sns;                // its supernodes, ascending; the last is the node's root
@@ -94,7 +95,10 @@ void node_block_rows(const NodePlanHost::Block& B, std::vector<int>& rows);
 // Factor columns of a block, row-major, (16 nk + 16 nrk) x 16 nk doubles: L11 (padding: identity), then L21.
 void node_block_columns(const NodePlanHost::Block& B, double* L);
 
-// Device bytes of one factor's plan on its own (no sharing with other factors).
-double nodeplan_bytes(const SupernodalFactor& f);
+// Device bytes of the plan that build_nodeplan makes of these factors (repeats included: subdomains of one
+// shape): what it holds, and what its set-up needs beside it while it runs. Not planned: the batch is
+// outside the form's limits.
+struct PlanBytes { double held = 0, setup = 0; bool planned = false; };
+PlanBytes nodeplan_bytes(const std::vector<const SupernodalFactor*>& F);
 
 }  // namespace hdd

@@ -529,11 +529,10 @@ bool NodePlan::build(const std::vector<const SupernodalFactor*>& F, const std::v
     tiles.alloc((size_t)P.tiles * 256); scale.alloc(P.scales);
     t.alloc(P.ysize); y.alloc(P.ysize); z.alloc((size_t)P.ysize + 1); c.alloc((size_t)P.csize + 1);
     // the blocks in chunks: their supernodes' columns uploaded and put in place, inverted and packed
-    constexpr size_t kChunk = size_t(24) << 20;  // doubles per chunk, unless one block needs more
     auto doubles = [](const NodePlanHost::Block& B) { return (size_t)(B.nk + B.nrk) * T * B.nk * T; };
     size_t largest = 0, total = 0;
     for (const auto& B : P.blocks) { largest = std::max(largest, doubles(B)); total += doubles(B); }
-    const size_t cap = std::min(total, std::max(largest, kChunk));
+    const size_t cap = std::min(total, std::max(largest, NodePlanHost::kSetupChunk));
     DBuf<double> dL, dX;
     hdd_check(hipMalloc(&dL.p, cap * sizeof(double)), "hipMalloc"); dL.n = cap;
     size_t xcap = 0;

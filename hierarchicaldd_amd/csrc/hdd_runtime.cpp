@@ -171,31 +171,6 @@ void ProblemHost::factorize(bool wait) {
     factor_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
-size_t ProblemHost::device_bytes() const {
-    // every level: flags (5 B), two smoothing buffers, b, r (4 B each per slot), neighbour and origin tables
-    double bytes = 0;
-    for (const PagedLevel& L : lv) bytes += (L.npages() + 1.0) * kPageCells * 21.0 + L.npages() * 36.0;
-    bytes += (lv[0].npages() + 1.0) * kPageCells * 16.0;  // x, b, q, s
-    // interface solver: dense-node plans of the factors, operators, vectors
-    for (int l = 0; l < sigma.levels; ++l) {
-        for (const Csr& A : sigma.Air[l]) bytes += 16.0 * A.nnz();
-        bytes += 8.0 * sigma.Arr[l].nnz() + 64.0 * sigma.n_if[l];
-        if (l + 1 < sigma.levels) bytes += 16.0 * sigma.Prr[l].nnz();
-        if (factors && l < (int)factors->lv.size()) {
-            const SigmaFactors::Level& F = factors->lv[l];
-            for (const SupernodalFactor& f : F.Aii) bytes += nodeplan_bytes(f);
-            bytes += nodeplan_bytes(F.Arr);
-        } else {
-            for (const Csr& A : sigma.Aii[l]) bytes += 64.0 * A.nnz();
-            bytes += 64.0 * sigma.Arr[l].nnz();
-        }
-    }
-    if (factors) {
-        bytes += nodeplan_bytes(factors->bottom) + 8.0 * factors->spec.V.size();
-    }
-    return (size_t)(bytes * 1.1) + (size_t(4) << 20);
-}
-
 Solver::Solver(const SolverParams& p, int n_pages, const uint64_t* page_offsets, const uint32_t* flags, const float* b, bool host)
     : P(p), host_only(host) {
     auto t0 = std::chrono::steady_clock::now();
@@ -205,7 +180,7 @@ Solver::Solver(const SolverParams& p, int n_pages, const uint64_t* page_offsets,
     setup_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
-Solver::Solver(const std::vector<std::shared_ptr<ProblemHost>>& problems) : prob(problems) {
+Solver::Solver(const std::vector<std::shared_ptr<ProblemHost>>& problems, bool heights) : prob(problems) {
     auto t0 = std::chrono::steady_clock::now();
     if (prob.empty()) throw std::runtime_error("a batch needs at least one problem");
     P = prob[0]->P;
@@ -215,7 +190,7 @@ Solver::Solver(const std::vector<std::shared_ptr<ProblemHost>>& problems) : prob
             o.sig_s != P.sig_s || o.sig_mg != P.sig_mg)
             throw std::runtime_error("every problem of a batch needs the same V-cycle and sigma schedule (levels and smoothing counts)");
     }
-    build_device();
+    build_device(heights);
     setup_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 
@@ -274,12 +249,13 @@ DevClusters LevelBuffers::clusters() const {
 // workgroup, the largest cluster rounded up to whole wavefronts. Each has the LDS value of every cell's
 // face neighbours and the list of cells outside it that its faces read. zero_outside: cells that are not
 // Active hold zero on this level (every level but 0), so that list is one of them. False when a
-// cluster is larger than kMaxCells or a workgroup's two copies exceed the LDS.
-static bool plan_clusters(LevelBuffers& LB, bool zero_outside) {
+// cluster is larger than kMaxCells or a workgroup's two copies exceed the LDS. With `bytes` only the device
+// bytes of the tables are found and LB is not used.
+static bool plan_clusters(const PagedLevel& H, bool zero_outside, LevelBuffers* LB, double* bytes = nullptr) {
     constexpr int kMaxCells = 8192, kSpread = 512, kLdsBytes = 150 * 1024;
     static const int d[6][3] = {{-1, 0, 0}, {1, 0, 0}, {0, -1, 0}, {0, 1, 0}, {0, 0, -1}, {0, 0, 1}};
-    const PagedLevel& H = LB.host;
     const int np = H.npages();
+    if (bytes) *bytes = 0;
     if (np == 0) return false;
     // cell c's neighbour across face q: its cell in the page, or in the face's neighbour page (outside = true)
     auto step = [](int c, int q, bool& outside) {
@@ -378,6 +354,10 @@ static bool plan_clusters(LevelBuffers& LB, bool zero_outside) {
         used += count[k];
     }
     if ((long long)nwg * slots * 6 > (1LL << 30)) return false;
+    if (bytes) {  // of each slot its cell and six neighbours
+        *bytes = 16.0 * nwg * slots;
+        return true;
+    }
     // a cluster's cells in x, y, z order: the neighbours of consecutive lanes are consecutive LDS values
     std::vector<int> cell((size_t)nwg * slots, -1), at((size_t)np * kPageCells, -1), fill = base;
     for (int p = 0; p < np; ++p)
@@ -428,17 +408,63 @@ static bool plan_clusters(LevelBuffers& LB, bool zero_outside) {
         halo_ptr.push_back((int)halo_cell.size());
     }
     if (2 * sizeof(float) * (size_t)(slots + most) > (size_t)kLdsBytes) return false;
-    LB.cl_slots = slots;
-    LB.cl_threads = threads;
-    LB.cl_entries = (slots + most + 3) / 4 * 4;
-    LB.cl_rest = !zero_outside;
+    LB->cl_slots = slots;
+    LB->cl_threads = threads;
+    LB->cl_entries = (slots + most + 3) / 4 * 4;
+    LB->cl_rest = !zero_outside;
     halo_cell.push_back(np * kPageCells);  // never empty
-    LB.cl_cell.upload(cell); LB.cl_nbr.upload(nbr);
-    LB.cl_halo_ptr.upload(halo_ptr); LB.cl_halo_cell.upload(halo_cell);
+    LB->cl_cell.upload(cell); LB->cl_nbr.upload(nbr);
+    LB->cl_halo_ptr.upload(halo_ptr); LB->cl_halo_cell.upload(halo_cell);
     return true;
 }
 
-void Solver::build_device() {
+// HDD_BOTTOM_LOCAL=0 in the environment keeps one launch per sweep on every level
+static bool clusters_enabled() {
+    const char* e = std::getenv("HDD_BOTTOM_LOCAL");
+    return !(e && std::string(e) == "0");
+}
+
+size_t ProblemHost::device_bytes(bool heights, size_t* setup_bytes) const {
+    double bytes = 0, setup = 0;
+    // every level: flags (5 B), two smoothing buffers, b, r (4 B each per slot), neighbour and origin tables, clusters
+    for (size_t l = 0; l < lv.size(); ++l) {
+        double clusters = 0;
+        if (clusters_enabled()) plan_clusters(lv[l], l > 0, nullptr, &clusters);
+        bytes += (lv[l].npages() + 1.0) * kPageCells * 21.0 + lv[l].npages() * 40.0 + 4.0 * lv[l].lut.size() + clusters;
+    }
+    bytes += (lv[0].npages() + 1.0) * kPageCells * 16.0;  // x, b, q, s
+    auto plan = [&](const std::vector<const SupernodalFactor*>& F) {
+        const PlanBytes b = solve_plan_bytes(F, heights);
+        bytes += b.held;
+        setup = std::max(setup, b.setup);
+    };
+    // interface solver: the exact solves' plans, operators (padded by up to a quarter), vectors
+    for (int l = 0; l < sigma.levels; ++l) {
+        double n_int = 0;
+        for (const Csr& A : sigma.Air[l]) { bytes += 20.0 * A.nnz(); n_int += A.rows; }
+        bytes += 10.0 * sigma.Arr[l].nnz() + 64.0 * sigma.n_if[l] + 8.0 * n_int;
+        if (l + 1 < sigma.levels) bytes += 20.0 * sigma.Prr[l].nnz();
+        if (factors && l < (int)factors->lv.size()) {
+            const SigmaFactors::Level& F = factors->lv[l];
+            std::vector<const SupernodalFactor*> fi;
+            for (int s = 0; s < (int)F.rep.size(); ++s)
+                if (sigma.Aii[l][s].rows > 0) fi.push_back(&F.Aii[F.rep[s]]);
+            plan(fi);
+            if (sigma.n_if[l] > 0) plan({&F.Arr});
+        } else {
+            for (const Csr& A : sigma.Aii[l]) bytes += 64.0 * A.nnz();
+            bytes += 64.0 * sigma.Arr[l].nnz();
+        }
+    }
+    if (factors) {
+        if (factors->bottom.n) plan({&factors->bottom});
+        bytes += 8.0 * factors->spec.V.size();
+    }
+    if (setup_bytes) *setup_bytes = (size_t)setup;
+    return (size_t)(bytes * 1.1) + (size_t(4) << 20);
+}
+
+void Solver::build_device(bool heights) {
     const int NP = nprob();
     auto tp = std::chrono::steady_clock::now();
     // the bottom levels' factors and spectra finish while the levels and plans above them are built
@@ -450,10 +476,9 @@ void Solver::build_device() {
     merge_levels();
     upload_levels();
     {
-        const char* e = std::getenv("HDD_BOTTOM_LOCAL");
-        if (!(e && std::string(e) == "0")) {
+        if (clusters_enabled()) {
             for (int l = 0; l < (int)lv.size(); ++l) {
-                const bool ok = plan_clusters(lv[l], l > 0);
+                const bool ok = plan_clusters(lv[l].host, l > 0, &lv[l]);
                 if (l + 1 == (int)lv.size()) bottom_local = ok;
             }
         }
@@ -506,7 +531,7 @@ void Solver::build_device() {
     std::vector<const SigmaFactors*> facs;
     for (auto& q : prob) { hosts.push_back(&q->sigma); facs.push_back(q->factors.get()); }
     host_phase("V-cycle levels uploaded", tp);
-    sigma = make_sigma_device(hosts, facs, P.sig_s, P.sig_mg, stream);
+    sigma = make_sigma_device(hosts, facs, P.sig_s, P.sig_mg, stream, heights);
     host_phase("interface solver on the device", tp);
     hdd_check(hipStreamSynchronize(stream), "setup sync");
 }

@@ -94,8 +94,10 @@ struct ProblemHost {
     // idempotent; with wait = false the bottom level's factor may still be in progress on
     // return (factors->wait_bottom() before reading it)
     void factorize(bool wait = true);
-    // device bytes of the problem inside a batch (pages of every level, vectors, interface plans)
-    size_t device_bytes() const;
+    // device bytes of the problem: pages of every level, vectors, interface plans (heights: in the per-height
+    // form); setup (may be nullptr): what building them needs beside that while it runs. For a batch the sums:
+    // its problems share what is alike.
+    size_t device_bytes(bool heights = false, size_t* setup = nullptr) const;
 };
 
 struct LevelBuffers {
@@ -218,7 +220,7 @@ public:
     Solver(const SolverParams& p, int n_pages, const uint64_t* page_offsets, const uint32_t* flags, const float* b,
            bool host_only = false);
     // a batch of problems set up on the host (factorised here if they are not yet)
-    explicit Solver(const std::vector<std::shared_ptr<ProblemHost>>& problems);
+    explicit Solver(const std::vector<std::shared_ptr<ProblemHost>>& problems, bool heights = false);
     ~Solver();
 
     int nprob() const { return (int)prob.size(); }
@@ -281,7 +283,7 @@ private:
     };
     std::vector<Graph> graphs;
     void record_apply();
-    void build_device();
+    void build_device(bool heights = false);
     void merge_levels();
     void upload_levels();
     void sweeps(int l, int count, bool interior, bool boundary);

@@ -112,7 +112,12 @@ void Server::setup_worker() {
         try {
             auto h = std::make_shared<ProblemHost>(r->P, (int)r->offsets.size(), r->offsets.data(), r->flags.data(), r->b.data());
             h->factorize();
-            r->bytes = h->device_bytes();
+            r->bytes = h->device_bytes(false, &r->setup_bytes);
+            if ((double)r->bytes > budget_) {
+                size_t setup = 0;
+                const size_t bytes = h->device_bytes(true, &setup);
+                if ((double)bytes <= budget_) { r->bytes = bytes; r->setup_bytes = setup; r->heights = true; }
+            }
             r->host = h;
             std::vector<uint32_t>().swap(r->flags);
             std::vector<float>().swap(r->b);
@@ -154,7 +159,9 @@ void Server::builder() {
                     if ((*it)->cancel) { finish_cancelled(*it); it = ready.erase(it); cv_done.notify_all(); }
                     else ++it;
                 }
-                if (!ready.empty() && units_ < prm.groups && in_use_ + (double)ready.front()->bytes <= budget_) break;
+                if (!ready.empty() && units_ < prm.groups &&
+                    (units_ == 0 || in_use_ + (double)ready.front()->bytes + (double)ready.front()->setup_bytes <= budget_))
+                    break;
                 if (ready.empty() && drained_for_builder()) {
                     builder_done_ = true;
                     lk.unlock();
@@ -165,24 +172,27 @@ void Server::builder() {
             }
             // arrival order; problems with another V-cycle/sigma schedule wait for a later unit
             const SolverParams lead = ready.front()->P;
+            const bool heights = ready.front()->heights;
             for (auto it = ready.begin(); it != ready.end() && (int)u->reqs.size() < prm.max_batch;) {
-                const double b = (double)(*it)->bytes;
-                if (!same_schedule((*it)->P, lead)) { ++it; continue; }
-                if (in_use_ + u->bytes + b > budget_) break;
+                const double b = (double)(*it)->bytes, setup = (double)(*it)->setup_bytes;
+                if (!same_schedule((*it)->P, lead) || (*it)->heights != heights) { ++it; continue; }
+                if (!u->reqs.empty() && in_use_ + u->bytes + b + std::max(u->setup_bytes, setup) > budget_) break;
                 u->bytes += b;
+                u->setup_bytes = std::max(u->setup_bytes, setup);
                 u->reqs.push_back(*it);
                 it = ready.erase(it);
             }
-            in_use_ += u->bytes;
+            in_use_ += u->bytes + u->setup_bytes;
             ++units_;
             for (auto& r : u->reqs) r->batch_size = (int)u->reqs.size();
         }
         try {
             std::vector<std::shared_ptr<ProblemHost>> hosts;
             for (auto& r : u->reqs) hosts.push_back(r->host);
-            u->S.reset(new Solver(hosts));
+            u->S.reset(new Solver(hosts, u->reqs.front()->heights));
         } catch (std::exception& e) {
             std::lock_guard<std::mutex> lk(mu);
+            in_use_ -= u->setup_bytes;
             for (auto& r : u->reqs) { r->failed = true; r->error = e.what(); r->done = true; r->t_done = now(); r->host.reset(); }
             in_use_ -= u->bytes;
             --units_;
@@ -191,6 +201,7 @@ void Server::builder() {
         }
         {
             std::lock_guard<std::mutex> lk(mu);
+            in_use_ -= u->setup_bytes;  // the set-up's own arrays are gone
             joining.push_back(std::move(u));
         }
         cv_driver.notify_all();

@@ -17,8 +17,10 @@
 //
 // Admission: a problem's device footprint is estimated from its host setup
 // (ProblemHost::device_bytes); a unit is admitted while the sum over resident
-// units stays within the HBM budget and there are fewer than `groups` units.
-// A problem larger than the whole budget is rejected.
+// units, with what its set-up needs while it runs, stays within the HBM budget
+// and there are fewer than `groups` units; with none resident it is built
+// anyway. A problem whose plans exceed the budget alone is solved with the
+// per-height plans, which take about half, and rejected if they do too.
 #pragma once
 #include <chrono>
 #include <condition_variable>
@@ -49,7 +51,8 @@ struct ServerRequest {
     double tol = 0;
     int max_it = 0;
     std::shared_ptr<ProblemHost> host;
-    size_t bytes = 0;
+    size_t bytes = 0, setup_bytes = 0;  // on the device, and beside that while it is built
+    bool heights = false;               // per-height plans: the others would exceed the budget
     // result
     std::vector<float> x;    // input page order
     int iterations = 0;
@@ -82,7 +85,7 @@ private:
         std::vector<std::shared_ptr<ServerRequest>> reqs;
         std::unique_ptr<Solver> S;
         PcgRun run;
-        double bytes = 0;
+        double bytes = 0, setup_bytes = 0;
     };
     void setup_worker();
     void builder();

@@ -79,8 +79,9 @@ struct TriPlan : TriHeights {
     void drop_heights() { static_cast<TriHeights&>(*this) = TriHeights(); }
     size_t factor_nnz = 0;
     static constexpr int kFusedGroups = 1 << 30;
-    // prob_of[m]: problem of factor m (empty: all problem 0)
-    void build(const std::vector<const SupernodalFactor*>& factors, const std::vector<int>& offs, const std::vector<int>& probs = {});
+    // prob_of[m]: problem of factor m (empty: all problem 0); heights: the per-height form, whatever the factors
+    void build(const std::vector<const SupernodalFactor*>& factors, const std::vector<int>& offs, const std::vector<int>& probs = {},
+               bool heights = false);
     // per-problem flags (device, 1 = iterating): supernodes of stopped problems are skipped; nullptr: none skipped
     const int* active = nullptr;
     // x = (A + eps I)^{-1} b; with refine > 0, each solve is followed by `refine`
@@ -191,9 +192,13 @@ struct SigmaDevice {
 
 // Device interface solver of a batch: the problems' operators stacked
 // block-diagonally (problem order), from their host operators and factors.
-// The setup's own device work (the bottom self-check) runs on `stream`.
+// The setup's own device work (the bottom self-check) runs on `stream`. heights:
+// every exact solve in the per-height form (about half the memory, slower).
 std::unique_ptr<SigmaDevice> make_sigma_device(const std::vector<const SigmaHost*>& hosts, const std::vector<const SigmaFactors*>& factors,
-                                               int smoothing, int n_mg, hipStream_t stream);
+                                               int smoothing, int n_mg, hipStream_t stream, bool heights = false);
+
+// Device bytes of the plan TriPlan::build makes of these factors.
+PlanBytes solve_plan_bytes(const std::vector<const SupernodalFactor*>& F, bool heights);
 void sigma_vcycles(SigmaDevice& S, hipStream_t s);
 void launch_interface_gather(SigmaDevice& S, const DevLevel& L0, const int* if_index, const float* z, const float* r, hipStream_t s);
 void launch_interface_gather(SigmaDevice& S, const DevLevel& L0, const int* if_index, const __half* z, const __half* r, hipStream_t s);

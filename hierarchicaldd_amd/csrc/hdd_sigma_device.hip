@@ -1070,12 +1070,20 @@ static bool heights_forced() {
     return (top && *top) || (wave && (std::string(wave) == "0" || std::string(wave) == "1"));
 }
 
-void TriPlan::build(const std::vector<const SupernodalFactor*>& factors, const std::vector<int>& offs, const std::vector<int>& probs) {
+PlanBytes solve_plan_bytes(const std::vector<const SupernodalFactor*>& F, bool heights) {
+    PlanBytes b;
+    if (!heights && !heights_forced()) b = nodeplan_bytes(F);
+    if (!b.planned) triplan_bytes(F, dense_top_min_rows(), &b.held, &b.setup);
+    return b;
+}
+
+void TriPlan::build(const std::vector<const SupernodalFactor*>& factors, const std::vector<int>& offs, const std::vector<int>& probs,
+                    bool heights) {
     F = factors; offsets = offs; prob_of = probs;
     for (size_t m = 0; m < F.size(); ++m) { n = std::max(n, offsets[m] + F[m]->n); factor_nnz += F[m]->nnz(); }
     if (n == 0) return;
     auto tp = std::chrono::steady_clock::now();
-    use_nodes = !heights_forced() && nodes.build(F, offsets, prob_of);
+    use_nodes = !heights && !heights_forced() && nodes.build(F, offsets, prob_of);
     setup_phase("  dense-node plan", (int)F.size(), tp, "factors");
     if (!use_nodes) build_heights();
 }
@@ -1623,7 +1631,7 @@ static void append_rows(Csr& M, const Csr& A, int col_off) {
 }
 
 std::unique_ptr<SigmaDevice> make_sigma_device(const std::vector<const SigmaHost*>& hosts, const std::vector<const SigmaFactors*>& factors,
-                                               int smoothing, int n_mg, hipStream_t stream) {
+                                               int smoothing, int n_mg, hipStream_t stream, bool heights) {
     const int NP = (int)hosts.size();
     if (NP == 0 || (int)factors.size() != NP) throw std::runtime_error("make_sigma_device: one host operator set and factor set per problem");
     std::unique_ptr<SigmaDevice> S(new SigmaDevice());
@@ -1680,9 +1688,9 @@ std::unique_ptr<SigmaDevice> make_sigma_device(const std::vector<const SigmaHost
         L.Arr.upload(arr, false);
         if (l + 1 < NL) { pr.cols = ifoff[l + 1][NP]; L.P.upload(pr, false); L.PT.upload(transpose(pr), false); }
         setup_phase("interface operators uploaded", l, tp);
-        L.Lii.build(fi, oi, pi);
+        L.Lii.build(fi, oi, pi, heights);
         setup_phase("Aii plan", l, tp);
-        L.Lrr.build(fr, orr, prr);
+        L.Lrr.build(fr, orr, prr, heights);
         setup_phase("Arr plan", l, tp);
         S->dense_top_rows += L.Lii.top_dense_rows + L.Lrr.top_dense_rows;
         L.u.alloc(std::max(1, L.n_if)); L.b.alloc(std::max(1, L.n_if)); L.r.alloc(std::max(1, L.n_if)); L.tmp.alloc(std::max(1, L.n_if));
@@ -1740,7 +1748,7 @@ std::unique_ptr<SigmaDevice> make_sigma_device(const std::vector<const SigmaHost
             boff += F.bottom_n_int + np;
         }
         setup_phase("bottom modes gathered", lb, tp);
-        S->Lbottom.build(fb, ob, pb);
+        S->Lbottom.build(fb, ob, pb, heights);
         setup_phase("bottom plan", lb, tp);
         if (autotune()) S->tuned_choices += S->Lbottom.tune(stream);
         setup_phase("bottom plan tuned", lb, tp);

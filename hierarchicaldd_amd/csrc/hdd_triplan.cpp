@@ -92,6 +92,30 @@ void dense_top_factor(const TriPlanHost::TopBlock& B, double* L) {
     if (outside) throw std::runtime_error("dense top: a row below the top is not in it");
 }
 
+void triplan_bytes(const std::vector<const SupernodalFactor*>& F, int top_min_rows, double* held, double* setup) {
+    *held = *setup = 0;
+    int members = 0;
+    for (const SupernodalFactor* f : F) members += top_min_rows > 0 && f->n >= top_min_rows;
+    std::map<const SupernodalFactor*, double> own;  // the lists and vectors of each factor
+    for (const SupernodalFactor* f : F) {
+        auto e = own.emplace(f, 0.0);
+        if (e.second) {
+            for (const Supernode& S : f->sn) {
+                const double n = S.n, nr = (double)S.rows.size();
+                *held += 8.0 * n * n + 4.0 * n * nr;  // the diagonal block's inverse twice, L21
+                e.first->second += 28.0 * n + 16.0 * nr + 4.0 * n * ((S.rows.size() + TriPlanHost::kTile - 1) / TriPlanHost::kTile) + 80.0;
+            }
+            int m = 0;
+            if (dense_top_cut(*f, top_min_rows, members, &m) != INT_MAX) {
+                const double ld = (m + TriPlanHost::kTopLd - 1) / TriPlanHost::kTopLd * TriPlanHost::kTopLd;
+                *held += 4.0 * ld * ld;
+                *setup = std::max(*setup, 16.0 * m * m);
+            }
+        }
+        *held += e.first->second;
+    }
+}
+
 void build_triplan(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, TriPlanHost& P, int top_min_rows) {
     P = TriPlanHost();
     for (size_t m = 0; m < F.size(); ++m) {

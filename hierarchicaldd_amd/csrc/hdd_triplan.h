@@ -108,6 +108,10 @@ struct TriPlanHost {
 // top_min_rows: factors with at least this many rows get a dense top (0: none).
 void build_triplan(const std::vector<const SupernodalFactor*>& F, const std::vector<int>& offsets, TriPlanHost& P, int top_min_rows = 0);
 
+// Device bytes of the plan that build_triplan makes of these factors (repeats included), and what its set-up
+// needs beside it while it runs.
+void triplan_bytes(const std::vector<const SupernodalFactor*>& F, int top_min_rows, double* held, double* setup);
+
 // The height from which the supernodes of f form its dense top, with the top's
 // rows in *m (a height above f's tree and *m = 0 when f gets none), in a plan
 // with `members` factors of at least top_min_rows rows (at most 64). Heights

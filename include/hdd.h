@@ -436,7 +436,9 @@ typedef struct hdd_server_params {
     int setup_threads;        /* host setup workers */
     int groups;               /* units resident and iterating on the device at once */
     int max_batch;            /* problems per unit */
-    double hbm_budget_bytes;  /* device bytes for resident problems; 0 = 90% of the free device memory */
+    double hbm_budget_bytes;  /* device bytes for resident problems; 0 = 90% of the free device memory. A problem
+                                 that exceeds it with the dense-node plans is solved with the per-height ones,
+                                 slower and a fraction of the size, and refused if it exceeds it with those */
 } hdd_server_params;
 
 typedef struct hdd_request_report {
