@@ -573,24 +573,25 @@ hdd_status hdd_stats(const hdd_ctx* ctx, double* out, int n) {
     for (auto& q : S.prob) nsub += q->sigma.nsub;
     // levels of the dense-node plans and fused heights of the per-height ones, and how many of
     // those use the wavefront-per-run form
-    double fused = 0, waved = 0;
+    double fused = 0, waved = 0, tuned = 0;
     if (G) {
         auto count = [&](const TriPlan& T) {
             fused += (double)T.nodes.levels.size();
+            tuned += T.tuned ? 1 : 0;
             for (size_t h = 0; h < T.fused.size(); ++h)
                 if (T.fused[h]) { fused += 1; waved += (h < T.wave.size() && T.wave[h]) ? 1 : 0; }
         };
         for (const SigmaLevel& L : G->lv) { count(L.Lii); count(L.Lrr); }
         count(G->Lbottom);
     }
-    double v[18] = {S.setup_seconds, G ? G->factor_seconds : 0.0, G ? (double)G->plan_bytes : 0.0,
+    double v[19] = {S.setup_seconds, G ? G->factor_seconds : 0.0, G ? (double)G->plan_bytes : 0.0,
                     (double)S.lv[0].host.npages(), (G && G->levels) ? (double)G->lv[0].n_if : (S.sigma_host().levels ? (double)S.sigma_host().n_if[0] : 0.0),
                     (G && G->levels) ? (double)G->lv[0].n_int : 0.0, (double)nsub,
                     G ? G->bottom_rho : -1.0, G ? (double)G->bottom_direct : 0.0, G ? (double)G->bottom_k : 0.0,
                     G ? G->bottom_seconds : 0.0, G ? (double)G->bottom_steps : 0.0, G ? G->bottom_check : -1.0,
                     G ? (double)G->tuned_choices : 0.0, G ? (double)G->dense_top_rows : 0.0, S.bottom_local ? 1.0 : 0.0,
-                    fused, waved};
-    for (int i = 0; i < n && i < 18; ++i) out[i] = v[i];
+                    fused, waved, tuned};
+    for (int i = 0; i < n && i < 19; ++i) out[i] = v[i];
     return HDD_OK;
 }
 

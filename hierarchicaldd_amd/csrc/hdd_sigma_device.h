@@ -52,6 +52,7 @@ struct TriHeights {          // the per-height form
     std::vector<int> sn_begin, sl_begin, sl_rows, row_begin, ci_begin, bi_begin, max_sz, big, fused, G, Gc, Gf, Gb, run_begin, run_max;
     std::vector<int> wave;  // per fused height: 1 = a wavefront per run (k_tri_*_wave), 0 = a workgroup per run (same results)
     bool wave_forced = false;  // HDD_FUSED_WAVE set: the tuner leaves `wave` alone
+    bool tuned = false;        // its launch shapes were timed
     // per fused height: a cap on the workgroups of its launch, each looping over runs (default:
     // no cap, a workgroup per run; the tuner tries caps; results do not depend on it)
     std::vector<int> pgrid;

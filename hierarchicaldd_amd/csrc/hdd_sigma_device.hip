@@ -1447,6 +1447,7 @@ int TriPlan::tune(hipStream_t s) {
     }
     (void)hipEventDestroy(e0); (void)hipEventDestroy(e1);
     hdd_check(hipStreamSynchronize(s));
+    tuned = true;
     return changed;
 }
 

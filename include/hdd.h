@@ -379,7 +379,8 @@ hdd_status hdd_profile_copy(hdd_ctx* ctx, int reps, double* avg_ms, double* byte
  * a workgroup per run, the same bits) is set in the environment at set-up, for
  * separators beyond the dense nodes' limits, and for refined solves at the first
  * hdd_set_sigma_refinement with steps > 0; they round differently.
- * n = number of slots provided (up to 18). No reference counterpart. */
+ * out[18]: per-height plans whose launch shapes the autotuner timed.
+ * n = number of slots provided (up to 19). No reference counterpart. */
 hdd_status hdd_stats(const hdd_ctx* ctx, double* out, int n);
 
 /* Measurement: runs `reps` exact solves of one triangular-solve plan of sigma
