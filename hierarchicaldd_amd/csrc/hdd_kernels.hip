@@ -797,13 +797,16 @@ __global__ void __launch_bounds__(256) k_unscale_project(DevLevel L, const __hal
 // reductions add, exactly as k_seg_dot does for a one-problem context, so the
 // value has the bits of hdd_inner_product on a context holding the same pages.
 // Calls take the tickets in turn and clear the one half a round away: calls that
-// overlapped (they may not) spoil no later call's ticket for more than a round.
+// overlapped (they may not) spoil no later call's ticket for more than a round. A
+// captured call keeps its ticket over all replays, so it clears it by itself first.
 constexpr int kNoAllocParts = 1024, kNoAllocTickets = 64;  // reduce_parts never exceeds the first
 struct NoAllocScratch {
     double part[kNoAllocParts];
     unsigned ticket[kNoAllocTickets];
 };
 static __device__ __align__(256) NoAllocScratch scratch;
+
+__global__ void k_clear_ticket(NoAllocScratch* w, int ticket) { w->ticket[ticket] = 0; }
 
 template <bool kWide>
 __global__ void __launch_bounds__(kDotThreads) k_dot_flat(const float* __restrict__ a, const float* __restrict__ b, size_t groups, int g,
@@ -967,6 +970,11 @@ void launch_inner_product_noalloc(const float* a, const float* b, int64_t n_page
     if (g > kNoAllocParts) throw std::runtime_error("inner product (no allocation): more partial sums than the scratch holds");
     static std::atomic<unsigned> calls{0};
     const int ticket = (int)(calls.fetch_add(1, std::memory_order_relaxed) % kNoAllocTickets);
+    if (s) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+        if (capture == hipStreamCaptureStatusActive) hipLaunchKernelGGL(k_clear_ticket, dim3(1), dim3(1), 0, s, noalloc_scratch(), ticket);
+    }
     // the caller's arrays may start anywhere
     const bool wide = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
     hipLaunchKernelGGL((wide ? k_dot_flat<true> : k_dot_flat<false>), dim3(g), dim3(kDotThreads), 0, s, a, b, n / 4, g, noalloc_scratch(), ticket, out);

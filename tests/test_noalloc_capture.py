@@ -1,0 +1,20 @@
+"""A captured hdd_inner_product_noalloc is right at every replay, whatever earlier calls left in its ticket
+(tests/noalloc_capture_check.cpp: on the CPU, the HIP calls replaced)."""
+import os
+import subprocess
+
+from hierarchicaldd_amd import build, hdd
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+def test_replays_do_not_depend_on_earlier_calls(tmp_path):
+    hdd.lib()
+    exe = str(tmp_path / "noalloc_capture_check")
+    cmd = [build.HIPCC, "-O1", "-std=c++17", "-rdynamic", "-x", "hip", "--offload-arch=gfx950", os.path.join(HERE, "noalloc_capture_check.cpp"),
+           "-o", exe, "-L", build.OUT, "-lhdd", f"-Wl,-rpath,{build.OUT}"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    print(r.stdout)
+    assert r.returncode == 0, r.stdout + r.stderr
