@@ -181,7 +181,9 @@ __global__ void __launch_bounds__(64 * kSweepPages) k_smooth(DevLevel L, const S
 // bit-identical to one launch per sweep. nbr gives each cell's face neighbours as
 // LDS values; a neighbour outside the workgroup is a cell no sweep writes, held
 // in the halo behind the slots. Where a face bit is not set it names the cell
-// itself, whose difference is an exact zero. The cells ping-pong between two
+// itself, whose difference is an exact zero while the cell is finite (an infinite
+// one becomes NaN, as the next sweep of it makes of it in any case: its set faces
+// give inf - inf). The cells ping-pong between two
 // copies (the halo is in both), one barrier per sweep. u is updated in place: no
 // other workgroup reads the Active cells of this one's clusters.
 //
@@ -651,7 +653,9 @@ __device__ __forceinline__ float block_max(float m) {
 // ticket adds them, in the order a second launch would (which cost 3-4 us more for each of the three
 // reductions of an iteration). The ticket is zero between launches. Partials are exchanged and loaded past
 // the caches, and a block draws its ticket when its exchange has returned, so no cache is written back or
-// invalidated: with a release and acquire of the device's scope instead, 1024 blocks took 45 us longer.
+// invalidated: with a release and acquire of the device's scope instead, 1024 blocks took 45 us longer, and
+// the 256 of a 256^3 domain's inner product, releasing on the ticket with the acquire left to the last of them,
+// 26.9 us for 24.8.
 template <class V>
 __device__ __forceinline__ void leave_partial(V* p, V v) {
     const V old = __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
