@@ -55,6 +55,9 @@ struct DevClusters {
 // in turn: count[i] sweeps of the interior (kSweepInterior) and / or boundary (kSweepBoundary) cells
 enum { kSweepInterior = 1, kSweepBoundary = 2 };
 struct SweepPhases { int n = 0, count[3] = {0, 0, 0}, cells[3] = {0, 0, 0}; };
+constexpr size_t kClusterLdsBytes = 150 * 1024;  // of a workgroup's two copies
+// once per plan, on its device, before its first launch: lets the kernels use the LDS that the plan needs
+void prepare_cluster_sweeps(const DevClusters& C);
 // u in place; u_zero: u is zero at the start (and not read); r (may be nullptr): the residual after the sweeps
 void launch_cluster_sweeps(const DevLevel& L, const DevClusters& C, float* u, const float* b, float* r, const SweepPhases& ph, bool u_zero,
                            hipStream_t s);

@@ -861,11 +861,7 @@ static void smooth_t(const DevLevel& L, const S* u_in, S* u_out, const S* b, boo
 }
 template <class S, int C>
 static void cluster_sweeps_c(const DevLevel& L, const DevClusters& W, S* u, const S* b, S* r, const SweepPhases& ph, bool u_zero, hipStream_t s) {
-    const size_t lds = 2 * (size_t)W.entries * sizeof(S);
-    if (lds > 48 * 1024)
-        hdd_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cluster_sweeps<S, C>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024),
-                  "cluster sweeps' LDS");
-    hipLaunchKernelGGL((k_cluster_sweeps<S, C>), dim3(W.nwg), dim3(W.threads), lds, s, L, W, u, b, r, ph, (int)u_zero);
+    hipLaunchKernelGGL((k_cluster_sweeps<S, C>), dim3(W.nwg), dim3(W.threads), 2 * (size_t)W.entries * sizeof(S), s, L, W, u, b, r, ph, (int)u_zero);
 }
 template <class S>
 static void cluster_sweeps_t(const DevLevel& L, const DevClusters& W, S* u, const S* b, S* r, const SweepPhases& ph, bool u_zero, hipStream_t s) {
@@ -879,6 +875,22 @@ static void cluster_sweeps_t(const DevLevel& L, const DevClusters& W, S* u, cons
         case 2: cluster_sweeps_c<S, 2>(L, W, u, b, r, ph, u_zero, s); break;
         case 4: cluster_sweeps_c<S, 4>(L, W, u, b, r, ph, u_zero, s); break;
         case 8: cluster_sweeps_c<S, 8>(L, W, u, b, r, ph, u_zero, s); break;
+        default: throw std::runtime_error("cluster sweeps: cells per thread");
+    }
+}
+template <class S, int C>
+static void allow_cluster_lds() {
+    hdd_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_cluster_sweeps<S, C>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)kClusterLdsBytes),
+              "cluster sweeps' LDS");
+}
+void prepare_cluster_sweeps(const DevClusters& W) {
+    if (!W.nwg || 2 * (size_t)W.entries * sizeof(float) <= 48 * 1024) return;
+    switch (W.slots / W.threads) {
+        case 1: allow_cluster_lds<float, 1>(); allow_cluster_lds<__half, 1>(); break;
+        case 2: allow_cluster_lds<float, 2>(); allow_cluster_lds<__half, 2>(); break;
+        case 4: allow_cluster_lds<float, 4>(); allow_cluster_lds<__half, 4>(); break;
+        case 8: allow_cluster_lds<float, 8>(); allow_cluster_lds<__half, 8>(); break;
         default: throw std::runtime_error("cluster sweeps: cells per thread");
     }
 }

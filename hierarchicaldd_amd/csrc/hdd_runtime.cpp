@@ -252,7 +252,7 @@ DevClusters LevelBuffers::clusters() const {
 // cluster is larger than kMaxCells or a workgroup's two copies exceed the LDS. With `bytes` only the device
 // bytes of the tables are found and LB is not used.
 static bool plan_clusters(const PagedLevel& H, bool zero_outside, LevelBuffers* LB, double* bytes = nullptr) {
-    constexpr int kMaxCells = 8192, kSpread = 512, kLdsBytes = 150 * 1024;
+    constexpr int kMaxCells = 8192, kSpread = 512;
     static const int d[6][3] = {{-1, 0, 0}, {1, 0, 0}, {0, -1, 0}, {0, 1, 0}, {0, 0, -1}, {0, 0, 1}};
     const int np = H.npages();
     if (bytes) *bytes = 0;
@@ -407,7 +407,7 @@ static bool plan_clusters(const PagedLevel& H, bool zero_outside, LevelBuffers* 
         halo_cell.insert(halo_cell.end(), halo[w].begin(), halo[w].end());
         halo_ptr.push_back((int)halo_cell.size());
     }
-    if (2 * sizeof(float) * (size_t)(slots + most) > (size_t)kLdsBytes) return false;
+    if (2 * sizeof(float) * (size_t)(slots + most) > kClusterLdsBytes) return false;
     LB->cl_slots = slots;
     LB->cl_threads = threads;
     LB->cl_entries = (slots + most + 3) / 4 * 4;
@@ -479,6 +479,7 @@ void Solver::build_device(bool heights) {
         if (clusters_enabled()) {
             for (int l = 0; l < (int)lv.size(); ++l) {
                 const bool ok = plan_clusters(lv[l].host, l > 0, &lv[l]);
+                prepare_cluster_sweeps(lv[l].clusters());
                 if (l + 1 == (int)lv.size()) bottom_local = ok;
             }
         }
