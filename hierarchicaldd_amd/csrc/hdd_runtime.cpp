@@ -31,6 +31,16 @@ void HostStage::init(size_t largest_bytes) {
     for (hipEvent_t& e : done) hdd_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
 }
 
+// Memory that the runtime copies at the link's rate by itself (pinned, registered, managed or a device's) needs no ring
+static bool pageable(const void* p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
 // memcpy of one chunk over the host's threads, in pieces of whole pages
 static void copy_parallel(char* to, const char* from, size_t bytes) {
     constexpr size_t kPiece = size_t(256) << 10;
@@ -40,7 +50,7 @@ static void copy_parallel(char* to, const char* from, size_t bytes) {
 }
 
 void HostStage::to_host(void* host, const void* dev, size_t bytes, hipStream_t s) {
-    if (bytes < kMin || !ring.p) {
+    if (bytes < kMin || !ring.p || !pageable(host)) {
         hdd_check(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s), "copy to the host");
         hdd_check(hipStreamSynchronize(s), "copy to the host");
         return;
@@ -62,7 +72,7 @@ void HostStage::to_host(void* host, const void* dev, size_t bytes, hipStream_t s
 }
 
 void HostStage::to_device(void* dev, const void* host, size_t bytes, hipStream_t s) {
-    if (bytes < kMin || !ring.p) {
+    if (bytes < kMin || !ring.p || !pageable(host)) {
         hdd_check(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s), "copy to the device");
         hdd_check(hipStreamSynchronize(s), "copy to the device");
         return;

@@ -161,7 +161,8 @@ class HostStage {
 public:
     ~HostStage();
     void init(size_t largest_bytes);  // at set-up: the pinned ring, when copies that long will use it
-    // both return when the copy is complete; copies below kMin bytes go to the runtime
+    // both return when the copy is complete; copies below kMin bytes, and of memory that is not pageable, go to
+    // the runtime
     void to_host(void* host, const void* dev, size_t bytes, hipStream_t s);
     void to_device(void* dev, const void* host, size_t bytes, hipStream_t s);
     static constexpr size_t kMin = size_t(4) << 20, kChunk = size_t(4) << 20;

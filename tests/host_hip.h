@@ -11,7 +11,7 @@
 static std::mutex g_mu;
 static std::map<void*, size_t> g_live;
 static size_t g_held = 0, g_peak = 0;
-static int g_attributes = 0, g_launches = 0;
+static int g_attributes = 0, g_launches = 0, g_copies = 0;
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
@@ -33,7 +33,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = std::calloc(1, n);
 hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
 hipError_t hipMemset(void* p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }
 hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind) { std::memcpy(to, from, n); return hipSuccess; }
-hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind, hipStream_t) { std::memcpy(to, from, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind, hipStream_t) { ++g_copies; std::memcpy(to, from, n); return hipSuccess; }
 hipError_t hipMemcpyToSymbol(const void*, const void*, size_t, size_t, hipMemcpyKind) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)std::malloc(1); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { std::free(s); return hipSuccess; }
