@@ -8,10 +8,12 @@ default smoothing counts), with every SPGrid page, flag and interface-solver
 plan resident in HBM before the timed region.
 
 Printed JSON line: value = solves/s (1 / time-to-tolerance); the roofline
-object covers the level-0 damped-Jacobi sweep kernel, timed with HIP events
-on the context stream; "sigma_solves" gives the same for one exact solve of
-each triangular-solve plan of the interface solver (time per solve, bytes of
-the factor entries read); cpu_baseline is the oracle (the CPU restatement of the
+object covers the interface solver's plan that takes the largest share of an
+iteration, timed with HIP events on the context stream; "sigma_solves" gives
+the same for one exact solve of each plan (time per solve, bytes of the distinct
+operator elements it reads), "vcycle_sweep" for the level-0 damped-Jacobi sweep
+(13 bytes a page slot; a level that fits the Infinity Cache, so not a fraction
+of the memory's rate alone; "vcycle_sweep_512" does not fit); cpu_baseline is the oracle (the CPU restatement of the
 reference dd_pcg) on a bounded sample: the complete 64^3 problem (setup +
 solve), set beside the GPU's rate on the same 64^3 problem.
 
@@ -51,6 +53,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+# bytes a sweep moves per page slot (u, b and a byte of flags read, u written) over those that
+# hdd_profile_sweep reports (the reference's four-byte flags)
+MOVED_FP32, MOVED_FP16 = 13 / 16, 7 / 10
 PROFILES = os.path.join(ROOT, "profiles")
 METRIC = "256³ time-to-1e-6 rel-res; batched solves/s; p50/p99 served latency"
 
@@ -129,11 +134,13 @@ def main():
 
     if args.sweep_only:
         sweep_ms, sweep_bytes = solver.profile_sweep(20)
+        sweep_bytes *= MOVED_FP32
         log(f"[bench] level-0 sweep: {sweep_ms * 1e3:.1f} us/launch, {sweep_bytes / 1e6:.1f} MB algorithmic")
         copy_ms, copy_bytes = solver.profile_copy(20)
         log(f"[bench] calibration copy: {copy_ms * 1e3:.1f} us/launch, {copy_bytes / 2:.0f} bytes read and {copy_bytes / 2:.0f} written")
         solver.set_fp16(True)
         h_ms, h_bytes = solver.profile_sweep(20)
+        h_bytes *= MOVED_FP16
         log(f"[bench] level-0 sweep, FP16 storage: {h_ms * 1e3:.1f} us/launch, {h_bytes / 1e6:.1f} MB algorithmic")
         return
 
@@ -152,6 +159,7 @@ def main():
 
     # the level-0 smoothing sweep (the V-cycle kernel), HIP events on the context stream
     sweep_ms, sweep_bytes = solver.profile_sweep(100)
+    sweep_bytes *= MOVED_FP32
     sweep_gbs = sweep_bytes / (sweep_ms * 1e-3) / 1e9
     log(f"[bench] level-0 sweep: {sweep_ms * 1e3:.1f} us/launch, {sweep_bytes / 1e6:.1f} MB algorithmic, {sweep_gbs:.0f} GB/s")
     copy_ms, copy_bytes = solver.profile_copy(50)
@@ -164,6 +172,7 @@ def main():
         t0 = time.time()
         dom512, cfg512 = domain.sparse_spheres(target_coverage=0.30)
         ms512, by512 = hdd.profile_sweep_grid(dom512, cfg512, 100)
+        by512 *= MOVED_FP32
         gbs512 = by512 / (ms512 * 1e-3) / 1e9
         sweep512 = {"kernel": "k_smooth (level-0 damped-Jacobi sweep, FP32)", "workload": dom512.meta.get("workload"),
                     "pages": dom512.n_pages, "algorithmic_bytes": by512, "us_per_launch": ms512 * 1e3, "achieved": gbs512,
@@ -173,8 +182,8 @@ def main():
         del dom512
 
     # exact solves of the interface solver's triangular-solve plans: mean time per solve with HIP
-    # events, algorithmic bytes = 4 B per factor entry per pass, two passes (subdomains that share
-    # one factor counted each); solves per PCG iteration from the sigma V-cycle's schedule
+    # events, algorithmic bytes = the distinct operator elements a solve reads (blocks that several
+    # subdomains share once); solves per PCG iteration from the sigma V-cycle's schedule
     sigma_solves = []
     n_sigma, _ = solver.sigma_info()
     plans = [(l, w) for l in range(n_sigma) for w in ("Aii", "Arr")] + ([(n_sigma - 1, "bottom")] if st["bottom_direct"] else [])
@@ -200,13 +209,14 @@ def main():
         t16.append(secs)
         it16.append(it)
     h_ms, h_bytes = solver.profile_sweep(100)
+    h_bytes *= MOVED_FP16
     solver.set_fp16(False)
     fp16 = {"time_to_tolerance_s": float(np.mean(t16)), "solves_per_s": 1.0 / float(np.mean(t16)), "iterations": int(np.median(it16)),
             "sweep_us": h_ms * 1e3, "sweep_achieved_GBs": h_bytes / (h_ms * 1e-3) / 1e9,
-            "sweep_frac": h_bytes / (h_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "sweep_bytes_per_slot": 10}
+            "sweep_frac": h_bytes / (h_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "sweep_bytes_per_slot": 7}
     fp16["traffic"] = counter_traffic(dom.n_pages, "k_smooth<__half, false>") if args.config == "sphere256" else None
     log(f"[bench] fp16-storage V-cycles: {fp16['iterations']} iterations, {fp16['time_to_tolerance_s']:.3f}s; "
-        f"level-0 sweep {h_ms * 1e3:.1f} us ({fp16['sweep_achieved_GBs']:.0f} GB/s algorithmic at 10 B/slot)")
+        f"level-0 sweep {h_ms * 1e3:.1f} us ({fp16['sweep_achieved_GBs']:.0f} GB/s algorithmic at 7 B/slot)")
     solver.close()
     cpu = None
     if not args.no_cpu_baseline:
@@ -258,13 +268,15 @@ def main():
 def solves_per_iteration(level, plan, n_sigma, cfg, bottom_direct):
     """Exact solves of one plan per PCG iteration (one preconditioner apply, sigma_mg V-cycles):
     above the bottom, sigma_smoothing smooths down and up (each one Aii and one Arr solve) and one
-    residual (one Aii solve); the bottom's 200 smooths are one combined solve when it is direct."""
+    residual (one Aii solve); a smooth from zero, the first of a level but for later cycles' level 0,
+    has no Aii solve; the bottom's 200 smooths are one combined solve when it is direct."""
     s, mg = cfg.sigma_smoothing, cfg.sigma_mg
+    from_zero = (mg if level > 0 else 1) if s > 0 else 0
     if plan == "bottom":
         return mg if bottom_direct else 0
     if level < n_sigma - 1:
-        return mg * (2 * s + 1 if plan == "Aii" else 2 * s)
-    return 0 if bottom_direct else mg * 200
+        return mg * (2 * s + 1) - from_zero if plan == "Aii" else mg * 2 * s
+    return 0 if bottom_direct else mg * 200 - (from_zero if plan == "Aii" else 0)
 
 
 def dof_updates_per_iteration(solver, cfg):
@@ -401,8 +413,10 @@ def sparse_leg(hdd):
                 rows.append(row)
     g.set_outer_fp64(False)
     ms, by = g.profile_sweep(50)
+    by *= MOVED_FP16
     g.set_fp16(False)
     ms32, by32 = g.profile_sweep(50)
+    by32 *= MOVED_FP32
     g.close()
     return {"metric": METRIC, "config": {**meta, "pages": dom.n_pages, "sub_size": cfg.sub_size,
                                          "vlevels": cfg.vlevels}, "setup_s": st["setup_s"], "solves": rows,

@@ -620,7 +620,7 @@ hdd_status hdd_profile_solve(hdd_ctx* ctx, int level, int which, int reps, doubl
         hdd_check(hipEventElapsedTime(&ms, a, e));
         (void)hipEventDestroy(a); (void)hipEventDestroy(e);
         *avg_ms = ms / reps;
-        if (bytes) *bytes = 8.0 * (double)P->factor_nnz;
+        if (bytes) *bytes = P->operator_bytes();
     })
 }
 

@@ -849,7 +849,7 @@ DevSegments Solver::segments() {
 // The apply is a fixed sequence of launches for a given state of the
 // smoothing ping-pong buffers and of the skip mode, so with use_graph it is
 // captured once into a HIP graph per such state and replayed: one graph launch
-// instead of ~2000 kernel launches per PCG iteration. Nothing in it allocates,
+// instead of the 80 to 260 kernel launches of an iteration. Nothing in it allocates,
 // copies or clears memory through the runtime (clears are fill kernels).
 // Off by default: the replay is bit-identical but measured no faster (the
 // iteration is bound by the GPU's dispatch of dependent kernels, not by host

@@ -99,6 +99,7 @@ struct TriPlan : TriHeights {
     // launch-shape autotuner (slice rows, contribution items per height); returns the choices changed
     int tune(hipStream_t s);
     size_t bytes() const;
+    double operator_bytes() const;  // of the operators that a solve reads, each distinct one once (per pass that reads it)
     static constexpr int kTuneMinRows = 20000;           // plans below this size keep their default shapes
     void rebuild_lists(hipStream_t s);
     void top_solve(const float* b_orig, float* x_orig, hipStream_t s);

@@ -1157,6 +1157,16 @@ size_t TriPlan::bytes() const {
            (top_rows.n + top_of.n + top_inc_ptr.n + top_base.n + top_ld.n + top_W.n + top_t.n) * 4 + (top_cpos.n + top_woff.n) * 8;
 }
 
+double TriPlan::operator_bytes() const {
+    // the forward and the backward operator of a node are tiles of their own, a closed node's inverse is read once
+    if (use_nodes && refine == 0) return 4.0 * (double)(nodes.tiles.n + nodes.scale.n);
+    std::map<const SupernodalFactor*, int> seen;
+    double entries = 0;
+    for (const SupernodalFactor* f : F)
+        if (seen.emplace(f, 1).second) entries += (double)f->nnz();
+    return (1 + refine) * 8.0 * entries;  // both passes
+}
+
 #define HDD_SN_DISPATCH(G, KERNEL, BLOCKS, SHMEM, ...)                                                           \
     switch (G) {                                                                                                \
         case 4: hipLaunchKernelGGL(KERNEL<4>, dim3(BLOCKS), dim3(256), SHMEM, __VA_ARGS__); break;              \

@@ -343,7 +343,7 @@ class DDSolver:
         return dict(zip(keys, out.tolist()))
 
     def profile_solve(self, level: int, which: str, reps: int = 20):
-        """Mean duration (ms) of one triangular-solve plan ("Aii", "Arr" or "bottom") and its algorithmic bytes."""
+        """Mean duration (ms) of one triangular-solve plan ("Aii", "Arr" or "bottom") and the bytes of its operators."""
         ms, by = C.c_double(), C.c_double()
         self._check(lib().hdd_profile_solve(self.h, level, {"Aii": 0, "Arr": 1, "bottom": 2}[which], reps, C.byref(ms), C.byref(by)))
         return ms.value, by.value

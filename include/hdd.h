@@ -133,7 +133,7 @@ hdd_status hdd_set_graph(hdd_ctx* ctx, int enable);
  * reference stores everything in float): fp16 = 0 (default) keeps the
  * reference's FP32 V-cycles; fp16 = 1 stores the V-cycle vectors u, b and r of
  * every level in FP16 with FP32 arithmetic (the smoothing sweep then moves
- * 10 B per cell instead of 16). The preconditioner is linear, so it runs on
+ * 7 B per cell instead of 13). The preconditioner is linear, so it runs on
  * r / max|r| of each problem and scales its result back, keeping the stored
  * values inside FP16's normal range; the interface solver, the PCG vectors and
  * reductions stay FP32/FP64. hdd_smooth and hdd_profile_sweep then act on the
@@ -147,7 +147,9 @@ hdd_status hdd_set_vcycle_storage(hdd_ctx* ctx, int fp16);
  * IFS/SIGMA_SMOOTHER.cpp:151); steps = 1..3 follows each solve with that many
  * steps of iterative refinement, x += (A + 1e-5 I)^{-1} (b - (A + 1e-5 I) x),
  * the residual accumulated in FP64, so the solves are accurate to FP32
- * rounding of their result (each step costs one more solve). */
+ * rounding of their result (each step costs one more solve). The first call
+ * with steps > 0 builds the plans they use; when it fails (out of device
+ * memory) the context is as it was, and the call can be made again. */
 hdd_status hdd_set_sigma_refinement(hdd_ctx* ctx, int steps);
 
 /* Summation order of the inner products of the PCG loop and hdd_inner_product:
@@ -332,8 +334,9 @@ hdd_status hdd_setup_seconds(const hdd_ctx* ctx, double* seconds);
 
 /* Measurement: runs `reps` level-0 smoothing sweeps (all Active cells) on the
  * context stream bracketed by HIP events; returns the mean duration of one
- * launch and the algorithmic HBM bytes of one launch (16 B per page slot:
- * flags, u and b read, u written; 10 B with FP16 V-cycle storage). No
+ * launch and the bytes of one launch as the reference's layout has them (16 B
+ * per page slot: flags, u and b read, u written; 10 B with FP16 V-cycle
+ * storage). The kernel itself reads a byte of flags: it moves 13 and 7. No
  * reference counterpart. */
 hdd_status hdd_profile_sweep(hdd_ctx* ctx, int reps, double* avg_ms, double* bytes_per_launch);
 
@@ -342,7 +345,7 @@ hdd_status hdd_profile_sweep(hdd_ctx* ctx, int reps, double* avg_ms, double* byt
  * divider, interface operators or factorisation), `reps` back-to-back launches
  * on a stream of its own bracketed by HIP events: mean duration of one launch
  * and 16 B per page slot. Lets a grid larger than the Infinity Cache (512^3
- * sparse: 572 MB) be timed without its set-up. No reference counterpart. */
+ * sparse: 578 MB) be timed without its set-up. No reference counterpart. */
 hdd_status hdd_profile_sweep_grid(const hdd_problem_desc* desc, int reps, double* avg_ms, double* bytes_per_launch);
 
 /* Measurement: runs `reps` plain copies of one level-0 float channel into the
@@ -367,9 +370,9 @@ hdd_status hdd_profile_copy(hdd_ctx* ctx, int reps, double* avg_ms, double* byte
  * as two dense triangular matvecs; HDD_DENSE_TOP=0 in the environment turns
  * them off, HDD_DENSE_TOP=k gives a dense top to factors of at least k rows,
  * 4096 by default), out[15] 1 if the interior V-cycle's 200 coarsest-level sweeps
- * run page by page in one launch (bit-identical to 200 launches; set-up picks
- * it when that level's Active cells couple only within their pages,
- * HDD_BOTTOM_LOCAL=0 turns it off), else 0, out[16] levels of the dense-node
+ * run in one launch (bit-identical to 200 launches; set-up picks it for every
+ * level whose Active cells couple only within clusters that fit a workgroup's
+ * LDS, HDD_BOTTOM_LOCAL=0 keeps a launch per sweep on all levels), else 0, out[16] levels of the dense-node
  * plans (one launch per level and pass), plus tree heights of the per-height
  * plans done by one fused launch per height (a workgroup or a wavefront per run
  * of supernodes), out[17] how many of those heights use the wavefront form.
@@ -386,8 +389,10 @@ hdd_status hdd_stats(const hdd_ctx* ctx, double* out, int n);
 /* Measurement: runs `reps` exact solves of one triangular-solve plan of sigma
  * level `level` (which = 0: all subdomains' (Aii + eps I), 1: (Arr + eps I),
  * 2: the bottom level's combined system) on the context stream, bracketed by
- * HIP events; returns the mean duration of one solve and its algorithmic
- * bytes (4 B per factor entry per pass, two passes, every subdomain counted).
+ * HIP events; returns the mean duration of one solve and the bytes of the
+ * operators it reads: each distinct one once per pass that reads it, however
+ * many subdomains share it (4 B per element of the dense nodes' tiles, or per
+ * factor entry and pass of the per-height plans).
  * The right-hand side is zero (the cost does not depend on the values). No
  * reference counterpart. */
 hdd_status hdd_profile_solve(hdd_ctx* ctx, int level, int which, int reps, double* avg_ms, double* bytes_per_solve);
