@@ -292,27 +292,35 @@ double constant_share(const P_::Block& B) {
         while (part[a] != a) a = part[a] = part[part[a]];
         return a;
     };
-    auto columns = [&](auto&& use) {  // use(column, row, entry) for the entries of the triangle, column after column
-        int col = 0;
-        const int* row = at.data();
-        for (int s : B.sns) {
-            const int n = f.sn[s].n, nr = (int)f.sn[s].rows.size();
-            for (int j = 0; j < n; ++j) {
-                for (int r = j; r < n; ++r) use(col + j, col + r, f.L11[s][(size_t)j * n + r]);
-                for (int a = 0; a < nr; ++a) use(col + j, row[a], f.L21[s][(size_t)j * nr + a]);
-            }
-            col += n;
-            row += nr;
+    // of each column of the triangle the square of its sum and the sum of its squares; its rows are coupled to it
+    std::vector<double> all(B.n), diag(B.n);
+    int col = 0;
+    const int* row = at.data();
+    for (int s : B.sns) {
+        const int n = f.sn[s].n, nr = (int)f.sn[s].rows.size();
+        for (int j = 0; j < n; ++j) {
+            double sum = 0, squares = 0;
+            int root = find(col + j);
+            auto entry = [&](int i, double l) {
+                sum += l;
+                squares += l * l;
+                if (l != 0 && part[i] != root) part[find(i)] = root;
+            };
+            const double *l11 = &f.L11[s][(size_t)j * n], *l21 = nr ? &f.L21[s][(size_t)j * nr] : nullptr;
+            for (int r = j; r < n; ++r) entry(col + r, l11[r]);
+            for (int a = 0; a < nr; ++a) entry(row[a], l21[a]);
+            all[col + j] = sum * sum;
+            diag[col + j] = squares;
         }
-    };
-    columns([&](int j, int i, double l) { if (l != 0 && i != j) part[find(i)] = find(j); });
-    std::vector<double> sum(B.n, 0.0), all(B.n, 0.0), diag(B.n, 0.0);  // of a column; of a part's entries, of its diagonal
-    std::vector<int> m(B.n, 0);
-    columns([&](int j, int i, double l) {
-        sum[j] += l;
-        diag[find(i)] += l * l;
-    });
-    for (int j = 0; j < B.n; ++j) { const int p = find(j); all[p] += sum[j] * sum[j]; ++m[p]; }
+        col += n;
+        row += nr;
+    }
+    std::vector<int> m(B.n, 0);  // rows of a part, at its root
+    for (int j = 0; j < B.n; ++j) {
+        const int p = find(j);
+        if (p != j) { all[p] += all[j]; diag[p] += diag[j]; }
+        ++m[p];
+    }
     double share = 0;
     for (int p = 0; p < B.n; ++p)
         if (m[p] > 1) share = std::max(share, diag[p] / (all[p] * std::sqrt((double)m[p])));
