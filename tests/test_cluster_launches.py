@@ -6,12 +6,13 @@ import subprocess
 from hierarchicaldd_amd import build, hdd
 
 HERE = os.path.dirname(os.path.abspath(__file__))
+PACKED_OFF = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]  # as the library is built
 
 
 def test_attributes_are_set_with_the_plan(tmp_path):
     hdd.lib()
     exe = str(tmp_path / "cluster_launch_check")
-    cmd = [build.HIPCC, "-O1", "-std=c++17", "-fopenmp", "-rdynamic", "-x", "hip", "--offload-arch=gfx950", os.path.join(HERE, "cluster_launch_check.cpp"),
+    cmd = [build.HIPCC, "-O1", "-std=c++17", "-fopenmp", "-rdynamic", "-x", "hip", "--offload-arch=gfx950", *PACKED_OFF, os.path.join(HERE, "cluster_launch_check.cpp"),
            "-o", exe, "-L", build.OUT, "-lhdd", f"-Wl,-rpath,{build.OUT}"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]

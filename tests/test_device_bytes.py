@@ -11,6 +11,7 @@ import pytest
 from hierarchicaldd_amd import build, domain, hdd
 
 HERE = os.path.dirname(os.path.abspath(__file__))
+PACKED_OFF = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]  # as the library is built
 
 
 @pytest.fixture(scope="module")
@@ -18,7 +19,7 @@ def check(tmp_path_factory):
     hdd.lib()
     d = tmp_path_factory.mktemp("device_bytes")
     exe = str(d / "device_bytes_check")
-    cmd = [build.HIPCC, "-O1", "-std=c++17", "-fopenmp", "-rdynamic", "-x", "hip", "--offload-arch=gfx950", os.path.join(HERE, "device_bytes_check.cpp"),
+    cmd = [build.HIPCC, "-O1", "-std=c++17", "-fopenmp", "-rdynamic", "-x", "hip", "--offload-arch=gfx950", *PACKED_OFF, os.path.join(HERE, "device_bytes_check.cpp"),
            "-o", exe, "-L", build.OUT, "-lhdd", f"-Wl,-rpath,{build.OUT}"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]

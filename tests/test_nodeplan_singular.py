@@ -16,12 +16,13 @@ import pytest
 from hierarchicaldd_amd import build, hdd
 
 HERE = os.path.dirname(os.path.abspath(__file__))
+PACKED_OFF = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]  # as the library is built
 
 
 @pytest.fixture(scope="module")
 def check(tmp_path_factory):
     lib = str(tmp_path_factory.mktemp("nodeplan") / "nodeplan_singular_check.so")
-    cmd = [build.HIPCC, "-O2", "-std=c++17", "-fPIC", "-shared", "-x", "hip", "--offload-arch=gfx950",
+    cmd = [build.HIPCC, "-O2", "-std=c++17", "-fPIC", "-shared", "-x", "hip", "--offload-arch=gfx950", *PACKED_OFF,
            os.path.join(HERE, "nodeplan_singular_check.cpp"), "-o", lib, "-L", build.OUT, "-lhdd", f"-Wl,-rpath,{build.OUT}"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]

@@ -7,12 +7,13 @@ import subprocess
 from hierarchicaldd_amd import build, hdd
 
 HERE = os.path.dirname(os.path.abspath(__file__))
+PACKED_OFF = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]  # as the library is built
 
 
 def test_failed_refinement_can_be_retried(tmp_path):
     hdd.lib()
     exe = str(tmp_path / "refinement_check")
-    cmd = [build.HIPCC, "-O1", "-std=c++17", "-fopenmp", "-rdynamic", "-x", "hip", "--offload-arch=gfx950", os.path.join(HERE, "refinement_check.cpp"),
+    cmd = [build.HIPCC, "-O1", "-std=c++17", "-fopenmp", "-rdynamic", "-x", "hip", "--offload-arch=gfx950", *PACKED_OFF, os.path.join(HERE, "refinement_check.cpp"),
            "-o", exe, "-L", build.OUT, "-lhdd", f"-Wl,-rpath,{build.OUT}"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-3000:]
