@@ -9,10 +9,16 @@
 
 namespace hdd {
 
+struct OutOfDeviceMemory : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
 inline void hdd_check(hipError_t e, const char* what = "HIP call") {
     if (e == hipSuccess) return;
     (void)hipGetLastError();  // reported here: the checks after later launches report their own
-    throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
+    const std::string message = std::string(what) + ": " + hipGetErrorString(e);
+    if (e == hipErrorOutOfMemory) throw OutOfDeviceMemory(message);
+    throw std::runtime_error(message);
 }
 
 // One paged level on the device. flags has (np+1)*256 entries (zero page last), kinds the

@@ -542,7 +542,13 @@ void Solver::build_device(bool heights) {
     std::vector<const SigmaFactors*> facs;
     for (auto& q : prob) { hosts.push_back(&q->sigma); facs.push_back(q->factors.get()); }
     host_phase("V-cycle levels uploaded", tp);
-    sigma = make_sigma_device(hosts, facs, P.sig_s, P.sig_mg, stream, heights);
+    try {
+        sigma = make_sigma_device(hosts, facs, P.sig_s, P.sig_mg, stream, heights);
+    } catch (const OutOfDeviceMemory&) {
+        if (heights) throw;
+        // the per-height plans may fit where the dense nodes, at up to five times their bytes, did not
+        sigma = make_sigma_device(hosts, facs, P.sig_s, P.sig_mg, stream, true);
+    }
     host_phase("interface solver on the device", tp);
     hdd_check(hipStreamSynchronize(stream), "setup sync");
 }

@@ -380,7 +380,8 @@ hdd_status hdd_profile_copy(hdd_ctx* ctx, int reps, double* avg_ms, double* byte
  * few levels of dense nodes. The per-height plans (a launch or more per tree
  * height) are built where HDD_DENSE_TOP=k or HDD_FUSED_WAVE=1 / 0 (a wavefront /
  * a workgroup per run, the same bits) is set in the environment at set-up, for
- * separators beyond the dense nodes' limits, and for refined solves at the first
+ * separators beyond the dense nodes' limits, for contexts whose dense nodes do
+ * not fit the device memory, and for refined solves at the first
  * hdd_set_sigma_refinement with steps > 0; they round differently.
  * out[18]: per-height plans whose launch shapes the autotuner timed.
  * n = number of slots provided (up to 19). No reference counterpart. */

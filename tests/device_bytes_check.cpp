@@ -42,6 +42,8 @@ static std::shared_ptr<ProblemHost> host_of(const Input& in) {
     return q;
 }
 
+// "create <memory> file": a context with that much device memory; prints the peak and whether its solves use
+//     dense nodes, or "failed: .."
 // "bytes <heights> file..": one context of the problems; prints estimate, set-up estimate, bytes held, peak
 // "server <budget> file": one request; prints "done" or "failed: .."
 int main(int argc, char** argv) {
@@ -56,6 +58,15 @@ int main(int argc, char** argv) {
         const auto r = s.wait(id);
         if (r->failed) std::printf("failed: %s\n", r->error.c_str());
         else std::printf("done %d\n", (int)r->heights);
+    } else if (what == "create") {
+        const auto host = host_of(read_input(argv[3]));
+        g_memory = (size_t)std::atof(argv[2]);
+        try {
+            Solver S({host});
+            std::printf("%zu %d\n", g_peak, (int)S.sigma->lv[0].Lrr.use_nodes);
+        } catch (const std::exception& e) {
+            std::printf("failed: %s\n", e.what());
+        }
     } else {
         const bool heights = std::atoi(argv[2]) != 0;
         std::vector<std::shared_ptr<ProblemHost>> hosts;

@@ -10,13 +10,15 @@
 
 static std::mutex g_mu;
 static std::map<void*, size_t> g_live;
-static size_t g_held = 0, g_peak = 0;
+static size_t g_held = 0, g_peak = 0, g_memory = ~size_t(0);  // device bytes; as many as there are
 static int g_attributes = 0, g_launches = 0, g_copies = 0;
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
-    *p = std::calloc(1, n);
     std::lock_guard<std::mutex> l(g_mu);
+    *p = nullptr;
+    if (n > g_memory - g_held) return hipErrorOutOfMemory;
+    *p = std::calloc(1, n);
     g_live[*p] = n;
     g_held += n;
     if (g_held > g_peak) g_peak = g_held;

@@ -83,3 +83,13 @@ def test_tight_budget_takes_the_smaller_plans(check):
     assert check("server", nodes - 1, problem) == "done 1"
     assert check("server", heights, problem) == "done 1"
     assert check("server", heights - 1, problem).startswith("failed: problem needs more device memory")
+
+
+def test_context_falls_back_when_the_dense_nodes_do_not_fit(check):
+    problem = [domain.small_box(33, 16, 3, seed=1)]
+    nodes, heights = (int(check("bytes", h, problem).split()[3]) for h in (0, 1))  # peaks of the two forms
+    assert check("create", nodes, problem) == f"{nodes} 1"
+    peak, dense = (int(v) for v in check("create", nodes - 1, problem).split())
+    assert dense == 0 and peak < nodes
+    assert check("create", heights, problem) == f"{heights} 0"
+    assert check("create", heights // 2, problem).startswith("failed: hipMalloc")
